@@ -3,14 +3,15 @@
 // restriction (mg.f90:249-806), getres (mg.f90:809-848), prolongation
 // (mg.f90:850-940) and sor_rb (modules/legacy/sors.f90:1-535), one rank.
 //
-// Each smoother sweep is one launch per colour over that colour's nodes
-// (x fastest), followed by a deterministic block-tree L1 residual and a
-// one-block kernel that applies sor_rb's exit rules on the device (res <= eps
-// on the coarsest level, res/res_s <= 0.6 elsewhere, at most 4 sweeps) and
-// clears the level's active flag.  Sweeps queued after the exit return at once, so
-// a V-cycle needs no host round trip; the host reads the fine residual once
-// per V-cycle for pdesolver's convergence test.  Levels below a few thousand
-// nodes run inside one workgroup (k_mg_coarse).
+// A sweep of a global level is one launch over tiles held in LDS (k_sweep):
+// red, black and the L1 residual, with sor_rb's exit rule (res/res_s <= 0.6,
+// at most 4 sweeps) taken by every block of the next launch.  Levels with
+// periodic ghosts to copy between the colours, and a coarsest level too large
+// for one workgroup, take one launch per colour, a deterministic block-tree
+// residual and a one-block decision.  Sweeps queued after the exit return at
+// once, so a V-cycle needs no host round trip; the host reads the fine
+// residual once per V-cycle for pdesolver's convergence test.  Levels below a
+// few thousand nodes run inside one workgroup (k_mg_coarse).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -307,6 +308,301 @@ __global__ __launch_bounds__(BLOCK) void k_decide(const double *partials, int64_
 }
 
 
+// --------------------------------------------------------------------------
+// Whole sweeps of a global level in one launch.  A block takes a TX x TY x TZ
+// tile, reads it with a halo of H nodes into LDS, runs the colour phases on
+// rings of the halo that shrink by one per phase (the halo's nodes relaxed
+// again by each tile that needs them: the same operands and expression, so
+// the same bits as the owner's) and writes its own nodes to the other of two
+// u arrays, which the next launch reads.  One launch per colour, residual and
+// decision spends 60 us per sweep at 128^3 (19.6 + 19.6 + 15.2 + 5) and 12 at
+// 16^3, all of it launches and L2 round trips; the fused sweep takes 29 us and
+// 9 (an idle one 3), FP64, split about evenly between the reads (390 KB per
+// block through one CU's L1), the three LDS phases and launch + decision.
+//
+// The two colours are held apart in LDS, so that the lanes of a phase read
+// consecutive words.  Row (j, k) of node colours: red nodes have i + j + k
+// odd; pair p of a row holds the nodes xb + 2 p and xb + 2 p + 1, xb even.
+// --------------------------------------------------------------------------
+
+// One sor_rb of at most 4 sweeps is 4 launches ("slots").  Every block of
+// slot s sums slot s - 1's block residuals in the same fixed order and so
+// takes the same exit decision; block 0 records it for slot s + 1.
+struct SlotState {
+  int64_t active;   // the slot swept
+  int64_t pad;
+  double res_s;     // the residual its decision compared against next
+};
+
+constexpr int SLOTS = 4;
+
+struct SlotCtl {
+  SlotState *state;     // SLOTS entries
+  double *partials;     // 2 x nparts: slot s writes half s & 1
+  int64_t nparts;       // blocks of the level's sweep launches
+};
+
+// Sum of slot s's block residuals, the same in every thread and block: this
+// thread's first one (read early), then the rest and the block's sum.
+__device__ inline double slot_first(const SlotCtl &sc, int s) {
+  const double *p = sc.partials + (int64_t)(s & 1) * sc.nparts;
+  return threadIdx.x < sc.nparts ? p[threadIdx.x] : 0.0;
+}
+
+template <int NT>
+__device__ inline double slot_sum(const SlotCtl &sc, int s, double a, double *red) {
+  const double *p = sc.partials + (int64_t)(s & 1) * sc.nparts;
+  for (int64_t t = (int64_t)threadIdx.x + NT; t < sc.nparts; t += NT) a = a + p[t];
+  for (int d = LEPIC_WAVE / 2; d > 0; d >>= 1) a = a + __shfl_down(a, d);
+  if (__lane_id() == 0) red[threadIdx.x / LEPIC_WAVE] = a;
+  __syncthreads();
+  double r = 0.0;
+  for (int w = 0; w < NT / LEPIC_WAVE; ++w) r = r + red[w];
+  __syncthreads();
+  return r;
+}
+
+// The exit rule of sor_rb above the coarsest level (sors.f90:446-454).
+__device__ inline bool sor_stops(double res, double res_s) {
+  return res_s > 0.0 && (res / res_s) <= 0.6;
+}
+
+// After the last slot: the counters of a sor_rb that ran all its sweeps (an
+// earlier exit has already left its own).  Called by one block of NT threads.
+template <int NT>
+__device__ inline void slots_finish(const SlotCtl &sc, MGCtl *ctl, double *red) {
+  if (sc.state[SLOTS - 1].active == 0) return;
+  const double res = slot_sum<NT>(sc, SLOTS - 1, slot_first(sc, SLOTS - 1), red);
+  if (threadIdx.x == 0) {
+    ctl->res = res;
+    ctl->total += SLOTS;
+  }
+}
+
+__global__ __launch_bounds__(BLOCK) void k_slots_finish(SlotCtl sc, MGCtl *ctl) {
+  __shared__ double red[BLOCK / LEPIC_WAVE];
+  slots_finish<BLOCK>(sc, ctl, red);
+}
+
+template <class T>
+struct Vec2 {
+  typedef T type __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+};
+
+// SWEEPS sweeps from src to dst.  RES: one sweep, the L1 residual after it
+// to this slot's partials, the exit decided from the slot before.  !RES: a
+// fixed count, zero != 0 when src is known to be 0 everywhere (not read).
+//
+// A thread owns one pair position (p, jj) of every HZ-th plane: with HZ even
+// the parity of its nodes, and with it every LDS offset, is the same in all
+// its planes, so a phase has no index arithmetic.
+template <class T, int TX, int TY, int TZ, int NT, int HZ, int SWEEPS, bool RES>
+__global__ __launch_bounds__(NT) void k_sweep(KLevelT<T> L, const T *src, T *dst, T omega, int ntx,
+                                              int nty, int zero, int slot, SlotCtl sc,
+                                              MGCtl *ctl) {
+  constexpr int H = 2 * SWEEPS + (RES ? 1 : 0);
+  constexpr int NP = (TX + 2 * H + 2) / 2;              // pairs per row
+  constexpr int BY = TY + 2 * H, BZ = TZ + 2 * H;       // rows of the black array
+  constexpr int RY = BY - 2, RZ = BZ - 2;               // rows of the red array
+  constexpr int BSY = NP, BSZ = BY * NP, RSY = NP, RSZ = RY * NP;
+  constexpr int R = (BZ + HZ - 1) / HZ;                 // planes per thread
+  static_assert(HZ % 2 == 0 && NP * BY * HZ <= NT, "a thread per pair of HZ planes");
+  __shared__ T sb[BZ * BSZ];
+  __shared__ T sr[RZ * RSZ];
+  __shared__ double red[NT / LEPIC_WAVE];
+  const KGrid &g = L.g;
+  const int n1 = g.n1, n2 = g.n2, n3 = g.n3;
+  const int64_t nodes = ((int64_t)n1 + 3) * (n2 + 3) * (n3 + 3);
+  // consecutive tiles on one XCD (blocks go to the XCDs in turn), so that they
+  // find each other's halos in its L2
+  const int per = (int)gridDim.x / LEPIC_XCDS;
+  const int tile = (int)blockIdx.x < per * LEPIC_XCDS
+                       ? ((int)blockIdx.x % LEPIC_XCDS) * per + (int)blockIdx.x / LEPIC_XCDS
+                       : (int)blockIdx.x;
+  const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
+  const int xs = 1 + bx * TX, ys = 1 + by * TY, zs = 1 + bz * TZ;
+  const int xb = (xs - H) & ~1, yb = ys - H, zb = zs - H;
+  const int p = (int)threadIdx.x % NP, jj = ((int)threadIdx.x / NP) % BY,
+            h = (int)threadIdx.x / BSZ;
+  const bool mine = h < HZ;
+  const int j = yb + jj, q = (j + zb + h) & 1;
+  const int ir = xb + 2 * p + 1 - q, ib = xb + 2 * p + q;   // the pair's red and black node
+  // how far outside the tile, in the plane (H: not a relaxed position)
+  auto ring_xy = [&](int i, bool in) {
+    const int d = max(max(xs - i, i - (xs + TX - 1)), max(ys - j, j - (ys + TY - 1)));
+    return in && i >= 1 && i <= n1 + 1 && j >= 1 && j <= n2 + 1 ? max(d, 0) : H;
+  };
+  const int ringr = ring_xy(ir, mine && jj >= 1 && jj <= RY);
+  const int ringk = ring_xy(ib, mine && jj >= 2 && jj <= RY - 1);
+
+  if (RES && slot > 0) {
+    const SlotState st = sc.state[slot - 1];
+    const double first = slot_first(sc, slot - 1);
+    bool active = false;
+    if (st.active) {
+      const double res = slot_sum<NT>(sc, slot - 1, first, red);
+      active = !sor_stops(res, st.res_s);
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc.state[slot].active = active ? 1 : 0;
+        sc.state[slot].res_s = res;
+        if (!active) {
+          ctl->res = res;
+          ctl->total += slot;
+        }
+      }
+      // the first idle slot after an odd number of sweeps brings u home
+      if (!active && (slot & 1)) {
+        const int64_t stride = (int64_t)gridDim.x * NT;
+        for (int64_t t = blockIdx.x * (int64_t)NT + threadIdx.x; t < nodes; t += stride)
+          dst[t] = src[t];
+      }
+    } else if (blockIdx.x == 0 && threadIdx.x == 0) {
+      sc.state[slot].active = 0;
+    }
+    if (!active) return;
+  } else if (RES && blockIdx.x == 0 && threadIdx.x == 0) {
+    sc.state[0].active = 1;
+    sc.state[0].res_s = 0.0;
+  }
+  // Every read is issued before anything waits (a launch starts with a cold
+  // L2, so each dependent read costs most of a microsecond), from addresses
+  // that need no test of what was read: clamped into the arrays, and nothing
+  // that nodes outside the relaxed range bring is used.
+  typedef typename Vec2<T>::type V2;
+  const int64_t off0 = (int64_t)(xb + 2 * p) + g.sy * (int64_t)j + g.sz * (int64_t)(zb + h);
+  const int64_t step = HZ * g.sz;
+  auto inside = [&](int64_t c) { return c < 0 ? 0 : (c > nodes - 2 ? nodes - 2 : c); };
+  constexpr int RH = R / 3;   // planes whose b is read before the first wait (more spill)
+  V2 uv[R], bv[R];
+  int lr[R], lk[R];
+  const bool relaxes = min(ringr, ringk) < H;
+  if (!zero) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      uv[r] = *reinterpret_cast<const V2 *>(src + inside(off0 + r * step));
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; ++r) uv[r] = V2{T(0), T(0)};
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) lr[r] = lk[r] = 1;
+  if (relaxes) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t c = inside(off0 + r * step);
+      lr[r] = L.bc[c + 1 - q];
+      lk[r] = L.bc[c + q];
+    }
+  }
+  auto read_b = [&](int r) {
+    bv[r] = *reinterpret_cast<const V2 *>(L.b + inside(off0 + r * step));
+  };
+#pragma unroll
+  for (int r = 0; r < RH; ++r) read_b(r);
+  // class of a node: 0 not relaxed, 1 plasma, 2 Neumann, 3 other
+  auto cls_of = [&](int lab, int k) {
+    if (lab > 0 || k < 1 || k > n3 + 1) return 0;
+    if (lab == 0 && (k == n3 + 1 || j == n2 + 1)) return 0;
+    return lab == -1 ? 1 : (lab == -2 ? 2 : 3);
+  };
+  const int m0 = h * BSZ + jj * BSY + p, e0 = (h - 1) * RSZ + (jj - 1) * RSY + p;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int kk = h + r * HZ, m = m0 + r * HZ * BSZ, e = e0 + r * HZ * RSZ;
+    lr[r] = cls_of(lr[r], zb + kk);
+    lk[r] = cls_of(lk[r], zb + kk);
+    if (off0 + r * step == nodes - 1) uv[r].x = uv[r].y;   // the last node has no pair
+    if (mine && kk < BZ) {
+      sb[m] = q ? uv[r].y : uv[r].x;
+      if (jj >= 1 && jj <= RY && kk >= 1 && kk <= RZ) sr[e] = q ? uv[r].x : uv[r].y;
+    }
+  }
+#pragma unroll
+  for (int r = RH; r < R; ++r) read_b(r);   // in flight during the first planes' relaxation
+  __syncthreads();
+  double a = 0.0;
+  auto relax = [&](int cls, T uc, T uw, T ue, T un, T us, T ut, T ub, T bb) {
+    if (cls == 2)
+      return (T(1) - omega) * uc +
+             div_ac(omega * (bb - L.an * un - L.as * us - T(2) * L.ae * ue - L.at * ut - L.ab * ub),
+                    L);
+    return (T(1) - omega) * uc +
+           div_ac(omega * (bb - L.aw * uw - L.an * un - L.as * us - L.ae * ue - L.at * ut -
+                           L.ab * ub),
+                  L);
+  };
+  auto resid = [&](T uc, T uw, T ue, T un, T us, T ut, T ub, T bb) {
+    const T rij = bb - (L.aw * uw + L.an * un + L.as * us + L.ae * ue + L.ac * uc + L.at * ut +
+                        L.ab * ub);
+    return fabs((double)rij);
+  };
+#pragma unroll
+  for (int s = 0; s < SWEEPS; ++s) {
+    const int red_ring = H - 1 - 2 * s, black_ring = H - 2 - 2 * s;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int kk = h + r * HZ, m = m0 + r * HZ * BSZ, e = e0 + r * HZ * RSZ;
+      if (ringr <= red_ring && kk >= H - red_ring && kk <= H + TZ - 1 + red_ring && lr[r])
+        sr[e] = relax(lr[r], sr[e], sb[m - q], sb[m + 1 - q], sb[m + BSY], sb[m - BSY],
+                      sb[m + BSZ], sb[m - BSZ], q ? bv[r].x : bv[r].y);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int kk = h + r * HZ, m = m0 + r * HZ * BSZ, e = e0 + r * HZ * RSZ;
+      if (ringk <= black_ring && kk >= H - black_ring && kk <= H + TZ - 1 + black_ring && lk[r]) {
+        const T uw = sr[e - 1 + q], ue = sr[e + q], un = sr[e + RSY], us = sr[e - RSY],
+                ut = sr[e + RSZ], ub = sr[e - RSZ], bb = q ? bv[r].y : bv[r].x;
+        const T u = relax(lk[r], sb[m], uw, ue, un, us, ut, ub, bb);
+        sb[m] = u;
+        if (RES && lk[r] == 1 && ringk == 0 && kk >= H && kk <= H + TZ - 1)
+          a = a + resid(u, uw, ue, un, us, ut, ub, bb);
+      }
+    }
+    __syncthreads();
+  }
+  if (RES) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int kk = h + r * HZ, m = m0 + r * HZ * BSZ, e = e0 + r * HZ * RSZ;
+      if (ringr == 0 && kk >= H && kk <= H + TZ - 1 && lr[r] == 1)
+        a = a + resid(sr[e], sb[m - q], sb[m + 1 - q], sb[m + BSY], sb[m - BSY], sb[m + BSZ],
+                      sb[m - BSZ], q ? bv[r].x : bv[r].y);
+    }
+  }
+  // the tile's nodes, with the ghost layer on the domain's faces
+  const int x0 = bx == 0 ? 0 : xs, x1 = bx == ntx - 1 ? n1 + 2 : xs + TX - 1;
+  const int y0 = by == 0 ? 0 : ys, y1 = by == nty - 1 ? n2 + 2 : ys + TY - 1;
+  const int z0 = bz == 0 ? 0 : zs,
+            z1 = tile + ntx * nty >= (int)gridDim.x ? n3 + 2 : zs + TZ - 1;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int kk = h + r * HZ, m = m0 + r * HZ * BSZ, e = e0 + r * HZ * RSZ;
+    const int k = zb + kk, i = xb + 2 * p;
+    if (!mine || j < y0 || j > y1 || k < z0 || k > z1) continue;
+    const T ur = sr[e], uk = sb[m];
+    const T lo = q ? ur : uk, hi = q ? uk : ur;
+    T *d = dst + (off0 + r * step);
+    if (i >= x0 && i < x1) {
+      *reinterpret_cast<V2 *>(d) = V2{lo, hi};
+    } else if (i == x1) {
+      d[0] = lo;
+    } else if (i == x0 - 1 && i < x1) {
+      d[1] = hi;
+    }
+  }
+  if (RES) {
+    for (int d = LEPIC_WAVE / 2; d > 0; d >>= 1) a = a + __shfl_down(a, d);
+    if (__lane_id() == 0) red[threadIdx.x / LEPIC_WAVE] = a;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double b = 0.0;
+      for (int w = 0; w < NT / LEPIC_WAVE; ++w) b = b + red[w];
+      sc.partials[(int64_t)(slot & 1) * sc.nparts + blockIdx.x] = b;
+    }
+  }
+}
+
 // r_pbc: residual of plane k = m, the periodic image of k = 0
 // (mg.f90:322-392).  The reference loops over coarse (j, i) and each
 // iteration writes up to nine overlapping entries, the later iteration
@@ -500,9 +796,14 @@ __global__ __launch_bounds__(BLOCK) void k_restrict(KLevelT<T> F, KLevelT<T> C, 
 // per node instead of once per coarse neighbour that reads it, and the
 // coarse correction u zeroed (nc nodes).  The restriction's few getres
 // calls outside that range (the n2 wrap at i = n1 + 2) still go to getres.
+// fin != nullptr: block 0 also closes the sor_rb before it (slots_finish).
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_getres(KLevelT<T> F, T *R, T *cu, int64_t nc,
-                                                  int flag_nmn) {
+                                                  int flag_nmn, SlotCtl sc, MGCtl *fin) {
+  if (fin && blockIdx.x == 0) {
+    __shared__ double red[BLOCK / LEPIC_WAVE];
+    slots_finish<BLOCK>(sc, fin, red);
+  }
   const int64_t t = blockIdx.x * (int64_t)BLOCK + threadIdx.x;
   if (t < nc) cu[t] = T(0);
   const KGrid &g = F.g;
@@ -556,7 +857,12 @@ __device__ inline void prolong_node(const KLevelT<T, B> &F, const KLevelT<T, B> 
 }
 
 template <class T>
-__global__ __launch_bounds__(BLOCK) void k_prolong(KLevelT<T> F, KLevelT<T> C) {
+__global__ __launch_bounds__(BLOCK) void k_prolong(KLevelT<T> F, KLevelT<T> C, SlotCtl sc,
+                                                   MGCtl *fin) {
+  if (fin && blockIdx.x == 0) {   // close the coarse level's sor_rb
+    __shared__ double red[BLOCK / LEPIC_WAVE];
+    slots_finish<BLOCK>(sc, fin, red);
+  }
   prolong_node(F, C, blockIdx.x * (int64_t)BLOCK + threadIdx.x);
 }
 
@@ -767,6 +1073,29 @@ __global__ void k_fill_d(T *a, int64_t n, T v) {
   if (i < n) a[i] = v;
 }
 
+// Tiles of the whole-sweep launches (k_sweep): the large one fills a CU's LDS
+// (155 KB in FP64) and relaxes the fewest halo nodes, the small one spreads a
+// level that would leave CUs idle.  Per sweep: 22 us against 10 at 64^3 (32
+// and 256 blocks), 28 against 42 at 128^3 (256 and 1800), 239 against 263 at
+// 256^3; a launch of one large block per CU takes 28 us whatever its count, so
+// the line is where the small tiles need as long, near 112^3 (196 blocks).
+constexpr int BIG_X = 33, BIG_Y = 17, BIG_Z = 17, BIG_NT = 1024;
+constexpr int SML_X = 17, SML_Y = 9, SML_Z = 9, SML_NT = 768;
+
+struct SweepGrid {
+  int nx, ny, nz;
+  bool big;
+  unsigned blocks() const { return (unsigned)nx * (unsigned)ny * (unsigned)nz; }
+};
+
+inline SweepGrid sweep_grid(const KGrid &g) {
+  auto tiles = [](int n, int t) { return (n + 1 + t - 1) / t; };
+  SweepGrid w{tiles(g.n1, BIG_X), tiles(g.n2, BIG_Y), tiles(g.n3, BIG_Z), true};
+  if ((int64_t)w.nx * w.ny * w.nz < 192)
+    w = SweepGrid{tiles(g.n1, SML_X), tiles(g.n2, SML_Y), tiles(g.n3, SML_Z), false};
+  return w;
+}
+
 template <class T>
 struct Solver {
   lepic_ctx *ctx;
@@ -784,6 +1113,13 @@ struct Solver {
   // the fine residual of a restriction (the finest level's ghosted size), or
   // nullptr: the restriction forms it per coarse node
   T *resbuf = nullptr;
+  // the second u array of the levels that run whole sweeps per launch
+  // (nullptr: one launch per colour), and the sweeps' exit bookkeeping
+  T *u2[MAX_LEVELS] = {};
+  SlotState *slot_state = nullptr;
+  double *slot_partials = nullptr;   // 2 x the most blocks of a sweep launch
+  MGCtl *fin = nullptr;              // the level whose last sor_rb is still to be closed
+  SlotCtl fin_sc = {};
 
   void coarse(double eps, int kmg) {
     CoarseArgs<T> A;
@@ -840,8 +1176,37 @@ struct Solver {
                        dig, nr);
   }
 
+  // A level sweeps in whole-sweep launches when it has no periodic ghosts to
+  // copy between the colours; the coarsest level's sor_rb (another exit rule,
+  // up to 10^6 sweeps) keeps one launch per colour.
+  bool tiled(int l, int dig) const { return !flag_pbc && dig != 0 && u2[l]; }
+
+  void sor_slots(int l) {
+    const KLevelT<T> &Lv = L[l];
+    const SweepGrid w = sweep_grid(Lv.g);
+    SlotCtl sc{slot_state, slot_partials, (int64_t)w.blocks()};
+    for (int s = 0; s < SLOTS; ++s) {
+      const T *src = (s & 1) ? u2[l] : Lv.u;
+      T *dst = (s & 1) ? Lv.u : u2[l];
+      if (w.big)
+        hipLaunchKernelGGL((k_sweep<T, BIG_X, BIG_Y, BIG_Z, BIG_NT, 2, 1, true>), dim3(w.blocks()),
+                           dim3(BIG_NT), 0, ctx->stream, Lv, src, dst, omega, w.nx, w.ny, 0, s, sc,
+                           &ctl[l]);
+      else
+        hipLaunchKernelGGL((k_sweep<T, SML_X, SML_Y, SML_Z, SML_NT, 4, 1, true>), dim3(w.blocks()),
+                           dim3(SML_NT), 0, ctx->stream, Lv, src, dst, omega, w.nx, w.ny, 0, s, sc,
+                           &ctl[l]);
+    }
+    fin = &ctl[l];
+    fin_sc = sc;
+  }
+
   // sor_rb: returns LEPIC_OK; sweeps are counted on the device.
   int sor_rb(int l, double eps, int kmg, int dig) {
+    if (!fixed && tiled(l, dig)) {
+      sor_slots(l);
+      return LEPIC_OK;
+    }
     if (fixed) {
       for (int c = 0; c < (dig == 0 ? nr_coarsest : nr_fixed); ++c) sor_sweep(l, eps, dig, 4, false);
       return LEPIC_OK;
@@ -873,7 +1238,8 @@ struct Solver {
     if (resbuf) {
       const int64_t nres = (int64_t)(g.n1 + 1) * (g.n2 + 1) * (g.n3 + 1);
       hipLaunchKernelGGL(k_getres<T>, dim3(grid_blocks(std::max(nc, nres), BLOCK)), dim3(BLOCK), 0,
-                         ctx->stream, F, resbuf, C.u, nc, flag_nmn);
+                         ctx->stream, F, resbuf, C.u, nc, flag_nmn, fin_sc, fin);
+      fin = nullptr;
     } else {
       hipLaunchKernelGGL(k_fill_d<T>, dim3(grid_blocks(nc, BLOCK)), dim3(BLOCK), 0, ctx->stream,
                          C.u, nc, T(0));
@@ -894,7 +1260,8 @@ struct Solver {
     const KGrid &g = L[l].g;
     int64_t nt = (int64_t)(g.n1 / 2 + 1) * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
     hipLaunchKernelGGL(k_prolong<T>, dim3(grid_blocks(nt, BLOCK)), dim3(BLOCK), 0, ctx->stream,
-                       L[l], L[l + 1]);
+                       L[l], L[l + 1], fin_sc, fin);
+    fin = nullptr;
   }
 
   static int64_t grid_nodes_k(const KGrid &g) {
@@ -934,6 +1301,10 @@ struct Solver {
         }
         if (ng >= 2 && ng - 2 < lc) prolongation(ng - 2);
       }
+    }
+    if (fin) {
+      hipLaunchKernelGGL(k_slots_finish, dim3(1), dim3(BLOCK), 0, ctx->stream, fin_sc, fin);
+      fin = nullptr;
     }
     return LEPIC_OK;
   }
@@ -1011,7 +1382,14 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   // coarse-level storage (kept across calls; labels zeroed once)
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
   const int64_t fine_nodes = ng > 1 ? grid_nodes(g) : 0;   // the restriction's residual
-  size_t need = sizeof(double) * (size_t)(2 * coarse_nodes + max_parts + rp_len + fine_nodes) +
+  // the whole-sweep launches' second u arrays, block residuals and slot states
+  const int64_t u2_nodes = ng > 1 && !mp->flag_pbc ? grid_nodes(g) + coarse_nodes : 0;
+  int64_t sweep_parts = 0;
+  for (int l = 0; l < ng; ++l)
+    sweep_parts = std::max<int64_t>(sweep_parts, sweep_grid(S.L[l].g).blocks());
+  const int64_t slot_len = 2 * sweep_parts + (int64_t)(SLOTS * sizeof(SlotState) / sizeof(double));
+  size_t need = sizeof(double) * (size_t)(2 * coarse_nodes + max_parts + rp_len + fine_nodes +
+                                          u2_nodes + slot_len) +
                 sizeof(int32_t) * (size_t)coarse_nodes + 4096;
   bool same = ctx->mg_mem && ctx->mg_ng == ng && ctx->mg_n[0] == g->n[0] &&
               ctx->mg_n[1] == g->n[1] && ctx->mg_n[2] == g->n[2] && ctx->mg_bytes >= need;
@@ -1033,7 +1411,10 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   S.rp = dmem + max_parts;
   double *lv = S.rp + rp_len;
   S.resbuf = fine_nodes ? lv + 2 * coarse_nodes : nullptr;
-  int32_t *lb = reinterpret_cast<int32_t *>(lv + 2 * coarse_nodes + fine_nodes);
+  double *u2 = lv + 2 * coarse_nodes + fine_nodes;
+  S.slot_state = reinterpret_cast<SlotState *>(u2 + u2_nodes);
+  S.slot_partials = u2 + u2_nodes + (int64_t)(SLOTS * sizeof(SlotState) / sizeof(double));
+  int32_t *lb = reinterpret_cast<int32_t *>(u2 + u2_nodes + slot_len);
   S.L[0].u = phi;
   S.L[0].b = const_cast<double *>(rho);
   S.L[0].bc = const_cast<int32_t *>(bcnd);
@@ -1044,6 +1425,10 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
     lv += 2 * nn;
     S.L[l].bc = lb;
     lb += nn;
+  }
+  for (int l = 0; l < ng && u2_nodes; ++l) {
+    S.u2[l] = u2;
+    u2 += Solver<double>::grid_nodes_k(S.L[l].g);
   }
   S.ctl = reinterpret_cast<MGCtl *>(ctx->d_ctrl + CTRL_MG);
   hipLaunchKernelGGL(k_reset_totals, dim3(1), dim3(64), 0, ctx->stream, S.ctl, MAX_LEVELS);

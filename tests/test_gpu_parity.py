@@ -253,6 +253,45 @@ def test_poisson_bitexact(gpu, oracle, rng, bmaker, pbc, ng, size):
     np.testing.assert_allclose(info_g["res"], info_o["res"], rtol=1e-9)
 
 
+# Whole-sweep launches (k_sweep): tiles of 17 x 9 x 9 nodes and, from 192 of
+# them, 33 x 17 x 17.  n + 1 relaxed nodes per axis: exactly one tile, one node
+# more, a ragged last tile, tiles of one axis only, both tile sizes, and the
+# Neumann rows.  ng = 2 and 3 put one and two levels on them.
+@pytest.mark.parametrize("n,ng,nmn", [((16, 8, 8), 1 + 1, 0), ((18, 10, 8), 2, 0),
+                                      ((32, 16, 16), 3, 0), ((36, 20, 28), 3, 1),
+                                      ((64, 8, 10), 2, 0), ((8, 12, 68), 3, 1),
+                                      ((144, 128, 160), 5, 0), ((96, 112, 160), 5, 1)])
+def test_poisson_tiles_bitexact(gpu, oracle, rng, n, ng, nmn):
+    """phi, sweep counts and V-cycles of the whole-sweep launches against the
+    oracle: phi within 1e-12 of max |phi| (the relaxed nodes' operands and
+    expression are the oracle's; only the residual's summation order differs)."""
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box(n)
+    bc = H.two_electrode_bcnd(n)
+    if nmn:
+        bc[2:n[2] + 1, 2:n[1] + 1, 0:2] = -2
+    rho = np.zeros(cfg.node_shape(n))
+    rho[bc <= 0] = 1e-4 * rng.standard_normal(int((bc <= 0).sum()))
+    phi0 = np.zeros(cfg.node_shape(n))
+    phi0[bc == 2] = 20.0
+    phi0[bc == 3] = -5.0
+    phi_g = torch.as_tensor(phi0.copy(), device=gpu)
+    bc_g, rho_g = torch.as_tensor(bc, device=gpu), torch.as_tensor(rho, device=gpu)
+    phi_o = phi0.copy()
+    st, info_o = oracle.pdesolver(n, h, phi_o, rho, bc, flag_pbc=0, flag_nmn=nmn, ng=ng, eps=1e-8,
+                                  omega=1.4)
+    assert st == 0
+    for graph in (True, True, False):     # capture, replay, eager: the same solve
+        phi_g.copy_(torch.as_tensor(phi0))
+        info_g = F.solve_poisson_legacy(phi_g, bc_g, rho_g, h, n, 20000, 1e-8, 1.4, ng, 0, nmn,
+                                        graph=graph)
+        assert info_g["cycles"] == info_o["cycles"]
+        assert info_g["sweeps"] == info_o["sweeps"]
+        np.testing.assert_allclose(phi_g.cpu().numpy(), phi_o, rtol=1e-12,
+                                   atol=1e-12 * np.abs(phi_o).max())
+        np.testing.assert_allclose(info_g["res"], info_o["res"], rtol=1e-9)
+
+
 def test_loader_host_bitexact(oracle):
     """The product's host loader reproduces the reference loader's ran2 stream."""
     from essaitemporaire_lepic_module_amd import particles as P
