@@ -469,6 +469,7 @@ __global__ __launch_bounds__(NT) void k_sweep(KLevelT<T> L, const T *src, T *dst
   // that need no test of what was read: clamped into the arrays, and nothing
   // that nodes outside the relaxed range bring is used.
   typedef typename Vec2<T>::type V2;
+  typedef typename Vec2<int32_t>::type I2;
   const int64_t off0 = (int64_t)(xb + 2 * p) + g.sy * (int64_t)j + g.sz * (int64_t)(zb + h);
   const int64_t step = HZ * g.sz;
   auto inside = [&](int64_t c) { return c < 0 ? 0 : (c > nodes - 2 ? nodes - 2 : c); };
@@ -489,9 +490,9 @@ __global__ __launch_bounds__(NT) void k_sweep(KLevelT<T> L, const T *src, T *dst
   if (relaxes) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int64_t c = inside(off0 + r * step);
-      lr[r] = L.bc[c + 1 - q];
-      lk[r] = L.bc[c + q];
+      const I2 l2 = *reinterpret_cast<const I2 *>(L.bc + inside(off0 + r * step));
+      lr[r] = q ? l2.x : l2.y;
+      lk[r] = q ? l2.y : l2.x;
     }
   }
   auto read_b = [&](int r) {
@@ -1201,10 +1202,50 @@ struct Solver {
     fin_sc = sc;
   }
 
-  // sor_rb: returns LEPIC_OK; sweeps are counted on the device.
-  int sor_rb(int l, double eps, int kmg, int dig) {
-    if (!fixed && tiled(l, dig)) {
-      sor_slots(l);
+  // nr_fixed sweeps of a level whose u is L[l].u on entry and on return: each
+  // launch writes the other array, which then takes its place (both legs of a
+  // V-cycle issue the same launches, so u is at home again after the second).
+  // zero: u is 0 everywhere and is not read.
+  void sor_fixed(int l, bool zero) {
+    const SweepGrid w = sweep_grid(L[l].g);
+    const SlotCtl none = {};
+    auto launch = [&](auto kernel, int tx, int ty, int tz, int nt) {
+      const KGrid &g = L[l].g;
+      const int nx = (g.n1 + tx) / tx, ny = (g.n2 + ty) / ty, nz = (g.n3 + tz) / tz;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nx * ny * nz), dim3(nt), 0, ctx->stream, L[l],
+                         (const T *)L[l].u, u2[l], omega, nx, ny, zero ? 1 : 0, 0, none,
+                         (MGCtl *)nullptr);
+      std::swap(L[l].u, u2[l]);
+      zero = false;
+    };
+    // Two sweeps a launch on the small tile (launch-bound levels: 7 us against
+    // 2 x 5 at 64^3); large levels are read-bound and take one, on the tile
+    // whose blocks leave room for others on the CU.  FP32 256^3 conjugate
+    // gradients: 33 x 9 x 9 8.9 ms, 33 x 15 x 17 with two sweeps 9.7, 33 x 9 x 9
+    // with two 9.3, 17 x 9 x 9 10.4, one launch per colour 10.9.  FP64 128^3
+    // preconditioner: 33 x 17 x 17 1.27 ms, 33 x 9 x 9 1.31, per colour 1.49.
+    constexpr int LY = sizeof(T) == 4 ? 9 : BIG_Y, LZ = sizeof(T) == 4 ? 9 : BIG_Z,
+                  LNT = sizeof(T) == 4 ? 512 : BIG_NT;
+    for (int c = 0; c < nr_fixed;) {
+      if (w.big) {
+        launch(k_sweep<T, BIG_X, LY, LZ, LNT, 2, 1, false>, BIG_X, LY, LZ, LNT);
+        c += 1;
+      } else if (c + 2 <= nr_fixed) {
+        launch(k_sweep<T, SML_X, SML_Y, SML_Z, 896, 4, 2, false>, SML_X, SML_Y, SML_Z, 896);
+        c += 2;
+      } else {
+        launch(k_sweep<T, SML_X, SML_Y, SML_Z, SML_NT, 4, 1, false>, SML_X, SML_Y, SML_Z, SML_NT);
+        c += 1;
+      }
+    }
+  }
+
+  // sor_rb: returns LEPIC_OK; sweeps are counted on the device.  zero: the
+  // level's u is 0 everywhere.
+  int sor_rb(int l, double eps, int kmg, int dig, bool zero = false) {
+    if (tiled(l, dig)) {
+      if (fixed) sor_fixed(l, zero);
+      else sor_slots(l);
       return LEPIC_OK;
     }
     if (fixed) {
@@ -1271,13 +1312,13 @@ struct Solver {
   // One V-cycle of mg (mg.f90:99-239).  Levels lc..ng-1 run inside
   // k_mg_coarse: the stretch from the down-leg sor_rb on lc to the up-leg
   // sor_rb on lc touches no level above lc and is issued as one launch.
-  int vcycle(int kmg, double epsa) {
+  int vcycle(int kmg, double epsa, bool zero = false) {
     for (int ig = 1; ig <= 2 * ng - 1; ++ig) {
       for (int il = 1; il <= ng - 1 && il <= 11; ++il) {
         const int l = il - 1;
         if (ig < ng && ig == il) {
           if (l < lc) {
-            int st = sor_rb(l, epsa, kmg, ig - ng);
+            int st = sor_rb(l, epsa, kmg, ig - ng, l > 0 || zero);
             if (st) return st;
             restriction(l);
           } else if (l == lc) {
@@ -1604,7 +1645,8 @@ __global__ void k_mix_correct(double *phi, const float *e32, const int32_t *bc, 
 // Set-up shared by the two solves that smooth in FP32: the FP32 correction
 // hierarchy and the FP64 work arrays on ctx->mgx_mem, laid out as
 // [MIX_COLS x MIX_BLOCKS partial sums][8 scalars][nf64 FP64 node arrays]
-// [e32, r32][periodic residual plane][coarse u, b][coarse labels].
+// [e32, r32][periodic residual plane][coarse u, b][fine residual][second u
+// arrays][coarse labels].
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -1671,10 +1713,13 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   }
   const int64_t nodes = grid_nodes(g);
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
+  // the whole-sweep launches' second u arrays
+  const int64_t u2_nodes = ng > 1 && !mp->flag_pbc ? nodes + coarse_nodes : 0;
   const size_t need = sizeof(double) * (size_t)(MIX_COLS * MIX_BLOCKS + 8) +
                       sizeof(double) * (size_t)nf64 * (size_t)nodes +
                       sizeof(T) * (size_t)(2 * nodes + 2 * coarse_nodes + rp_len) +
                       sizeof(T) * (size_t)(ng > 1 ? nodes : 0) +   // the restriction's residual
+                      sizeof(T) * (size_t)u2_nodes +
                       sizeof(int32_t) * (size_t)coarse_nodes + 4096;
   if (!ctx->mgx_mem || ctx->mgx_bytes < need) {
     if (ctx->mgx_mem) {
@@ -1699,7 +1744,12 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   S.rp = lv;
   lv += rp_len;
   S.resbuf = ng > 1 ? lv + 2 * coarse_nodes : nullptr;
-  int32_t *lb = reinterpret_cast<int32_t *>(lv + 2 * coarse_nodes + (ng > 1 ? nodes : 0));
+  T *u2 = lv + 2 * coarse_nodes + (ng > 1 ? nodes : 0);
+  int32_t *lb = reinterpret_cast<int32_t *>(u2 + u2_nodes);
+  for (int l = 0; l < ng && u2_nodes; ++l) {
+    S.u2[l] = u2;
+    u2 += Solver<T>::grid_nodes_k(S.L[l].g);
+  }
   S.L[0].u = M.e32;
   S.L[0].b = M.r32;
   S.L[0].bc = const_cast<int32_t *>(bcnd);
@@ -1747,7 +1797,7 @@ extern "C" int lepic_poisson_solve_mixed(lepic_ctx *ctx, const lepic_grid *g, do
   // captured graph per solve configuration
   auto inner = [&]() -> int {
     for (int c = 0; c < xp->inner_cycles; ++c) {
-      int st = S.vcycle(2, 0.0);
+      int st = S.vcycle(2, 0.0, c == 0);
       if (st) return st;
     }
     hipLaunchKernelGGL(k_mix_correct, dim3(grid_blocks(nodes, 256)), dim3(256), 0, ctx->stream,
@@ -1961,7 +2011,7 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_dir(KLevel L, const T *e32, const
 }
 
 // phi += a p_new, r -= a q (a = scal[3] / scal[2]) on plasma nodes; r32 = r,
-// e32 = 0, p = p_new; the L1 sum of r to partials column 0.
+// e32 = 0 (unless null), p = p_new; the L1 sum of r to partials column 0.
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_pcg_update(double *phi, const int32_t *bc,
                                                       const double *pn, const double *q,
@@ -1982,7 +2032,7 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_update(double *phi, const int32_t
       l1 = l1 + fabs(rv);
     }
     p[t] = pv;
-    e32[t] = T(0);
+    if (e32) e32[t] = T(0);
   }
   const double s = block_sum_d(l1, red);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
@@ -2033,7 +2083,7 @@ int pcg_solve(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   hipStream_t &s = ctx->stream;
   auto iteration = [&]() -> int {
     for (int c = 0; c < xp->inner_cycles; ++c) {
-      int st = S.vcycle(2, 0.0);
+      int st = S.vcycle(2, 0.0, c == 0);
       if (st) return st;
     }
     hipLaunchKernelGGL(k_pcg_zq<T>, dim3(rb), dim3(BLOCK), 0, s, M.e32, q, M.partials, nodes);
@@ -2042,7 +2092,7 @@ int pcg_solve(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
                        M.partials, nodes);
     hipLaunchKernelGGL(k_pcg_sum, dim3(2), dim3(BLOCK), 0, s, M.partials, (int64_t)rb, 2, scal);
     hipLaunchKernelGGL(k_pcg_update<T>, dim3(rb), dim3(BLOCK), 0, s, phi, bcnd, pn, q, p, r, M.r32,
-                       M.e32, scal, M.partials, nodes);
+                       S.tiled(0, -1) ? (T *)nullptr : M.e32, scal, M.partials, nodes);
     hipLaunchKernelGGL(k_pcg_sum, dim3(1), dim3(BLOCK), 0, s, M.partials, (int64_t)rb, 0, scal);
     return LEPIC_OK;
   };

@@ -170,3 +170,29 @@ def test_pcg_warm_start_graph_and_refusals(gpu):
     with pytest.raises(_native.LepicError):
         F.solve_poisson_pcg(phi, torch.as_tensor(bad, device=gpu), rg, h, n3, 20000, 1e-10,
                             1.4, 5)
+
+
+# The fixed sweeps of a level run in whole-sweep launches over tiles unless
+# the walls are flagged periodic; on an all-electrode box that flag changes
+# nothing else, so the two solves have to agree bit for bit.  Sizes: one
+# tile, one node more, ragged last tiles, both tile sizes (the large from 192
+# of 33 x 17 x 17), one and several levels; one sweep per launch, two, both.
+@pytest.mark.parametrize("n,ng,nu", [((16, 8, 8), 2, 2), ((18, 10, 8), 2, 1), ((36, 20, 28), 3, 3),
+                                     ((64, 8, 10), 2, 2), ((8, 12, 68), 3, 2),
+                                     ((144, 136, 160), 4, 2), ((160, 144, 112), 5, 3)])
+def test_mixed_tiles_bitexact(gpu, rng, n, ng, nu):
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box(n)
+    bc = torch.as_tensor(H.two_electrode_bcnd(n), device=gpu)
+    rho = np.zeros(cfg.node_shape(n))
+    rho[1:-1, 1:-1, 1:-1] = 1e-4 * rng.standard_normal(rho[1:-1, 1:-1, 1:-1].shape)
+    rho = torch.where(bc <= 0, torch.as_tensor(rho, device=gpu), 0.0)
+    out = []
+    for pbc, graph in ((1, False), (0, True), (0, False)):
+        phi = torch.where(bc == 2, 20.0, torch.where(bc == 3, -5.0, 0.0)).double()
+        info = F.solve_poisson_mixed(phi, bc, rho, h, n, 4, 1e-13, 1.4, ng, pbc, 0,
+                                     inner_cycles=3, nu=nu, nu_coarsest=8, graph=graph)
+        out.append((phi, info))
+    for phi, info in out[1:]:
+        assert torch.equal(phi, out[0][0])
+        assert info == out[0][1]
