@@ -652,10 +652,13 @@ __global__ void k_rpbc(KLevelT<T> F, T *rp, int flag_nmn) {
 // Restriction (mg.f90:413-718): coarse labels injected from the fine grid and
 // the 27-point full-weighting residual with the reference's neighbour rules.
 // R != nullptr: getres of every node of the fine residual range, formed
-// beforehand by k_getres (the same expression, so the same bits).
+// beforehand (the same expression, so the same bits).  masked: R is 0 on the
+// ghost nodes and on electrodes outside the plane j = n2 (which the wrap of
+// j = 1 reads whatever its label), so that the 27 values need no label.
 template <class T, class LB>
 __device__ inline void restrict_node(const KLevelT<T, LB> &F, const KLevelT<T, LB> &C, const T *rp,
-                                     int flag_nmn, int64_t t, const T *R = nullptr) {
+                                     int flag_nmn, int64_t t, const T *R = nullptr,
+                                     bool masked = false) {
   const KGrid &g = F.g;
   const KGrid &gc = C.g;
   const int m = g.n3;
@@ -679,7 +682,31 @@ __device__ inline void restrict_node(const KLevelT<T, LB> &F, const KLevelT<T, L
   if (kr == 1) bc2[gidx(gc, i, j, 0)] = bc[gidx(g, ir, jr, 0)];
   if (kr == M1) bc2[gidx(gc, i, j, m / 2 + 2)] = bc[gidx(g, ir, jr, m + 2)];
   T re = T(0);
-  if (lab <= 0) {
+  if (lab <= 0 && masked && jr != 1 && (kr != 1 || !rp)) {
+    const int64_t c = gidx(g, ir, jr, kr);
+    T v[3][3][3];
+#pragma unroll
+    for (int b_ = 0; b_ < 3; ++b_) {
+      const bool edge = jr + b_ - 1 == g.n2;
+#pragma unroll
+      for (int c_ = 0; c_ < 3; ++c_)
+#pragma unroll
+        for (int a_ = 0; a_ < 3; ++a_) {
+          const int64_t q = c + (a_ - 1) + g.sy * (b_ - 1) + g.sz * (c_ - 1);
+          v[a_][b_][c_] = R[q];
+          if (edge && bc[q] > 0) v[a_][b_][c_] = T(0);
+        }
+    }
+    auto r = [&](int a, int b_, int c_) { return v[a + 1][b_ + 1][c_ + 1]; };
+    re = (T(8) * r(0, 0, 0) +
+          T(4) * (r(1, 0, 0) + r(-1, 0, 0) + r(0, 1, 0) + r(0, -1, 0) + r(0, 0, 1) + r(0, 0, -1)) +
+          T(2) * (r(1, 1, 0) + r(-1, 1, 0) + r(1, -1, 0) + r(-1, -1, 0) + r(1, 0, 1) + r(-1, 0, 1) +
+                  r(0, 1, 1) + r(0, -1, 1) + r(1, 0, -1) + r(-1, 0, -1) + r(0, 1, -1) +
+                  r(0, -1, -1)) +
+          r(1, 1, 1) + r(-1, 1, 1) + r(1, -1, 1) + r(-1, -1, 1) + r(1, 1, -1) + r(-1, 1, -1) +
+          r(1, -1, -1) + r(-1, -1, -1)) /
+         T(64);
+  } else if (lab <= 0) {
     const int n2 = g.n2;
     const int64_t rs = g.n1 + 2;
     auto B = [&](int a, int b_, int c) { return bc[gidx(g, a, b_, c)]; };
@@ -878,10 +905,11 @@ __global__ __launch_bounds__(BLOCK) void k_prolong(KLevelT<T> F, KLevelT<T> C, S
 // --------------------------------------------------------------------------
 constexpr int CBLOCK = 1024;
 // u, b and the labels of every level the workgroup handles live in its LDS
-// during the launch (2 x 8704 doubles and 8704 int16 labels, 153 KB): each
+// during the launch (2 x 9056 doubles and 9056 int16 labels, 159 KB): each
 // barrier-separated phase then waits on LDS instead of L2.  lc is the first level from which the remaining
 // levels fit.
-constexpr int64_t COARSE_LDS_NODES = 8704;
+constexpr int64_t COARSE_LDS_NODES = 9056;
+constexpr int COARSE_SLOTS = (int)((COARSE_LDS_NODES / 2 + CBLOCK - 1) / CBLOCK);
 
 template <class T>
 struct CoarseArgs {
@@ -926,23 +954,51 @@ __device__ inline KLevelT<T, int16_t> lds_level(const CoarseArgs<T> &A, T *lds, 
   return v;
 }
 
-// Workgroup sum in a fixed order: butterfly within each wave, then the 16
-// wave sums in index order.  Every thread gets the result.
-__device__ inline double wg_sum(double a, double *red) {
-  for (int d = 32; d > 0; d >>= 1) a += __shfl_xor(a, d);
-  const int wave = threadIdx.x / LEPIC_WAVE;
-  if (__lane_id() == 0) red[wave] = a;
-  __syncthreads();
-  double r = 0.0;
-  for (int w = 0; w < CBLOCK / LEPIC_WAVE; ++w) r = r + red[w];
-  __syncthreads();
-  return r;
+// a + the value CTRL (a DPP row operation) brings, 0 where it brings none.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double a) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, ROWS, 0xf, true);
+  return a + __hiloint2double(hi, lo);
 }
 
-// sor_rb (sors.f90:1-535) on level l: at most nr sweeps, exit rules as k_decide
-// (with A.fixed, exactly nr sweeps and no residual).
+__device__ inline double read_lane(double a, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), lane),
+                          __builtin_amdgcn_readlane(__double2loint(a), lane));
+}
+
+// Sum of each 16-lane row in its last lane.
+__device__ inline double row_sum(double a) {
+  a = dpp_add<0x111, 0xf>(a);   // row_shr:1, 2, 4, 8
+  a = dpp_add<0x112, 0xf>(a);
+  a = dpp_add<0x114, 0xf>(a);
+  return dpp_add<0x118, 0xf>(a);
+}
+
+// Sum over a full wave in a fixed order, the same in every lane (register
+// moves: six steps of shuffles through LDS take five times as long).
+__device__ inline double wave_sum(double a) {
+  a = row_sum(a);
+  a = dpp_add<0x142, 0xa>(a);   // row_bcast:15 into rows 1 and 3
+  a = dpp_add<0x143, 0xc>(a);   // row_bcast:31 into rows 2 and 3
+  return read_lane(a, LEPIC_WAVE - 1);
+}
+
+// Workgroup sum in a fixed order, every thread gets it: the waves' sums to
+// red[0..15], one barrier, and a row sum of those.  The next call needs a
+// barrier in between.
+__device__ inline double wg_sum(double a, double *red) {
+  static_assert(CBLOCK / LEPIC_WAVE == 16, "a row of wave sums");
+  a = wave_sum(a);
+  if (__lane_id() == 0) red[threadIdx.x / LEPIC_WAVE] = a;
+  __syncthreads();
+  return read_lane(row_sum(red[__lane_id() & 15]), 15);
+}
+
+// sor_rb (sors.f90:1-535) on level l with periodic walls: at most nr sweeps,
+// exit rules as k_decide (with A.fixed, exactly nr sweeps and no residual).
 template <class T>
-__device__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int dig, int64_t nr,
+__device__ __forceinline__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int dig, int64_t nr,
                           double *red) {
   const KLevelT<T, int16_t> Lv = lds_level(A, S, Lb, l);
   const KGrid &g = Lv.g;
@@ -955,12 +1011,10 @@ __device__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int 
     for (int colour = 0; colour < 2; ++colour) {
       for (int64_t t = threadIdx.x; t < nsor; t += CBLOCK) sor_node(Lv, colour, A.omega, t);
       __syncthreads();
-      if (A.flag_pbc) {
-        for (int64_t t = threadIdx.x; t < npy; t += CBLOCK) per_y_node(Lv, t);
-        __syncthreads();
-        for (int64_t t = threadIdx.x; t < npz; t += CBLOCK) per_z_node(Lv, t);
-        __syncthreads();
-      }
+      for (int64_t t = threadIdx.x; t < npy; t += CBLOCK) per_y_node(Lv, t);
+      __syncthreads();
+      for (int64_t t = threadIdx.x; t < npz; t += CBLOCK) per_z_node(Lv, t);
+      __syncthreads();
     }
     ++ksor;
     if (A.fixed) {
@@ -969,7 +1023,7 @@ __device__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int 
     }
     double a = 0.0;
     for (int64_t t = threadIdx.x; t < nres; t += CBLOCK) a = a + resid_node(Lv, t);
-    res = wg_sum(a, red);
+    res = wg_sum(a, red);   // two barriers and more before red is written again
     bool stop;
     if (dig == 0) stop = (res <= A.eps);
     else stop = (res_s > 0.0 && (res / res_s) <= 0.6);
@@ -986,27 +1040,202 @@ __device__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int 
   }
 }
 
+// One level without periodic walls: sor_rb by the workgroup's first NT
+// threads, and on the way down (restricts) the restriction to level l + 1 by
+// all of them.  Every sweep of the loops that index, read labels and b and
+// sum anew costs 2 us at any size (a chain of LDS reads, 64-bit index
+// products, shuffles and five barriers), so here
+//  - a thread keeps its nodes' offsets, classes, b and u in registers for the
+//    whole sor_rb (SL pairs of a red and a black node; with them b's place in
+//    LDS is free to hold the residual that the restriction reads),
+//  - the residual of the red nodes shares its reads with the next sweep's
+//    relaxation of them, which is taken back if that sweep is not to run: two
+//    barriers per sweep, and no residual where the sweep count ends the sor_rb,
+//  - a level of at most 64 SL nodes per colour is left to one wave, whose LDS
+//    accesses are in order without a barrier.
+// Launch of 16^3 and below, FP64: 98 -> 68 us; 8^3 and below 47 -> 32.
+template <class T, int NT, int SL>
+__device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int dig,
+                                int64_t nr, bool restricts, double *red) {
+  const KLevelT<T, int16_t> Lv = lds_level(A, S, Lb, l);
+  const KGrid &g = Lv.g;
+  const int tid = (int)threadIdx.x;
+  const bool works = NT == CBLOCK || tid < NT;
+  const int sy = (int)g.sy, sz = (int)g.sz;
+  const int ni2 = g.n1 / 2 + 1;
+  const int nsor = ni2 * (g.n2 + 1) * (g.n3 + 1);
+  T *u = Lv.u, *bl = Lv.b;
+  const T omega = A.omega;
+  // per node: LDS offset << 5 | a node (not a filled-up slot) << 4 | first plane
+  // of a Neumann level << 3 | residual wanted by the restriction << 2 | class
+  // (0 not relaxed, 1 plasma, 2 Neumann, 3 other)
+  int pk[2][SL];
+  T bb[2][SL], uc[2][SL];
+  auto sync = [&]() {
+    if (NT == CBLOCK) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  if (works) {
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      pk[0][s] = pk[1][s] = 0;
+      const int t = tid + s * NT;
+      if (t < nsor) {
+        const uint32_t r = mdiv_q((uint32_t)t, Lv.d_h1), rk = mdiv_q(r, Lv.d_n2p1);
+        const int i2 = t - (int)r * ni2, j = 1 + (int)(r - rk * (uint32_t)(g.n2 + 1)),
+                  k = 1 + (int)rk;
+        const int is = 1 + ((j + k) & 1);   // red: i + j + k odd
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int i = (c ? 3 - is : is) + 2 * i2;
+          if (i <= g.n1 + 1) {
+            const int at = i + sy * j + sz * k, lab = Lv.bc[at];
+            const int cls = lab > 0 || (lab == 0 && (k == g.n3 + 1 || j == g.n2 + 1)) ? 0
+                      : (lab == -1 ? 1 : (lab == -2 ? 2 : 3));
+            pk[c][s] = at << 5 | 16 | (i == 1 && A.flag_nmn == 1 ? 8 : 0) |
+                       (lab <= 0 || j == g.n2 ? 4 : 0) | cls;
+          }
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        bb[c][s] = bl[pk[c][s] >> 5];
+        uc[c][s] = u[pk[c][s] >> 5];
+      }
+    }
+    auto relax = [&](int cls, T c, T uw, T ue, T un, T us, T ut, T ub, T b) {
+      if (cls == 2)
+        return (T(1) - omega) * c +
+               div_ac(omega * (b - Lv.an * un - Lv.as * us - T(2) * Lv.ae * ue - Lv.at * ut -
+                               Lv.ab * ub),
+                      Lv);
+      return (T(1) - omega) * c +
+             div_ac(omega * (b - Lv.aw * uw - Lv.an * un - Lv.as * us - Lv.ae * ue - Lv.at * ut -
+                             Lv.ab * ub),
+                    Lv);
+    };
+    double a = 0.0;
+    // one colour: its L1 residual before (pre) or after (post) the relaxation
+    auto phase = [&](auto colour, bool relaxes, bool pre, bool post, T *old) {
+      constexpr int c = decltype(colour)::value;
+#pragma unroll
+      for (int s = 0; s < SL; ++s) {
+        const int cls = pk[c][s] & 3;
+        if (s * NT < nsor && cls) {
+          int at = pk[c][s] >> 5;
+          asm("" : "+v"(at));   // the neighbours' addresses formed here, not kept over the sweeps
+          const T uw = u[at - 1], ue = u[at + 1], un = u[at + sy], us = u[at - sy],
+                  ut = u[at + sz], ub = u[at - sz];
+          auto resid = [&]() {
+            const T rij = bb[c][s] - (Lv.aw * uw + Lv.an * un + Lv.as * us + Lv.ae * ue +
+                                      Lv.ac * uc[c][s] + Lv.at * ut + Lv.ab * ub);
+            a = a + fabs((double)rij);
+          };
+          if (pre && cls == 1) resid();
+          if (relaxes) {
+            if (old) old[s] = uc[c][s];
+            uc[c][s] = relax(cls, uc[c][s], uw, ue, un, us, ut, ub, bb[c][s]);
+            u[at] = uc[c][s];
+          }
+          if (post && cls == 1) resid();
+        }
+      }
+    };
+    const std::integral_constant<int, 0> RED{};
+    const std::integral_constant<int, 1> BLACK{};
+    int64_t ksor = 0;
+    double res = 0.0, res_s = 0.0;
+    phase(RED, true, false, false, nullptr);
+    sync();
+    for (;;) {
+      ++ksor;
+      const bool last = ksor >= nr, judged = !A.fixed && !last;
+      a = 0.0;
+      phase(BLACK, true, false, judged, nullptr);
+      sync();
+      if (last) break;
+      T old[SL];
+      phase(RED, true, judged, false, old);
+      if (judged) {
+        if (NT == CBLOCK) {
+          res = wg_sum(a, red);
+        } else {
+          res = wave_sum(a);
+          sync();
+        }
+        const bool stop = dig == 0 ? res <= A.eps : res_s > 0.0 && (res / res_s) <= 0.6;
+        res_s = res;
+        if (stop) {   // the next sweep's red half is not to be
+#pragma unroll
+          for (int s = 0; s < SL; ++s)
+            if (s * NT < nsor && (pk[0][s] & 3)) {
+              uc[0][s] = old[s];
+              u[pk[0][s] >> 5] = old[s];
+            }
+          sync();
+          break;
+        }
+      } else {
+        sync();
+      }
+    }
+    if (tid == 0 && !A.fixed) A.ctl[l].total += ksor;
+    if (restricts) {
+      // getres (mg.f90:809-848) of every node, 0 on electrodes, in b's place
+      // (the plane j = n2 keeps its electrodes' too: see restrict_node)
+#pragma unroll
+      for (int s = 0; s < SL; ++s)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int at = pk[c][s] >> 5;
+          if (pk[c][s] & 4) {
+            const bool first = pk[c][s] & 8;
+            const T aw = first ? T(0) : Lv.aw, ae = first ? T(2) * Lv.ae : Lv.ae,
+                    uw = first ? T(0) : u[at - 1];
+            bl[at] = bb[c][s] - (aw * uw + ae * u[at + 1] + Lv.an * u[at + sy] + Lv.as * u[at - sy] +
+                                 Lv.ac * uc[c][s] + Lv.at * u[at + sz] + Lv.ab * u[at - sz]);
+          } else if (pk[c][s] & 16) {
+            bl[at] = T(0);
+          }
+        }
+    }
+  }
+  __syncthreads();
+  if (!restricts) return;
+  const KLevelT<T, int16_t> Cv = lds_level(A, S, Lb, l + 1);
+  const int nt = ni2 * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
+  for (int t = tid; t < nt; t += CBLOCK)
+    restrict_node(Lv, Cv, (const T *)nullptr, A.flag_nmn, t, (const T *)bl, true);
+  __syncthreads();
+  if (works) {
+#pragma unroll
+    for (int s = 0; s < SL; ++s)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        if (pk[c][s] & 3) bl[pk[c][s] >> 5] = bb[c][s];
+  }
+  // the up leg's reads of b lie behind further barriers
+}
+
 template <class T>
-__device__ void wg_restriction(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l) {
+__device__ __forceinline__ void wg_restriction(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l) {
   const KLevelT<T, int16_t> F = lds_level(A, S, Lb, l);
   const KLevelT<T, int16_t> C = lds_level(A, S, Lb, l + 1);
   const KGrid &g = F.g;
-  const int64_t nc = ((int64_t)C.g.n1 + 3) * ((int64_t)C.g.n2 + 3) * ((int64_t)C.g.n3 + 3);
-  for (int64_t t = threadIdx.x; t < nc; t += CBLOCK) C.u[t] = T(0);
-  const T *rpp = nullptr;
-  if (A.flag_pbc) {
-    const int64_t nent = ((int64_t)g.n1 + 2) * ((int64_t)g.n2 + 2);
-    for (int64_t t = threadIdx.x; t < nent; t += CBLOCK) rpbc_entry(F, A.rp, A.flag_nmn, t);
-    rpp = A.rp;
-  }
+  const int64_t nent = ((int64_t)g.n1 + 2) * ((int64_t)g.n2 + 2);
+  for (int64_t t = threadIdx.x; t < nent; t += CBLOCK) rpbc_entry(F, A.rp, A.flag_nmn, t);
   __syncthreads();
   const int64_t nt = (int64_t)(g.n1 / 2 + 1) * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
-  for (int64_t t = threadIdx.x; t < nt; t += CBLOCK) restrict_node(F, C, rpp, A.flag_nmn, t);
+  for (int64_t t = threadIdx.x; t < nt; t += CBLOCK) restrict_node(F, C, (const T *)A.rp, A.flag_nmn, t);
   __syncthreads();
 }
 
 template <class T>
-__device__ void wg_prolongation(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l) {  // L[l] += P(L[l+1])
+__device__ __forceinline__ void wg_prolongation(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l) {  // L[l] += P(L[l+1])
   const KLevelT<T, int16_t> F = lds_level(A, S, Lb, l);
   const KLevelT<T, int16_t> C = lds_level(A, S, Lb, l + 1);
   const KGrid &g = F.g;
@@ -1018,12 +1247,11 @@ __device__ void wg_prolongation(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l
 // The V-cycle of mg (mg.f90:1-246) restricted to levels lc..ng-1; the
 // prolongation into level lc-1 is left to the caller.
 // The host sizes lc so that levels lc..ng-1 hold at most COARSE_LDS_NODES
-// nodes together.  u and b of every level are copied in at the start (the
-// global copies of the levels below lc hold what the global-memory version
-// would read: zeros at the ghost nodes no restriction writes, values that
-// the V-cycle overwrites before reading elsewhere), and u of level lc, the
-// only array read after the launch, is copied back at the end.
-template <class T>
+// nodes together.  Level lc's b and labels are copied in at the start; u is 0
+// on every level then, and b 0 at the ghost nodes, which no restriction
+// writes.  u of level lc, the only array read after the launch, is copied back
+// at the end.
+template <class T, bool PBC>
 __global__ __launch_bounds__(CBLOCK) void k_mg_coarse(CoarseArgs<T> A) {
   __shared__ double red[CBLOCK / LEPIC_WAVE];
   __shared__ T lds[2 * COARSE_LDS_NODES];
@@ -1031,34 +1259,57 @@ __global__ __launch_bounds__(CBLOCK) void k_mg_coarse(CoarseArgs<T> A) {
   T *const S = lds;
   int16_t *const Lb = labs;
   const int ng = A.ng;
-  // level lc's labels are the ones the last global restriction wrote; the
-  // coarser levels' global labels are never written (0, as at allocation),
-  // and the workgroup's restrictions write their values into LDS before any
-  // read, leaving 0 where none writes
-  for (int l = A.lc; l < ng; ++l) {
-    T *p = lds + A.lds_off[l];
-    int16_t *q = labs + A.lab_off[l];
-    const int nn = A.lds_nn[l];
-    for (int t = threadIdx.x; t < nn; t += CBLOCK) {
-      p[t] = A.L[l].u[t];
-      p[nn + t] = A.L[l].b[t];
-      q[t] = label16(A.L[l].bc[t]);
+  {
+    constexpr int RL = (int)((COARSE_LDS_NODES + CBLOCK - 1) / CBLOCK);
+    const KLevelT<T> &G = A.L[A.lc];
+    const KGrid &g = G.g;
+    const int nn = A.lds_nn[A.lc], nx = g.n1 + 1, nb = nx * (g.n2 + 1) * (g.n3 + 1);
+    int at[RL];
+    T bv[RL];
+    int32_t lv[RL];
+#pragma unroll
+    for (int r = 0; r < RL; ++r) {   // every read before the first wait
+      const int t = (int)threadIdx.x + r * CBLOCK;
+      lv[r] = t < nn ? G.bc[t] : 0;
+      const uint32_t row = mdiv_q((uint32_t)t, G.d_n1p1), rk = mdiv_q(row, G.d_n2p1);
+      at[r] = t < nb ? (int)gidx(g, 1 + t - (int)row * nx, 1 + (int)(row - rk * (g.n2 + 1)),
+                                 1 + (int)rk)
+                     : -1;
+      bv[r] = at[r] >= 0 ? G.b[at[r]] : T(0);
+    }
+    const int all = A.lds_off[ng - 1] + 2 * A.lds_nn[ng - 1];
+    for (int t = threadIdx.x; t < all; t += CBLOCK) lds[t] = T(0);
+    for (int t = threadIdx.x; t < all / 2; t += CBLOCK) labs[t] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RL; ++r) {
+      const int t = (int)threadIdx.x + r * CBLOCK;
+      if (t < nn) labs[t] = label16(lv[r]);
+      if (at[r] >= 0) lds[nn + at[r]] = bv[r];
     }
   }
   __syncthreads();
   const int64_t nr = A.fixed ? A.nr_fixed : 4;
-  for (int l = A.lc; l <= ng - 2; ++l) {
-    wg_sor_rb(A, S, Lb, l, l + 1 - ng, nr, red);
-    __syncthreads();
-    wg_restriction(A, S, Lb, l);
-  }
-  wg_sor_rb(A, S, Lb, ng - 1, 0, A.fixed ? A.nr_coarsest : (A.first_cycle ? 1000000 : 4), red);
-  __syncthreads();
-  if (ng - 2 >= A.lc) wg_prolongation(A, S, Lb, ng - 2);
-  for (int l = ng - 2; l >= A.lc; --l) {
-    wg_sor_rb(A, S, Lb, l, ng - 1 - l, nr, red);
-    __syncthreads();
-    if (l - 1 >= A.lc) wg_prolongation(A, S, Lb, l - 1);
+  const int64_t nr_last = A.fixed ? A.nr_coarsest : (A.first_cycle ? 1000000 : 4);
+  // down from lc, the coarsest level, back up (one place that calls each
+  // routine: inlined, the arguments stay in scalar memory)
+  const int m = ng - 1 - A.lc;
+  for (int v = 0; v <= 2 * m; ++v) {
+    const int l = v <= m ? A.lc + v : A.lc + 2 * m - v;
+    const int dig = v == m ? 0 : (v < m ? l + 1 - ng : ng - 1 - l);
+    const int64_t count = v == m ? nr_last : nr;
+    if (v > m) wg_prolongation(A, S, Lb, l);
+    if (PBC) {
+      wg_sor_rb(A, S, Lb, l, dig, count, red);
+      __syncthreads();
+      if (v < m) wg_restriction(A, S, Lb, l);
+    } else {
+      const KGrid &g = A.L[l].g;
+      if ((g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1) <= 2 * LEPIC_WAVE)
+        wg_level<T, LEPIC_WAVE, 2>(A, S, Lb, l, dig, count, v < m, red);
+      else
+        wg_level<T, CBLOCK, COARSE_SLOTS>(A, S, Lb, l, dig, count, v < m, red);
+    }
   }
   __syncthreads();
   {
@@ -1148,7 +1399,10 @@ struct Solver {
       A.lab_off[l] = off / 2;
       off += 2 * A.lds_nn[l];
     }
-    hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
+    if (flag_pbc)
+      hipLaunchKernelGGL((k_mg_coarse<T, true>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
+    else
+      hipLaunchKernelGGL((k_mg_coarse<T, false>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
   }
 
   // One sweep; first: the sor_rb's first, whose red half arms ctl[l].

@@ -292,6 +292,47 @@ def test_poisson_tiles_bitexact(gpu, oracle, rng, n, ng, nmn):
         np.testing.assert_allclose(info_g["res"], info_o["res"], rtol=1e-9)
 
 
+# The one-workgroup levels (wg_level): one wave up to 128 nodes of a colour
+# (6 x 4 x 4: 100, 6 x 6 x 4: 140), one to five per thread (34 x 32 x 4 is 3060
+# of a colour, 10 x 80 x 4 2430, 2 x 2 x 340 6138 nodes in all), electrodes
+# inside, and rows labelled 0 at j = 1 and k = 1, whose restriction reads the
+# plane j = n2 (electrodes in it too) and nothing below k = 1.
+@pytest.mark.parametrize("n,ng,zero,nmn", [((12, 8, 8), 3, 0, 0), ((12, 12, 8), 3, 1, 0),
+                                           ((20, 12, 16), 3, 1, 1), ((68, 64, 8), 3, 0, 0),
+                                           ((20, 160, 8), 3, 1, 0), ((4, 4, 680), 2, 0, 0),
+                                           ((32, 32, 32), 5, 1, 0)])
+def test_poisson_coarse_levels_bitexact(gpu, oracle, rng, n, ng, zero, nmn):
+    """phi within 1e-12 of max |phi| and the sweep counts of every level equal
+    to the oracle's (same operands and expressions; only the residual's
+    summation order differs)."""
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box(n)
+    bc = H.two_electrode_bcnd(n)
+    inside = bc == -1
+    bc[inside & (rng.random(bc.shape) < 0.1)] = 4
+    if zero:
+        bc[2:n[2] + 1, 0:2, 2:n[0] + 1] = 0
+        bc[0:2, 2:n[1] + 1, 2:n[0] + 1] = 0
+    if nmn:
+        bc[2:n[2] + 1, 2:n[1] + 1, 0:2] = -2
+    rho = np.zeros(cfg.node_shape(n))
+    rho[bc <= 0] = 1e-4 * rng.standard_normal(int((bc <= 0).sum()))
+    phi0 = np.zeros(cfg.node_shape(n))
+    phi0[bc == 2] = 20.0
+    phi0[bc == 4] = -5.0
+    phi_o = phi0.copy()
+    st, info_o = oracle.pdesolver(n, h, phi_o, rho, bc, flag_pbc=0, flag_nmn=nmn, ng=ng, eps=1e-8,
+                                  omega=1.4, ncycl=6)
+    assert st == 0
+    phi_g = torch.as_tensor(phi0, device=gpu)
+    info_g = F.solve_poisson_legacy(phi_g, torch.as_tensor(bc, device=gpu),
+                                    torch.as_tensor(rho, device=gpu), h, n, 6, 1e-8, 1.4, ng, 0, nmn)
+    assert info_g["cycles"] == info_o["cycles"]
+    assert info_g["sweeps"] == info_o["sweeps"]
+    np.testing.assert_allclose(phi_g.cpu().numpy(), phi_o, rtol=1e-12,
+                               atol=1e-12 * np.abs(phi_o).max())
+
+
 def test_loader_host_bitexact(oracle):
     """The product's host loader reproduces the reference loader's ran2 stream."""
     from essaitemporaire_lepic_module_amd import particles as P
