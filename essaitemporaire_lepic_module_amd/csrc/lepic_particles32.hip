@@ -732,9 +732,8 @@ __global__ void k_round4(const double4 *__restrict__ a, float4 *b, int64_t nodes
 //   claim  -- every tile takes a run of slots per cell with one atomic and
 //             writes its particles' source indices there (order within a
 //             cell is the atomics' order at this point);
-//   rank   -- one wave per cell puts the cell's source indices in ascending
-//             order, which is the stable order;
-//   gather -- every slot copies its particle from the source index.
+//   place  -- the lanes of a cell put its source indices in ascending order,
+//             which is the stable order, and copy the particles into it.
 // ---------------------------------------------------------------------------
 constexpr int SBOX = 8192;   // cells of a tile's counting box (32 KB)
 
@@ -947,23 +946,34 @@ __global__ __launch_bounds__(BLOCK) void k_sort_claim(KG32 g, const int32_t *__r
     if (c[q] >= 0) idx[bs.cnt[l[q]] + rank[q]] = (int32_t)(i0 + q);
 }
 
-// Rank: one wave per cell sorts the cell's source indices ascending (they are
-// distinct).  Up to 256: a bitonic sort of the cell padded to 64 x R
-// entries, R per lane (position q*64 + lane in register q: partners 64 or
-// more apart in the same lane, nearer ones across lanes); larger cells:
+// Place: W lanes per cell sort its source indices ascending (they are
+// distinct) in registers, bitonic over the cell padded to W x R entries
+// (position q*W + ln in register q: partners W or more apart in the same
+// lane, nearer ones across lanes), and copy the particles; cells beyond 4 W:
 // each index's rank counted over the cell.
-template <int R>
-__device__ inline void wave_bitonic(int v[R], int lane) {
+//
+// A cell's particles come from the lines of all cells around it, so the copy
+// is bound by how often a source line is fetched.  Slot order, blocks in turn
+// over the XCDs, fetches every line 5.5 times (24 GB and 4.3 ms for 134M
+// electrons, besides 0.9 ms for a separate sort of the indices).  Here the
+// cells in flight on an XCD are a brick (16 x 8 x 8: about what its 32 CUs
+// hold at once), whose sources and their neighbours fit its 4 MB L2: fetched 2.4
+// times, 4.1 ms for both (5.3M ions on 93 x 61 x 47: 139 -> 76 us); what is left is
+// the rate of scattered reads a CU keeps in flight.
+constexpr int BRX = 16, BRY = 8, BRZ = 8;
+
+template <int W, int R>
+__device__ inline void cell_bitonic(int v[R], int ln) {
 #pragma unroll
-  for (int k = 2; k <= 64 * R; k <<= 1) {
+  for (int k = 2; k <= W * R; k <<= 1) {
 #pragma unroll
     for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= 64) {
-        const int r = j / 64;
+      if (j >= W) {
+        const int r = j / W;
 #pragma unroll
         for (int q = 0; q < R; ++q) {
           if ((q & r) != 0) continue;
-          const int p = q * 64 + lane;
+          const int p = q * W + ln;
           const bool up = (p & k) == 0;
           const int a = v[q], b = v[q | r];
           v[q] = up ? min(a, b) : max(a, b);
@@ -972,10 +982,10 @@ __device__ inline void wave_bitonic(int v[R], int lane) {
       } else {
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-          const int p = q * 64 + lane;
+          const int p = q * W + ln;
           const int o = __shfl_xor(v[q], j);
           const bool up = (p & k) == 0;
-          const bool low = (lane & j) == 0;
+          const bool low = (ln & j) == 0;
           v[q] = (low == up) ? min(v[q], o) : max(v[q], o);
         }
       }
@@ -983,75 +993,61 @@ __device__ inline void wave_bitonic(int v[R], int lane) {
   }
 }
 
-template <int R>
-__device__ inline void rank_small(const int32_t *__restrict__ idx, int32_t *sidx, int64_t b, int s,
-                                  int lane) {
-  int v[R];
-#pragma unroll
-  for (int q = 0; q < R; ++q) v[q] = q * 64 + lane < s ? idx[b + q * 64 + lane] : 0x7FFFFFFF;
-  wave_bitonic<R>(v, lane);
-#pragma unroll
-  for (int q = 0; q < R; ++q)
-    if (q * 64 + lane < s) sidx[b + q * 64 + lane] = v[q];
+__device__ inline void place_one(const KP32 &src, const KP32 &dst, int c, int64_t to, int from) {
+  const float fx = src.fx[from], fy = src.fy[from], fz = src.fz[from];
+  const float vx = src.vx[from], vy = src.vy[from], vz = src.vz[from];
+  dst.cell[to] = c;
+  dst.fx[to] = fx; dst.fy[to] = fy; dst.fz[to] = fz;
+  dst.vx[to] = vx; dst.vy[to] = vy; dst.vz[to] = vz;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_sort_rank(const int32_t *__restrict__ count,
-                                                     const int32_t *__restrict__ start,
-                                                     int64_t ncells, const int32_t *__restrict__ idx,
-                                                     int32_t *sidx) {
-  const int64_t c = (int64_t)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
-  if (c >= ncells) return;
-  const int lane = __lane_id();
-  const int s = count[c];
-  const int64_t b = start[c];
-  if (s == 0) return;
-  if (s <= 64) {
-    rank_small<1>(idx, sidx, b, s, lane);
-  } else if (s <= 128) {
-    rank_small<2>(idx, sidx, b, s, lane);
-  } else if (s <= 256) {
-    rank_small<4>(idx, sidx, b, s, lane);
+template <int W, int R>
+__device__ inline void place_cell(const KP32 &src, const KP32 &dst, const int32_t *__restrict__ idx,
+                                  int c, int64_t b, int s, int ln) {
+  int v[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) v[q] = q * W + ln < s ? idx[b + q * W + ln] : 0x7FFFFFFF;
+  cell_bitonic<W, R>(v, ln);
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+    if (q * W + ln < s) place_one(src, dst, c, b + q * W + ln, v[q]);
+}
+
+template <int W>
+__global__ __launch_bounds__(BLOCK) void k_sort_place(KG32 g, KP32 src, KP32 dst,
+                                                      const int32_t *__restrict__ count,
+                                                      const int32_t *__restrict__ start,
+                                                      const int32_t *__restrict__ idx, int bricks_x,
+                                                      int bricks_y) {
+  // consecutive bricks on one XCD (the grid is a multiple of LEPIC_XCDS blocks)
+  constexpr int CELLS = BLOCK / W, BLOCKS = BRX * BRY * BRZ / CELLS;   // per block, per brick
+  const int t = ((int)blockIdx.x % LEPIC_XCDS) * ((int)gridDim.x / LEPIC_XCDS) +
+                (int)blockIdx.x / LEPIC_XCDS;
+  const int brick = t / BLOCKS, l = (t - brick * BLOCKS) * CELLS + (int)threadIdx.x / W;
+  const int br = brick / bricks_x, bz = br / bricks_y;
+  const int cx = (brick - br * bricks_x) * BRX + l % BRX,
+            cy = (br - bz * bricks_y) * BRY + l / BRX % BRY, cz = bz * BRZ + l / (BRX * BRY);
+  const int ln = (int)threadIdx.x % W;
+  int c = 0, s = 0;
+  int64_t b = 0;
+  if (cx < g.n1 && cy < g.n2 && cz < g.n3) {
+    c = cx + g.n1 * (cy + g.n2 * cz);
+    s = count[c];
+    b = start[c];
+  }
+  if (!__any(s > W)) {
+    place_cell<W, 1>(src, dst, idx, c, b, s, ln);
+  } else if (!__any(s > 2 * W)) {
+    place_cell<W, 2>(src, dst, idx, c, b, s, ln);
+  } else if (!__any(s > 4 * W)) {
+    place_cell<W, 4>(src, dst, idx, c, b, s, ln);
   } else {
-    for (int e = lane; e < s; e += 64) {
+    for (int e = ln; e < s; e += W) {
       const int v = idx[b + e];
       int r = 0;
       for (int j = 0; j < s; ++j) r += idx[b + j] < v ? 1 : 0;
-      sidx[b + r] = v;
+      place_one(src, dst, c, b + r, v);
     }
-  }
-}
-
-// Four destination slots per thread: one 16-byte read of the source slots,
-// the 28 scattered reads in flight together, 16-byte stores (sidx and the
-// destination arrays are 16-byte aligned at multiples of 4 slots).
-__global__ __launch_bounds__(BLOCK) void k_sort_gather(KP32 src, KP32 dst,
-                                                       const int32_t *__restrict__ sidx,
-                                                       int64_t m) {
-  const int64_t d0 = (blockIdx.x * (int64_t)BLOCK + threadIdx.x) * 4;
-  if (d0 >= m) return;
-  if (d0 + 4 <= m) {
-    const int4 j = *reinterpret_cast<const int4 *>(sidx + d0);
-    const int4 c = make_int4(src.cell[j.x], src.cell[j.y], src.cell[j.z], src.cell[j.w]);
-    const float4 fx = make_float4(src.fx[j.x], src.fx[j.y], src.fx[j.z], src.fx[j.w]);
-    const float4 fy = make_float4(src.fy[j.x], src.fy[j.y], src.fy[j.z], src.fy[j.w]);
-    const float4 fz = make_float4(src.fz[j.x], src.fz[j.y], src.fz[j.z], src.fz[j.w]);
-    const float4 vx = make_float4(src.vx[j.x], src.vx[j.y], src.vx[j.z], src.vx[j.w]);
-    const float4 vy = make_float4(src.vy[j.x], src.vy[j.y], src.vy[j.z], src.vy[j.w]);
-    const float4 vz = make_float4(src.vz[j.x], src.vz[j.y], src.vz[j.z], src.vz[j.w]);
-    *reinterpret_cast<int4 *>(dst.cell + d0) = c;
-    *reinterpret_cast<float4 *>(dst.fx + d0) = fx;
-    *reinterpret_cast<float4 *>(dst.fy + d0) = fy;
-    *reinterpret_cast<float4 *>(dst.fz + d0) = fz;
-    *reinterpret_cast<float4 *>(dst.vx + d0) = vx;
-    *reinterpret_cast<float4 *>(dst.vy + d0) = vy;
-    *reinterpret_cast<float4 *>(dst.vz + d0) = vz;
-    return;
-  }
-  for (int64_t d = d0; d < m; ++d) {
-    const int64_t j = sidx[d];
-    dst.cell[d] = src.cell[j];
-    dst.fx[d] = src.fx[j]; dst.fy[d] = src.fy[j]; dst.fz[d] = src.fz[j];
-    dst.vx[d] = src.vx[j]; dst.vy[d] = src.vy[j]; dst.vz[d] = src.vz[j];
   }
 }
 
@@ -1279,14 +1275,12 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
   }
   const int64_t ncells = (int64_t)g->n[0] * g->n[1] * g->n[2];
   const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
-  // scratch: count, start, cursor (ncells each), block sums, idx and sidx (n each)
-  const size_t words = (size_t)(3 * ncells + nb + 2 * n + 64);
+  // scratch: count, start, cursor (ncells each), block sums, idx (n)
+  const size_t words = (size_t)(3 * ncells + nb + n + 64);
   int32_t *w = reinterpret_cast<int32_t *>(lepic_scratch(ctx, sizeof(int32_t) * words, 0));
   if (!w) return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: scratch");
   int32_t *count = w, *start = w + ncells, *cursor = w + 2 * ncells, *bsum = w + 3 * ncells;
   int32_t *idx = bsum + nb + 16;
-  idx += (16 - (reinterpret_cast<uintptr_t>(idx) / 4) % 16) % 16;
-  int32_t *sidx = idx + ((n + 15) & ~(int64_t)15);   // 64-byte aligned, like idx
   int64_t *total = ctx->d_ctrl + CTRL_COUNT_OUT;
   const KG32 kg = make_kg32(g, 0.0);
   const hipStream_t s = ctx->stream;
@@ -1301,17 +1295,24 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
                      ncells);
   hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, src->cell,
                      n, cursor, idx);
-  hipLaunchKernelGGL(k_sort_rank, dim3(grid_blocks(ncells, BLOCK / 64)), dim3(BLOCK), 0, s, count,
-                     start, ncells, idx, sidx);
+  // lanes per cell: the mean cell and twice its spread in one entry per lane
+  const double mean = (double)n / (double)ncells, wide = mean + 2.0 * std::sqrt(mean);
+  const int bx = (g->n[0] + BRX - 1) / BRX, by = (g->n[1] + BRY - 1) / BRY,
+            bz = (g->n[2] + BRZ - 1) / BRZ;
+  auto place = [&](auto kernel, int w) {
+    const int64_t blocks = (int64_t)bx * by * bz * (BRX * BRY * BRZ * w / BLOCK);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((blocks + LEPIC_XCDS - 1) / LEPIC_XCDS * LEPIC_XCDS)),
+                       dim3(BLOCK), 0, s, kg, kp32(src), kp32(dst), count, start, idx, bx, by);
+  };
+  if (wide <= 8.0) place(k_sort_place<8>, 8);
+  else if (wide <= 16.0) place(k_sort_place<16>, 16);
+  else if (wide <= 32.0) place(k_sort_place<32>, 32);
+  else place(k_sort_place<64>, 64);
   LEPIC_LAUNCH_CHECK(ctx, "sort32 passes");
   LEPIC_HIP(ctx, hipMemcpyAsync(ctx->h_pinned, total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   LEPIC_HIP(ctx, hipStreamSynchronize(s));
   const int64_t m = ctx->h_pinned[0];
   if (m < 0 || m > n) return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: inconsistent count");
-  if (m > 0)
-    hipLaunchKernelGGL(k_sort_gather, dim3(grid_blocks((m + 3) / 4, BLOCK)), dim3(BLOCK), 0, s,
-                       kp32(src), kp32(dst), sidx, m);
-  LEPIC_LAUNCH_CHECK(ctx, "k_sort_gather");
   dst->n = m;
   return LEPIC_OK;
 }

@@ -177,6 +177,32 @@ def test_sort32_stable_bitexact(gpu, oracle, rng, case):
     _same32(g, ref)
 
 
+# k_sort_place: 8, 16, 32 and 64 lanes per cell (mean 2, 6, 18, 60); one and
+# two entries per lane, four (cells of 22 and 210), more (96 and 5018); bricks
+# of 16 x 8 x 8 cells whole, ragged and cut to a row.
+@pytest.mark.parametrize("n,mean,crowd", [((16, 8, 8), 2, 0), ((17, 9, 10), 2, 20),
+                                          ((33, 7, 3), 6, 90), ((9, 20, 17), 18, 0),
+                                          ((18, 16, 9), 60, 150), ((50, 1, 1), 18, 5000),
+                                          ((1, 1, 40), 60, 0)])
+def test_sort32_place_bitexact(gpu, oracle, rng, n, mean, crowd):
+    """The stable order with holes dropped, exactly, and every field moved."""
+    from essaitemporaire_lepic_module_amd import particles32 as P32
+    n, h = H.box(n)
+    cells = n[0] * n[1] * n[2]
+    count = mean * cells + crowd
+    q, _ = _pair(oracle, P32, rng, n, h, count)
+    a = q.arrays()
+    a["cell"][:] = rng.integers(0, cells, count)
+    a["cell"][rng.permutation(count)[:crowd]] = cells // 2
+    a["cell"][rng.random(count) < 0.03] = -1
+    q = oracle.Particles32(count + 16).set(*(a[k] for k in oracle.FIELDS32))
+    g = P32.ParticleSet32(count + 16, gpu).from_host(*(a[k] for k in oracle.FIELDS32))
+    ref = oracle.sort32(n, h, q)
+    P32.sort32(g, n, h)
+    assert g.n == ref.n
+    _same32(g, ref)
+
+
 def test_collisions32_deposit_exact(gpu, oracle, rng):
     """MCC on FP32 sets (cfg2's argon chemistry): products and kills adjust
     the fixed-point density exactly -- afterwards it equals a fresh deposit
