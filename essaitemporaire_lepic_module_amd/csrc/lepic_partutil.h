@@ -30,14 +30,24 @@ inline KBC kbc(const lepic_bc_params *b) {
   return k;
 }
 
-__device__ inline int wave_min(int v) {
-  for (int d = 32; d > 0; d >>= 1) v = min(v, __shfl_xor(v, d));
-  return v;
-}
-__device__ inline int wave_max(int v) {
-  for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d));
-  return v;
-}
+// Reductions of a full wave by DPP row operations (row_shr:1, 2, 4, 8, then
+// row_bcast:15 and :31, the result in lane 63, handed to every lane): register
+// moves instead of six shuffles through LDS.  A lane without a source takes
+// old.  Every lane of the wave calls them.
+#define LEPIC_WAVE_REDUCE(name, old, expr)                                                    \
+  __device__ inline int name(int v) {                                                         \
+    { int o = __builtin_amdgcn_update_dpp(old, v, 0x111, 0xf, 0xf, false); v = expr; }        \
+    { int o = __builtin_amdgcn_update_dpp(old, v, 0x112, 0xf, 0xf, false); v = expr; }        \
+    { int o = __builtin_amdgcn_update_dpp(old, v, 0x114, 0xf, 0xf, false); v = expr; }        \
+    { int o = __builtin_amdgcn_update_dpp(old, v, 0x118, 0xf, 0xf, false); v = expr; }        \
+    { int o = __builtin_amdgcn_update_dpp(old, v, 0x142, 0xa, 0xf, false); v = expr; }        \
+    { int o = __builtin_amdgcn_update_dpp(old, v, 0x143, 0xc, 0xf, false); v = expr; }        \
+    return __builtin_amdgcn_readlane(v, LEPIC_WAVE - 1);                                      \
+  }
+LEPIC_WAVE_REDUCE(wave_min, v, min(v, o))
+LEPIC_WAVE_REDUCE(wave_max, v, max(v, o))
+LEPIC_WAVE_REDUCE(wave_sum_i, 0, v + o)
+#undef LEPIC_WAVE_REDUCE
 
 __device__ inline double wave_sum_d(double v) {
   for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
