@@ -651,6 +651,41 @@ __global__ void k_rpbc(KLevelT<T> F, T *rp, int flag_nmn) {
 
 // Restriction (mg.f90:413-718): coarse labels injected from the fine grid and
 // the 27-point full-weighting residual with the reference's neighbour rules.
+
+// The labels of coarse node (i, j, k) and of the ghost nodes next to it; the
+// node's own.
+template <class T, class LB>
+__device__ inline LB restrict_labels(const KLevelT<T, LB> &F, const KLevelT<T, LB> &C, int i, int j,
+                                     int k) {
+  const KGrid &g = F.g, &gc = C.g;
+  const int ir = 2 * i - 1, jr = 2 * j - 1, kr = 2 * k - 1;
+  const LB *bc = F.bc;
+  LB *bc2 = C.bc;
+  const LB lab = bc[gidx(g, ir, jr, kr)];
+  bc2[gidx(gc, i, j, k)] = lab;
+  if (ir == 1) bc2[gidx(gc, 0, j, k)] = bc[gidx(g, 0, jr, kr)];
+  if (ir == g.n1 + 1) bc2[gidx(gc, g.n1 / 2 + 2, j, k)] = bc[gidx(g, g.n1 + 2, jr, kr)];
+  if (jr == 1) bc2[gidx(gc, i, 0, k)] = bc[gidx(g, ir, 0, kr)];
+  if (jr == g.n2 + 1) bc2[gidx(gc, i, g.n2 / 2 + 2, k)] = bc[gidx(g, ir, g.n2 + 2, kr)];
+  if (kr == 1) bc2[gidx(gc, i, j, 0)] = bc[gidx(g, ir, jr, 0)];
+  if (kr == g.n3 + 1) bc2[gidx(gc, i, j, g.n3 / 2 + 2)] = bc[gidx(g, ir, jr, g.n3 + 2)];
+  return lab;
+}
+
+// The weighted sum; r(a, b, c): the residual at that offset, 0 where the
+// reference takes none.
+template <class T, class RD>
+__device__ inline T restrict_sum(RD r) {
+  return (T(8) * r(0, 0, 0) +
+          T(4) * (r(1, 0, 0) + r(-1, 0, 0) + r(0, 1, 0) + r(0, -1, 0) + r(0, 0, 1) + r(0, 0, -1)) +
+          T(2) * (r(1, 1, 0) + r(-1, 1, 0) + r(1, -1, 0) + r(-1, -1, 0) + r(1, 0, 1) + r(-1, 0, 1) +
+                  r(0, 1, 1) + r(0, -1, 1) + r(1, 0, -1) + r(-1, 0, -1) + r(0, 1, -1) +
+                  r(0, -1, -1)) +
+          r(1, 1, 1) + r(-1, 1, 1) + r(1, -1, 1) + r(-1, -1, 1) + r(1, 1, -1) + r(-1, 1, -1) +
+          r(1, -1, -1) + r(-1, -1, -1)) /
+         T(64);
+}
+
 // R != nullptr: getres of every node of the fine residual range, formed
 // beforehand (the same expression, so the same bits).  masked: R is 0 on the
 // ghost nodes and on electrodes outside the plane j = n2 (which the wrap of
@@ -672,15 +707,7 @@ __device__ inline void restrict_node(const KLevelT<T, LB> &F, const KLevelT<T, L
   const int ir = 2 * i - 1, jr = 2 * j - 1, kr = 2 * k - 1;
   const int N1 = g.n1 + 1, N2 = g.n2 + 1, M1 = m + 1;
   const LB *bc = F.bc;
-  LB *bc2 = C.bc;
-  const LB lab = bc[gidx(g, ir, jr, kr)];
-  bc2[gidx(gc, i, j, k)] = lab;
-  if (ir == 1) bc2[gidx(gc, 0, j, k)] = bc[gidx(g, 0, jr, kr)];
-  if (ir == N1) bc2[gidx(gc, g.n1 / 2 + 2, j, k)] = bc[gidx(g, g.n1 + 2, jr, kr)];
-  if (jr == 1) bc2[gidx(gc, i, 0, k)] = bc[gidx(g, ir, 0, kr)];
-  if (jr == N2) bc2[gidx(gc, i, g.n2 / 2 + 2, k)] = bc[gidx(g, ir, g.n2 + 2, kr)];
-  if (kr == 1) bc2[gidx(gc, i, j, 0)] = bc[gidx(g, ir, jr, 0)];
-  if (kr == M1) bc2[gidx(gc, i, j, m / 2 + 2)] = bc[gidx(g, ir, jr, m + 2)];
+  const LB lab = restrict_labels(F, C, i, j, k);
   T re = T(0);
   if (lab <= 0 && masked && jr != 1 && (kr != 1 || !rp)) {
     const int64_t c = gidx(g, ir, jr, kr);
@@ -697,15 +724,7 @@ __device__ inline void restrict_node(const KLevelT<T, LB> &F, const KLevelT<T, L
           if (edge && bc[q] > 0) v[a_][b_][c_] = T(0);
         }
     }
-    auto r = [&](int a, int b_, int c_) { return v[a + 1][b_ + 1][c_ + 1]; };
-    re = (T(8) * r(0, 0, 0) +
-          T(4) * (r(1, 0, 0) + r(-1, 0, 0) + r(0, 1, 0) + r(0, -1, 0) + r(0, 0, 1) + r(0, 0, -1)) +
-          T(2) * (r(1, 1, 0) + r(-1, 1, 0) + r(1, -1, 0) + r(-1, -1, 0) + r(1, 0, 1) + r(-1, 0, 1) +
-                  r(0, 1, 1) + r(0, -1, 1) + r(1, 0, -1) + r(-1, 0, -1) + r(0, 1, -1) +
-                  r(0, -1, -1)) +
-          r(1, 1, 1) + r(-1, 1, 1) + r(1, -1, 1) + r(-1, -1, 1) + r(1, 1, -1) + r(-1, 1, -1) +
-          r(1, -1, -1) + r(-1, -1, -1)) /
-         T(64);
+    re = restrict_sum<T>([&](int a, int b_, int c_) { return v[a + 1][b_ + 1][c_ + 1]; });
   } else if (lab <= 0) {
     const int n2 = g.n2;
     const int64_t rs = g.n1 + 2;
@@ -819,19 +838,95 @@ __global__ __launch_bounds__(BLOCK) void k_restrict(KLevelT<T> F, KLevelT<T> C, 
   restrict_node(F, C, rp, flag_nmn, blockIdx.x * (int64_t)BLOCK + threadIdx.x, R);
 }
 
-// The restriction's first half: getres (mg.f90:809-848) at every node of
+// The restriction without periodic walls: a block takes RCX x RCY x RCZ coarse
+// nodes (one per thread), forms getres (mg.f90:809-848) of the fine nodes they
+// read in LDS, 0 where the reference takes none, and sums the 27 values there.
+// The residual goes to memory and back otherwise, and 27 labels are waited for
+// before the values they admit: 16 + 15 us at 128^3, 11 + 5 at 32^3 (FP64), 87
+// + 78 at 256^3 (FP32); this launch 20, 6.5 and 90.  The wrap of j = 1 (labels
+// <= 0 there) takes the general routine.  fin != nullptr: one more block, the
+// last, closes the sor_rb before it (slots_finish).
+constexpr int RCX = 16, RCY = 4, RCZ = 4;
+static_assert(RCX * RCY * RCZ == BLOCK, "a thread per coarse node");
+
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_restrict_tile(KLevelT<T> F, KLevelT<T> C, int flag_nmn,
+                                                         int ntx, int nty, SlotCtl sc, MGCtl *fin) {
+  constexpr int FX = 2 * RCX + 1, FY = 2 * RCY + 1, FZ = 2 * RCZ + 1;
+  constexpr int UN = sizeof(T) == 8 ? 11 : 4;   // nodes of a thread read before the first wait
+  __shared__ T R[FX * FY * FZ];
+  if (fin && blockIdx.x == gridDim.x - 1) {
+    __shared__ double red[BLOCK / LEPIC_WAVE];
+    slots_finish<BLOCK>(sc, fin, red);
+    return;
+  }
+  const KGrid &g = F.g;
+  const int per = (int)(gridDim.x - (fin ? 1 : 0)) / LEPIC_XCDS;   // consecutive tiles on one XCD
+  const int tile = (int)blockIdx.x < per * LEPIC_XCDS
+                       ? ((int)blockIdx.x % LEPIC_XCDS) * per + (int)blockIdx.x / LEPIC_XCDS
+                       : (int)blockIdx.x;
+  const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
+  const int x0 = 2 * bx * RCX, y0 = 2 * by * RCY, z0 = 2 * bz * RCZ;   // R's first fine node
+#pragma unroll 1
+  for (int t0 = threadIdx.x; t0 < FX * FY * FZ; t0 += UN * BLOCK) {
+    // read within the residual range whatever the node, so that no read waits for a test
+    int lab[UN];
+    bool first[UN];
+    T v[UN][8];
+#pragma unroll
+    for (int e = 0; e < UN; ++e) {
+      const int t = imin(t0 + e * BLOCK, FX * FY * FZ - 1);
+      const int z = t / (FX * FY), r = t - z * (FX * FY), y = r / FX, x = r - y * FX;
+      const int i = imax(1, imin(g.n1 + 1, x0 + x)), j = imax(1, imin(g.n2 + 1, y0 + y)),
+                k = imax(1, imin(g.n3 + 1, z0 + z));
+      const int64_t c = gidx(g, i, j, k);
+      const T *u = F.u;
+      lab[e] = F.bc[c];
+      v[e][0] = F.b[c];
+      v[e][1] = u[c - 1]; v[e][2] = u[c + 1];
+      v[e][3] = u[c + g.sy]; v[e][4] = u[c - g.sy];
+      v[e][5] = u[c]; v[e][6] = u[c + g.sz]; v[e][7] = u[c - g.sz];
+      if (i != x0 + x || j != y0 + y || k != z0 + z) lab[e] = 1;
+      first[e] = i == 1 && flag_nmn == 1;
+    }
+#pragma unroll
+    for (int e = 0; e < UN; ++e) {
+      const int t = t0 + e * BLOCK;
+      const T aw = first[e] ? T(0) : F.aw, ae = first[e] ? T(2) * F.ae : F.ae,
+              uw = first[e] ? T(0) : v[e][1];
+      const T res = v[e][0] - (aw * uw + ae * v[e][2] + F.an * v[e][3] + F.as * v[e][4] +
+                               F.ac * v[e][5] + F.at * v[e][6] + F.ab * v[e][7]);
+      if (t < FX * FY * FZ) R[t] = lab[e] <= 0 ? res : T(0);
+    }
+  }
+  __syncthreads();
+  const int lx = (int)threadIdx.x % RCX, ly = (int)threadIdx.x / RCX % RCY,
+            lz = (int)threadIdx.x / (RCX * RCY);
+  const int i = 1 + bx * RCX + lx, j = 1 + by * RCY + ly, k = 1 + bz * RCZ + lz;
+  const int ni = g.n1 / 2 + 1, nj = g.n2 / 2 + 1, nk = g.n3 / 2 + 1;
+  if (i > ni || j > nj || k > nk) return;
+  const int lab = F.bc[gidx(g, 2 * i - 1, 2 * j - 1, 2 * k - 1)];
+  if (lab <= 0 && j == 1) {
+    restrict_node(F, C, (const T *)nullptr, flag_nmn, (i - 1) + (int64_t)ni * (nj * (int64_t)(k - 1)));
+    return;
+  }
+  restrict_labels(F, C, i, j, k);
+  T re = T(0);
+  if (lab <= 0) {
+    const T *c = R + (2 * lx + 1) + FX * (2 * ly + 1) + FX * FY * (2 * lz + 1);
+    re = restrict_sum<T>([&](int a, int b, int c_) { return c[a + FX * b + FX * FY * c_]; });
+  }
+  C.b[gidx(C.g, i, j, k)] = re;
+}
+
+// The periodic restriction's first half: getres (mg.f90:809-848) at every node of
 // the fine level's residual range (1..n+1 in each direction) into R, once
 // per node instead of once per coarse neighbour that reads it, and the
 // coarse correction u zeroed (nc nodes).  The restriction's few getres
 // calls outside that range (the n2 wrap at i = n1 + 2) still go to getres.
-// fin != nullptr: block 0 also closes the sor_rb before it (slots_finish).
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_getres(KLevelT<T> F, T *R, T *cu, int64_t nc,
-                                                  int flag_nmn, SlotCtl sc, MGCtl *fin) {
-  if (fin && blockIdx.x == 0) {
-    __shared__ double red[BLOCK / LEPIC_WAVE];
-    slots_finish<BLOCK>(sc, fin, red);
-  }
+                                                  int flag_nmn) {
   const int64_t t = blockIdx.x * (int64_t)BLOCK + threadIdx.x;
   if (t < nc) cu[t] = T(0);
   const KGrid &g = F.g;
@@ -865,31 +960,36 @@ __device__ inline void prolong_node(const KLevelT<T, B> &F, const KLevelT<T, B> 
   const int ir = 2 * i - 1, jr = 2 * j - 1, kr = 2 * k - 1;
   T *u = F.u;
   const B *bc = F.bc;
-  int64_t c;
-  c = gidx(g, ir, jr, kr);
-  if (bc[c] <= 0) u[c] = u[c] + r000;
-  c = gidx(g, ir, jr - 1, kr);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + r0m0) / T(2);
-  c = gidx(g, ir - 1, jr - 1, kr);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + r0m0 + rmm0 + rm00) / T(4);
-  c = gidx(g, ir - 1, jr, kr);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + rm00) / T(2);
-  c = gidx(g, ir, jr, kr - 1);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + r00m) / T(2);
-  c = gidx(g, ir, jr - 1, kr - 1);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + r00m + r0mm + r0m0) / T(4);
-  c = gidx(g, ir - 1, jr, kr - 1);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + r00m + rm0m + rm00) / T(4);
-  c = gidx(g, ir - 1, jr - 1, kr - 1);
-  if (bc[c] <= 0) u[c] = u[c] + (r000 + r00m + rm0m + rm00 + r0m0 + r0mm + rmmm + rmm0) / T(8);
+  const T add[8] = {r000,
+                    (r000 + r0m0) / T(2),
+                    (r000 + r0m0 + rmm0 + rm00) / T(4),
+                    (r000 + rm00) / T(2),
+                    (r000 + r00m) / T(2),
+                    (r000 + r00m + r0mm + r0m0) / T(4),
+                    (r000 + r00m + rm0m + rm00) / T(4),
+                    (r000 + r00m + rm0m + rm00 + r0m0 + r0mm + rmmm + rmm0) / T(8)};
+  const int64_t c0 = gidx(g, ir, jr, kr);
+  const int64_t c[8] = {c0, c0 - g.sy, c0 - g.sy - 1, c0 - 1,
+                        c0 - g.sz, c0 - g.sz - g.sy, c0 - g.sz - 1, c0 - g.sz - g.sy - 1};
+  T old[8];
+  int lab[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {   // no read waits for a label
+    old[q] = u[c[q]];
+    lab[q] = bc[c[q]];
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (lab[q] <= 0) u[c[q]] = old[q] + add[q];
 }
 
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_prolong(KLevelT<T> F, KLevelT<T> C, SlotCtl sc,
                                                    MGCtl *fin) {
-  if (fin && blockIdx.x == 0) {   // close the coarse level's sor_rb
+  if (fin && blockIdx.x == gridDim.x - 1) {   // one more block closes the coarse level's sor_rb
     __shared__ double red[BLOCK / LEPIC_WAVE];
     slots_finish<BLOCK>(sc, fin, red);
+    return;
   }
   prolong_node(F, C, blockIdx.x * (int64_t)BLOCK + threadIdx.x);
 }
@@ -1362,8 +1462,7 @@ struct Solver {
   // fixed sweep counts (the inner smoother of the mixed-precision solve):
   // nr_fixed per sor_rb, nr_coarsest on the coarsest level, no residuals
   int fixed = 0, nr_fixed = 2, nr_coarsest = 64;
-  // the fine residual of a restriction (the finest level's ghosted size), or
-  // nullptr: the restriction forms it per coarse node
+  // the fine residual of a periodic restriction (the finest level's ghosted size)
   T *resbuf = nullptr;
   // the second u array of the levels that run whole sweeps per launch
   // (nullptr: one launch per colour), and the sweeps' exit bookkeeping
@@ -1436,7 +1535,7 @@ struct Solver {
   // up to 10^6 sweeps) keeps one launch per colour.
   bool tiled(int l, int dig) const { return !flag_pbc && dig != 0 && u2[l]; }
 
-  void sor_slots(int l) {
+  void sor_slots(int l, bool zero) {
     const KLevelT<T> &Lv = L[l];
     const SweepGrid w = sweep_grid(Lv.g);
     SlotCtl sc{slot_state, slot_partials, (int64_t)w.blocks()};
@@ -1445,12 +1544,12 @@ struct Solver {
       T *dst = (s & 1) ? Lv.u : u2[l];
       if (w.big)
         hipLaunchKernelGGL((k_sweep<T, BIG_X, BIG_Y, BIG_Z, BIG_NT, 2, 1, true>), dim3(w.blocks()),
-                           dim3(BIG_NT), 0, ctx->stream, Lv, src, dst, omega, w.nx, w.ny, 0, s, sc,
-                           &ctl[l]);
+                           dim3(BIG_NT), 0, ctx->stream, Lv, src, dst, omega, w.nx, w.ny,
+                           zero && s == 0 ? 1 : 0, s, sc, &ctl[l]);
       else
         hipLaunchKernelGGL((k_sweep<T, SML_X, SML_Y, SML_Z, SML_NT, 4, 1, true>), dim3(w.blocks()),
-                           dim3(SML_NT), 0, ctx->stream, Lv, src, dst, omega, w.nx, w.ny, 0, s, sc,
-                           &ctl[l]);
+                           dim3(SML_NT), 0, ctx->stream, Lv, src, dst, omega, w.nx, w.ny,
+                           zero && s == 0 ? 1 : 0, s, sc, &ctl[l]);
     }
     fin = &ctl[l];
     fin_sc = sc;
@@ -1499,7 +1598,7 @@ struct Solver {
   int sor_rb(int l, double eps, int kmg, int dig, bool zero = false) {
     if (tiled(l, dig)) {
       if (fixed) sor_fixed(l, zero);
-      else sor_slots(l);
+      else sor_slots(l, zero);
       return LEPIC_OK;
     }
     if (fixed) {
@@ -1529,32 +1628,34 @@ struct Solver {
     KLevelT<T> &F = L[l];
     KLevelT<T> &C = L[l + 1];
     const KGrid &g = F.g;
-    int64_t nc = grid_nodes_k(C.g);
-    if (resbuf) {
-      const int64_t nres = (int64_t)(g.n1 + 1) * (g.n2 + 1) * (g.n3 + 1);
-      hipLaunchKernelGGL(k_getres<T>, dim3(grid_blocks(std::max(nc, nres), BLOCK)), dim3(BLOCK), 0,
-                         ctx->stream, F, resbuf, C.u, nc, flag_nmn, fin_sc, fin);
+    const int64_t nc = grid_nodes_k(C.g);
+    if (!flag_pbc) {
+      // whole sweeps and the one-workgroup levels start from 0 without reading u
+      if (l + 1 < lc && !(l + 1 < ng - 1 && u2[l + 1]))
+        hipLaunchKernelGGL(k_fill_d<T>, dim3(grid_blocks(nc, BLOCK)), dim3(BLOCK), 0, ctx->stream,
+                           C.u, nc, T(0));
+      const int nx = (g.n1 / 2 + RCX) / RCX, ny = (g.n2 / 2 + RCY) / RCY,
+                nz = (g.n3 / 2 + RCZ) / RCZ;
+      hipLaunchKernelGGL(k_restrict_tile<T>, dim3((unsigned)nx * ny * nz + (fin ? 1 : 0)),
+                         dim3(BLOCK), 0, ctx->stream, F, C, flag_nmn, nx, ny, fin_sc, fin);
       fin = nullptr;
-    } else {
-      hipLaunchKernelGGL(k_fill_d<T>, dim3(grid_blocks(nc, BLOCK)), dim3(BLOCK), 0, ctx->stream,
-                         C.u, nc, T(0));
+      return;
     }
-    const T *rpp = nullptr;
-    if (flag_pbc) {
-      int64_t nent = (int64_t)(g.n1 + 2) * (g.n2 + 2);
-      hipLaunchKernelGGL(k_rpbc<T>, dim3(grid_blocks(nent, BLOCK)), dim3(BLOCK), 0, ctx->stream, F,
-                         rp, flag_nmn);
-      rpp = rp;
-    }
-    int64_t nt = (int64_t)(g.n1 / 2 + 1) * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
+    const int64_t nres = (int64_t)(g.n1 + 1) * (g.n2 + 1) * (g.n3 + 1);
+    hipLaunchKernelGGL(k_getres<T>, dim3(grid_blocks(std::max(nc, nres), BLOCK)), dim3(BLOCK), 0,
+                       ctx->stream, F, resbuf, C.u, nc, flag_nmn);
+    const int64_t nent = (int64_t)(g.n1 + 2) * (g.n2 + 2);
+    hipLaunchKernelGGL(k_rpbc<T>, dim3(grid_blocks(nent, BLOCK)), dim3(BLOCK), 0, ctx->stream, F,
+                       rp, flag_nmn);
+    const int64_t nt = (int64_t)(g.n1 / 2 + 1) * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
     hipLaunchKernelGGL(k_restrict<T>, dim3(grid_blocks(nt, BLOCK)), dim3(BLOCK), 0, ctx->stream, F,
-                       C, rpp, flag_nmn, (const T *)resbuf);
+                       C, (const T *)rp, flag_nmn, (const T *)resbuf);
   }
 
   void prolongation(int l) {  // L[l] += P(L[l+1])
     const KGrid &g = L[l].g;
     int64_t nt = (int64_t)(g.n1 / 2 + 1) * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
-    hipLaunchKernelGGL(k_prolong<T>, dim3(grid_blocks(nt, BLOCK)), dim3(BLOCK), 0, ctx->stream,
+    hipLaunchKernelGGL(k_prolong<T>, dim3(grid_blocks(nt, BLOCK) + (fin ? 1 : 0)), dim3(BLOCK), 0, ctx->stream,
                        L[l], L[l + 1], fin_sc, fin);
     fin = nullptr;
   }
@@ -1676,7 +1777,7 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   }
   // coarse-level storage (kept across calls; labels zeroed once)
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
-  const int64_t fine_nodes = ng > 1 ? grid_nodes(g) : 0;   // the restriction's residual
+  const int64_t fine_nodes = ng > 1 && mp->flag_pbc ? grid_nodes(g) : 0;   // the restriction's residual
   // the whole-sweep launches' second u arrays, block residuals and slot states
   const int64_t u2_nodes = ng > 1 && !mp->flag_pbc ? grid_nodes(g) + coarse_nodes : 0;
   int64_t sweep_parts = 0;
@@ -1686,7 +1787,8 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   size_t need = sizeof(double) * (size_t)(2 * coarse_nodes + max_parts + rp_len + fine_nodes +
                                           u2_nodes + slot_len) +
                 sizeof(int32_t) * (size_t)coarse_nodes + 4096;
-  bool same = ctx->mg_mem && ctx->mg_ng == ng && ctx->mg_n[0] == g->n[0] &&
+  const int layout = ng + (mp->flag_pbc ? 256 : 0);   // the arrays' places depend on both
+  bool same = ctx->mg_mem && ctx->mg_ng == layout && ctx->mg_n[0] == g->n[0] &&
               ctx->mg_n[1] == g->n[1] && ctx->mg_n[2] == g->n[2] && ctx->mg_bytes >= need;
   if (!same) {
     if (ctx->mg_mem) {
@@ -1697,7 +1799,7 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
     LEPIC_HIP(ctx, hipMalloc(&ctx->mg_mem, need));
     LEPIC_HIP(ctx, hipMemsetAsync(ctx->mg_mem, 0, need, ctx->stream));
     ctx->mg_bytes = need;
-    ctx->mg_ng = ng;
+    ctx->mg_ng = layout;
     for (int d = 0; d < 3; ++d) ctx->mg_n[d] = g->n[d];
   }
   char *mem = reinterpret_cast<char *>(ctx->mg_mem);
@@ -1969,10 +2071,11 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
   // the whole-sweep launches' second u arrays
   const int64_t u2_nodes = ng > 1 && !mp->flag_pbc ? nodes + coarse_nodes : 0;
+  const int64_t res_nodes = ng > 1 && mp->flag_pbc ? nodes : 0;   // the restriction's residual
   const size_t need = sizeof(double) * (size_t)(MIX_COLS * MIX_BLOCKS + 8) +
                       sizeof(double) * (size_t)nf64 * (size_t)nodes +
                       sizeof(T) * (size_t)(2 * nodes + 2 * coarse_nodes + rp_len) +
-                      sizeof(T) * (size_t)(ng > 1 ? nodes : 0) +   // the restriction's residual
+                      sizeof(T) * (size_t)res_nodes +
                       sizeof(T) * (size_t)u2_nodes +
                       sizeof(int32_t) * (size_t)coarse_nodes + 4096;
   if (!ctx->mgx_mem || ctx->mgx_bytes < need) {
@@ -1997,8 +2100,8 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   T *lv = M.r32 + nodes;
   S.rp = lv;
   lv += rp_len;
-  S.resbuf = ng > 1 ? lv + 2 * coarse_nodes : nullptr;
-  T *u2 = lv + 2 * coarse_nodes + (ng > 1 ? nodes : 0);
+  S.resbuf = res_nodes ? lv + 2 * coarse_nodes : nullptr;
+  T *u2 = lv + 2 * coarse_nodes + res_nodes;
   int32_t *lb = reinterpret_cast<int32_t *>(u2 + u2_nodes);
   for (int l = 0; l < ng && u2_nodes; ++l) {
     S.u2[l] = u2;
