@@ -96,6 +96,16 @@ enum : int {
 int lepic_fail(lepic_ctx *ctx, int code, const std::string &msg);
 int lepic_hip_check(lepic_ctx *ctx, hipError_t e, const char *what);
 void *lepic_scratch(lepic_ctx *ctx, size_t bytes, int which);
+// Particle indices ordered by cell (lepic_particles32.hip), on scratch 0 until
+// its next use: first slots and counts per cell, the indices, their number.
+struct CellOrder {
+  int32_t *count, *start, *cursor, *bsum, *idx;
+  int32_t *extra;    // the words asked for besides
+  int64_t *total;
+};
+int lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o);
+int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
+                    const CellOrder &o);
 // Resolves, once per device, the static scratch lepic_efield_noalloc uses
 // (lepic_fields.hip); the device must be current.
 void lepic_efield_scratch_setup(int device);

@@ -1116,6 +1116,50 @@ unsigned long long *int_replicas(lepic_ctx *ctx, int64_t nodes) {
 
 }  // namespace
 
+// The order of n particles by cell id (count, scan and claim of the sort): ids
+// below 0 are dropped, the order within a cell is the atomics'.
+int lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o) {
+  const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
+  const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
+  const size_t words = (size_t)(3 * ncells + nb + n + extra + 64);
+  int32_t *w = reinterpret_cast<int32_t *>(lepic_scratch(ctx, sizeof(int32_t) * words, 0));
+  if (!w) return lepic_fail(ctx, LEPIC_ERR_HIP, "cell order: scratch");
+  o.extra = w;                              // 256-byte aligned
+  o.count = w + ((extra + 15) & ~(int64_t)15);
+  o.start = o.count + ncells;
+  o.cursor = o.start + ncells;
+  o.bsum = o.cursor + ncells;
+  o.idx = o.bsum + nb;
+  o.total = ctx->d_ctrl + CTRL_COUNT_OUT;
+  return LEPIC_OK;
+}
+
+int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
+                    const CellOrder &o) {
+  lepic_grid g;
+  for (int d = 0; d < 3; ++d) {
+    g.n[d] = dims[d];
+    g.h[d] = 1.0;
+  }
+  const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
+  const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
+  const KG32 kg = make_kg32(&g, 0.0);
+  const hipStream_t s = ctx->stream;
+  hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, o.count, ncells);
+  hipLaunchKernelGGL(k_sort_count, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell,
+                     n, o.count);
+  hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum);
+  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, o.bsum, nb, o.total);
+  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
+                     o.start);
+  hipLaunchKernelGGL(k_copy_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, o.start, o.cursor,
+                     ncells);
+  hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell,
+                     n, o.cursor, o.idx);
+  LEPIC_LAUNCH_CHECK(ctx, "cell order");
+  return LEPIC_OK;
+}
+
 extern "C" {
 
 int lepic_pset_to32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset *src,
@@ -1279,27 +1323,11 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
     return LEPIC_OK;
   }
   const int64_t ncells = (int64_t)g->n[0] * g->n[1] * g->n[2];
-  const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
-  // scratch: count, start, cursor (ncells each), block sums, idx (n)
-  const size_t words = (size_t)(3 * ncells + nb + n + 64);
-  int32_t *w = reinterpret_cast<int32_t *>(lepic_scratch(ctx, sizeof(int32_t) * words, 0));
-  if (!w) return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: scratch");
-  int32_t *count = w, *start = w + ncells, *cursor = w + 2 * ncells, *bsum = w + 3 * ncells;
-  int32_t *idx = bsum + nb + 16;
-  int64_t *total = ctx->d_ctrl + CTRL_COUNT_OUT;
   const KG32 kg = make_kg32(g, 0.0);
   const hipStream_t s = ctx->stream;
-  hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, count, ncells);
-  hipLaunchKernelGGL(k_sort_count, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, src->cell,
-                     n, count);
-  hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, count, ncells, bsum);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, bsum, nb, total);
-  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, count, ncells, bsum,
-                     start);
-  hipLaunchKernelGGL(k_copy_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, start, cursor,
-                     ncells);
-  hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, src->cell,
-                     n, cursor, idx);
+  CellOrder o;
+  if ((st = lepic_order_alloc(ctx, g->n, n, 0, o)) || (st = lepic_order_run(ctx, g->n, src->cell, n, o)))
+    return st;
   // lanes per cell: the mean cell and twice its spread in one entry per lane
   const double mean = (double)n / (double)ncells, wide = mean + 2.0 * std::sqrt(mean);
   const int bx = (g->n[0] + BRX - 1) / BRX, by = (g->n[1] + BRY - 1) / BRY,
@@ -1307,14 +1335,14 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
   auto place = [&](auto kernel, int w) {
     const int64_t blocks = (int64_t)bx * by * bz * (BRX * BRY * BRZ * w / BLOCK);
     hipLaunchKernelGGL(kernel, dim3((unsigned)((blocks + LEPIC_XCDS - 1) / LEPIC_XCDS * LEPIC_XCDS)),
-                       dim3(BLOCK), 0, s, kg, kp32(src), kp32(dst), count, start, idx, bx, by);
+                       dim3(BLOCK), 0, s, kg, kp32(src), kp32(dst), o.count, o.start, o.idx, bx, by);
   };
   if (wide <= 8.0) place(k_sort_place<8>, 8);
   else if (wide <= 16.0) place(k_sort_place<16>, 16);
   else if (wide <= 32.0) place(k_sort_place<32>, 32);
   else place(k_sort_place<64>, 64);
   LEPIC_LAUNCH_CHECK(ctx, "sort32 passes");
-  LEPIC_HIP(ctx, hipMemcpyAsync(ctx->h_pinned, total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+  LEPIC_HIP(ctx, hipMemcpyAsync(ctx->h_pinned, o.total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   LEPIC_HIP(ctx, hipStreamSynchronize(s));
   const int64_t m = ctx->h_pinned[0];
   if (m < 0 || m > n) return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: inconsistent count");
