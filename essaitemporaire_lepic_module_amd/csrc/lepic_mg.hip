@@ -6,8 +6,8 @@
 // A sweep of a global level is one launch over tiles held in LDS (k_sweep):
 // red, black and the L1 residual, with sor_rb's exit rule (res/res_s <= 0.6,
 // at most 4 sweeps) taken by every block of the next launch.  Levels with
-// periodic ghosts to copy between the colours, and a coarsest level too large
-// for one workgroup, take one launch per colour, a deterministic block-tree
+// periodic walls take two launches per sweep (k_per_half); a coarsest level too
+// large for one workgroup takes one per colour, a deterministic block-tree
 // residual and a one-block decision.  Sweeps queued after the exit return at
 // once, so a V-cycle needs no host round trip; the host reads the fine
 // residual once per V-cycle for pdesolver's convergence test.  Levels below a
@@ -32,6 +32,36 @@ struct MGCtl {
   int64_t pad[11];
 };
 static_assert(sizeof(MGCtl) == 16 * sizeof(int64_t), "MGCtl layout");
+
+// a + the value CTRL (a DPP row operation) brings, 0 where it brings none.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double a) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, ROWS, 0xf, true);
+  return a + __hiloint2double(hi, lo);
+}
+
+__device__ inline double read_lane(double a, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), lane),
+                          __builtin_amdgcn_readlane(__double2loint(a), lane));
+}
+
+// Sum of each 16-lane row in its last lane.
+__device__ inline double row_sum(double a) {
+  a = dpp_add<0x111, 0xf>(a);   // row_shr:1, 2, 4, 8
+  a = dpp_add<0x112, 0xf>(a);
+  a = dpp_add<0x114, 0xf>(a);
+  return dpp_add<0x118, 0xf>(a);
+}
+
+// Sum over a full wave in a fixed order, the same in every lane (register
+// moves: six steps of shuffles through LDS take five times as long).
+__device__ inline double wave_sum(double a) {
+  a = row_sum(a);
+  a = dpp_add<0x142, 0xa>(a);   // row_bcast:15 into rows 1 and 3
+  a = dpp_add<0x143, 0xc>(a);   // row_bcast:31 into rows 2 and 3
+  return read_lane(a, LEPIC_WAVE - 1);
+}
 
 // One multigrid level: geometry, stencil coefficients and the level's u, b
 // and labels.  T is the storage and arithmetic type of u and b (double for
@@ -604,6 +634,269 @@ __global__ __launch_bounds__(NT) void k_sweep(KLevelT<T> L, const T *src, T *dst
   }
 }
 
+// --------------------------------------------------------------------------
+// Levels with periodic walls: two launches per sweep and one at the end.
+// sor_rb copies the ghost planes after every colour; here a colour reads
+// through the copies (per_source: the node that a boundary node has its value
+// from) and the copies are made once, at the end.  Only the first red half
+// reads the ghosts as they stand.  The black residual is summed with the black
+// half, the red one with the next sweep's red half, which goes to the other of
+// two arrays of red values (X; black stays in u): if the decision, taken by
+// every block of the black half as in k_sweep, ends the sor_rb, that half is
+// not used.  9 launches of 6 to 7 us in place of 32 of 3 to 4 (two colours, four copies,
+// residual, decision, four times): solve of 96 x 40 x 72 14.3 -> 10.3 ms.
+// --------------------------------------------------------------------------
+constexpr int PER_BLOCKS = 1024;   // block residuals that every block sums
+
+__device__ inline bool per_ok(int lab) { return lab == 0 || lab == -2; }
+
+// The node (i, j, k) has its value from after the copies of sors.f90:184-239
+// (y planes, then z planes): j and k of that node.
+template <class T>
+__device__ inline void per_source(const KLevelT<T> &L, int i, int &j, int &k) {
+  const KGrid &g = L.g;
+  if (k == g.n3 + 1 && per_ok(L.bc[gidx(g, i, j, g.n3 + 1)])) k = 1;
+  else if (k == 0 && per_ok(L.bc[gidx(g, i, j, 1)])) k = g.n3;
+  if (j == g.n2 + 1 && per_ok(L.bc[gidx(g, i, g.n2 + 1, k)])) j = 1;
+  else if (j == 0 && per_ok(L.bc[gidx(g, i, 1, k)])) j = g.n2;
+}
+
+// u where a node of one colour's array X (nodes 1..n+1) is read, through the
+// copies with pull.
+template <class T>
+__device__ inline T per_read(const KLevelT<T> &L, const T *X, int i, int j, int k, bool pull) {
+  const KGrid &g = L.g;
+  if (pull) per_source(L, i, j, k);
+  const bool in = i >= 1 && i <= g.n1 + 1 && j >= 1 && j <= g.n2 + 1 && k >= 1 && k <= g.n3 + 1;
+  return (in ? X : (const T *)L.u)[gidx(g, i, j, k)];
+}
+
+template <class T>
+struct Nbr6 {
+  T uw, ue, un, us, ut, ub;
+};
+
+// The six neighbours of a node of [1, n+1].
+template <class T>
+__device__ inline Nbr6<T> per_neighbours(const KLevelT<T> &L, const T *X, int i, int j, int k,
+                                         bool pull) {
+  const KGrid &g = L.g;
+  const int64_t c = gidx(g, i, j, k);
+  Nbr6<T> v;
+  if (j > 1 && j < g.n2 && k > 1 && k < g.n3) {
+    v.uw = (i == 1 ? (const T *)L.u : X)[c - 1];
+    v.ue = (i == g.n1 + 1 ? (const T *)L.u : X)[c + 1];
+    v.un = X[c + g.sy]; v.us = X[c - g.sy];
+    v.ut = X[c + g.sz]; v.ub = X[c - g.sz];
+  } else {
+    v.uw = per_read(L, X, i - 1, j, k, pull); v.ue = per_read(L, X, i + 1, j, k, pull);
+    v.un = per_read(L, X, i, j + 1, k, pull); v.us = per_read(L, X, i, j - 1, k, pull);
+    v.ut = per_read(L, X, i, j, k + 1, pull); v.ub = per_read(L, X, i, j, k - 1, pull);
+  }
+  return v;
+}
+
+// Node t of a colour: false when it is none.
+template <class T>
+__device__ inline bool per_node(const KLevelT<T> &L, int colour, int t, int &i, int &j, int &k) {
+  const KGrid &g = L.g;
+  const uint32_t r = mdiv_q((uint32_t)t, L.d_h1), rk = mdiv_q(r, L.d_n2p1);
+  j = 1 + (int)(r - rk * (uint32_t)(g.n2 + 1));
+  k = 1 + (int)rk;
+  const int red = 1 + ((j + k) & 1);   // red: i + j + k odd
+  i = (colour ? 3 - red : red) + 2 * (t - (int)r * (g.n1 / 2 + 1));
+  return i <= g.n1 + 1;
+}
+
+template <class T>
+__device__ inline double per_resid(const KLevelT<T> &L, T b, T uc, const Nbr6<T> &v) {
+  const T rij = b - (L.aw * v.uw + L.an * v.un + L.as * v.us + L.ae * v.ue + L.ac * uc +
+                     L.at * v.ut + L.ab * v.ub);
+  return fabs((double)rij);
+}
+
+// A block's sum of a to out[blockIdx.x].
+__device__ inline void per_partial(double a, double *out) {
+  __shared__ double red[BLOCK / LEPIC_WAVE];
+  a = wave_sum(a);
+  if (__lane_id() == 0) red[threadIdx.x / LEPIC_WAVE] = a;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double b = 0.0;
+    for (int w = 0; w < BLOCK / LEPIC_WAVE; ++w) b = b + red[w];
+    out[blockIdx.x] = b;
+  }
+}
+
+// The residual after sweep s from its partials (black of even sweeps, of odd
+// ones, red): a thread's share, and the block's sum of them in every thread.
+__device__ inline double per_share(const SlotCtl &sc, int s) {
+  double v[2 * PER_BLOCKS / BLOCK];
+#pragma unroll
+  for (int q = 0; q < PER_BLOCKS / BLOCK; ++q) {
+    const int64_t t = threadIdx.x + q * BLOCK;
+    v[2 * q] = t < sc.nparts ? sc.partials[(s & 1) * sc.nparts + t] : 0.0;
+    v[2 * q + 1] = t < sc.nparts ? sc.partials[2 * sc.nparts + t] : 0.0;
+  }
+  double a = 0.0;
+#pragma unroll
+  for (int q = 0; q < 2 * PER_BLOCKS / BLOCK; ++q) a = a + v[q];
+  return a;
+}
+
+__device__ inline double per_sum(double a) {
+  __shared__ double red[BLOCK / LEPIC_WAVE];
+  a = wave_sum(a);
+  if (__lane_id() == 0) red[threadIdx.x / LEPIC_WAVE] = a;
+  __syncthreads();
+  double r = 0.0;
+  for (int w = 0; w < BLOCK / LEPIC_WAVE; ++w) r = r + red[w];
+  __syncthreads();
+  return r;
+}
+
+// An edge ghost that the y copy writes and the z copy does not (labels that
+// differ between it and the node beside it) takes, from a ghost or copied node
+// of its source plane, the value before the last black half: the owner of a
+// black node leaves it there, k_per_end does the others.
+template <class T>
+__device__ inline void per_edge(const KLevelT<T> &L, int i, int j, int k, T old) {
+  const KGrid &g = L.g;
+  auto ok = [&](int b, int c) { return per_ok(L.bc[gidx(g, i, b, c)]); };
+  if (j == g.n2 && k == 1 && ok(1, g.n3 + 1) && !ok(0, g.n3 + 1) && ok(g.n2, g.n3 + 1))
+    L.u[gidx(g, i, 0, g.n3 + 1)] = old;
+  if (j == g.n2 && k == g.n3 && ok(1, 0) && !ok(0, 1) && ok(g.n2, 1)) L.u[gidx(g, i, 0, 0)] = old;
+  if (j == 1 && k == g.n3 && ok(g.n2 + 1, 0) && !ok(g.n2 + 1, 1) && ok(1, 1))
+    L.u[gidx(g, i, g.n2 + 1, 0)] = old;
+}
+
+// One half of sweep s.  colour 0: red, from X (s even: u, else u2) to Xn;
+// colour 1: black in u, the red values in X.  ctl null: a fixed sweep count.
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T *Xn, int colour,
+                                                    T omega, int s, SlotCtl sc, MGCtl *ctl) {
+  const bool judged = ctl != nullptr;
+  const KGrid &g = L.g;
+  const int n = (g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1);
+  const T *own = colour ? (const T *)L.u : X, *other = colour ? X : (const T *)L.u;
+  T *out = colour ? L.u : Xn;
+  const bool pull = colour == 1 || s > 0;
+  int i = 0, j = 0, k = 0, lab = 1;
+  T b = T(0), uc = T(0);
+  Nbr6<T> v = {};
+  bool node = false;
+  auto load = [&](int t) {
+    node = t < n && per_node(L, colour, t, i, j, k);
+    if (!node) return;
+    const int64_t c = gidx(g, i, j, k);
+    lab = L.bc[c];
+    b = L.b[c];
+    uc = own[c];
+    v = per_neighbours(L, other, i, j, k, pull);
+  };
+  // everything the launch reads is under way before the decision
+  int t = blockIdx.x * BLOCK + threadIdx.x;
+  load(t);
+  if (judged && s > 0) {
+    const double share = colour ? per_share(sc, s - 1) : 0.0;
+    const SlotState st = sc.state[s - 1];
+    if (colour == 0) {
+      if (st.active == 0) return;
+    } else {
+      bool active = st.active != 0;
+      double res = 0.0;
+      if (active) {
+        res = per_sum(share);
+        active = !sor_stops(res, st.res_s);
+        if (!active && blockIdx.x == 0 && threadIdx.x == 0) {
+          ctl->res = res;
+          ctl->total += s;
+        }
+      }
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc.state[s].active = active ? 1 : 0;
+        sc.state[s].res_s = res;
+      }
+      if (!active) return;
+    }
+  } else if (judged && colour == 1 && blockIdx.x == 0 && threadIdx.x == 0) {
+    sc.state[0].active = 1;
+    sc.state[0].res_s = 0.0;
+  }
+  double a = 0.0;
+  for (;;) {
+    if (node) {
+      const int64_t c = gidx(g, i, j, k);
+      if (colour == 1 && (j == 1 || j == g.n2) && (k == 1 || k == g.n3)) per_edge(L, i, j, k, uc);
+      if (judged && colour == 0 && s > 0 && lab == -1) a = a + per_resid(L, b, uc, v);
+      if (!(lab > 0 || (lab == 0 && (k == g.n3 + 1 || j == g.n2 + 1)))) {
+        if (lab == -2)
+          uc = (T(1) - omega) * uc +
+               div_ac(omega * (b - L.an * v.un - L.as * v.us - T(2) * L.ae * v.ue - L.at * v.ut -
+                               L.ab * v.ub),
+                      L);
+        else
+          uc = (T(1) - omega) * uc +
+               div_ac(omega * (b - L.aw * v.uw - L.an * v.un - L.as * v.us - L.ae * v.ue -
+                               L.at * v.ut - L.ab * v.ub),
+                      L);
+        out[c] = uc;
+      } else if (colour == 0) {
+        out[c] = uc;   // the other array's copy of a node that is not relaxed
+      }
+      if (judged && colour == 1 && lab == -1) a = a + per_resid(L, b, uc, v);
+    }
+    t += gridDim.x * BLOCK;
+    if (t >= n) break;
+    load(t);
+  }
+  if (judged && (colour == 1 || s > 0))
+    per_partial(a, sc.partials + (colour ? (int64_t)(s & 1) : 2) * sc.nparts);
+}
+
+// The end of a sor_rb: the red values back in u, the periodic copies, and with
+// resid the last red residual (when all sweeps ran).  count: the sweeps, of a
+// fixed count (ctl null).
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_per_end(KLevelT<T> L, MDiv d_n2p3, const T *u2, int count,
+                                                   int resid, SlotCtl sc, MGCtl *ctl) {
+  bool all = false;
+  if (ctl) {
+    count = 0;
+    for (int s = 0; s < SLOTS; ++s) count += sc.state[s].active != 0 ? 1 : 0;
+    all = count == SLOTS;
+    if (all && blockIdx.x == 0 && threadIdx.x == 0) ctl->total += SLOTS;
+  }
+  const KGrid &g = L.g;
+  const T *X = (count & 1) ? u2 : (const T *)L.u;
+  const int nx = g.n1 + 3, nodes = nx * (g.n2 + 3) * (g.n3 + 3);
+  double a = 0.0;
+  for (int t = blockIdx.x * BLOCK + threadIdx.x; t < nodes; t += gridDim.x * BLOCK) {
+    const uint32_t r = mdiv_q((uint32_t)t, L.d_n1p3), rk = mdiv_q(r, d_n2p3);
+    const int i = t - (int)r * nx, j = (int)(r - rk * (uint32_t)(g.n2 + 3)), k = (int)rk;
+    const bool is_red = (i + j + k) & 1;
+    int sj = j, sk = k;
+    per_source(L, i, sj, sk);
+    const bool in = i >= 1 && i <= g.n1 + 1 && j >= 1 && j <= g.n2 + 1 && k >= 1 && k <= g.n3 + 1;
+    if (resid && all && in && is_red && L.bc[t] == -1)
+      a = a + per_resid(L, L.b[t], X[t], per_neighbours(L, (const T *)L.u, i, j, k, true));
+    if (sj != j && (sk == 0 || sk == g.n3 + 1)) {   // an edge ghost (per_edge)
+      const bool copied = per_ok(L.bc[gidx(g, i, sj, sk == 0 ? 1 : g.n3 + 1)]);
+      if (copied && !is_red) continue;
+      if (copied) sk = sk == 0 ? g.n3 : 1;
+    }
+    if (sj != j || sk != k) L.u[t] = per_read(L, is_red ? X : (const T *)L.u, i, sj, sk, false);
+    else if (is_red && in && (count & 1)) L.u[t] = u2[t];
+  }
+  if (resid && all) per_partial(a, sc.partials + 2 * sc.nparts);
+}
+
+__global__ __launch_bounds__(BLOCK) void k_per_res(SlotCtl sc, MGCtl *ctl) {
+  if (sc.state[SLOTS - 1].active == 0) return;
+  const double res = per_sum(per_share(sc, SLOTS - 1));
+  if (threadIdx.x == 0) ctl->res = res;
+}
+
 // r_pbc: residual of plane k = m, the periodic image of k = 0
 // (mg.f90:322-392).  The reference loops over coarse (j, i) and each
 // iteration writes up to nine overlapping entries, the later iteration
@@ -1054,36 +1347,6 @@ __device__ inline KLevelT<T, int16_t> lds_level(const CoarseArgs<T> &A, T *lds, 
   return v;
 }
 
-// a + the value CTRL (a DPP row operation) brings, 0 where it brings none.
-template <int CTRL, int ROWS>
-__device__ inline double dpp_add(double a) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, ROWS, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, ROWS, 0xf, true);
-  return a + __hiloint2double(hi, lo);
-}
-
-__device__ inline double read_lane(double a, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), lane),
-                          __builtin_amdgcn_readlane(__double2loint(a), lane));
-}
-
-// Sum of each 16-lane row in its last lane.
-__device__ inline double row_sum(double a) {
-  a = dpp_add<0x111, 0xf>(a);   // row_shr:1, 2, 4, 8
-  a = dpp_add<0x112, 0xf>(a);
-  a = dpp_add<0x114, 0xf>(a);
-  return dpp_add<0x118, 0xf>(a);
-}
-
-// Sum over a full wave in a fixed order, the same in every lane (register
-// moves: six steps of shuffles through LDS take five times as long).
-__device__ inline double wave_sum(double a) {
-  a = row_sum(a);
-  a = dpp_add<0x142, 0xa>(a);   // row_bcast:15 into rows 1 and 3
-  a = dpp_add<0x143, 0xc>(a);   // row_bcast:31 into rows 2 and 3
-  return read_lane(a, LEPIC_WAVE - 1);
-}
-
 // Workgroup sum in a fixed order, every thread gets it: the waves' sums to
 // red[0..15], one barrier, and a row sum of those.  The next call needs a
 // barrier in between.
@@ -1464,11 +1727,11 @@ struct Solver {
   int fixed = 0, nr_fixed = 2, nr_coarsest = 64;
   // the fine residual of a periodic restriction (the finest level's ghosted size)
   T *resbuf = nullptr;
-  // the second u array of the levels that run whole sweeps per launch
+  // the second u array of the levels that sweep in one or two launches
   // (nullptr: one launch per colour), and the sweeps' exit bookkeeping
   T *u2[MAX_LEVELS] = {};
   SlotState *slot_state = nullptr;
-  double *slot_partials = nullptr;   // 2 x the most blocks of a sweep launch
+  double *slot_partials = nullptr;   // 3 x the most blocks of a sweep launch
   MGCtl *fin = nullptr;              // the level whose last sor_rb is still to be closed
   SlotCtl fin_sc = {};
 
@@ -1530,10 +1793,32 @@ struct Solver {
                        dig, nr);
   }
 
-  // A level sweeps in whole-sweep launches when it has no periodic ghosts to
-  // copy between the colours; the coarsest level's sor_rb (another exit rule,
-  // up to 10^6 sweeps) keeps one launch per colour.
+  // A level sweeps in whole-sweep launches, with periodic walls in two per
+  // sweep; the coarsest level's sor_rb (another exit rule, up to 10^6 sweeps)
+  // keeps one launch per colour.
   bool tiled(int l, int dig) const { return !flag_pbc && dig != 0 && u2[l]; }
+  bool periodic(int l, int dig) const { return flag_pbc && dig != 0 && u2[l]; }
+
+  void sor_periodic(int l) {
+    const KLevelT<T> &Lv = L[l];
+    const KGrid &g = Lv.g;
+    const int64_t n = (int64_t)(g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1);
+    const unsigned nb = std::min<unsigned>(grid_blocks(n, BLOCK), PER_BLOCKS);
+    const SlotCtl sc{slot_state, slot_partials, (int64_t)nb};
+    MGCtl *c = fixed ? nullptr : &ctl[l];
+    const int sweeps = fixed ? nr_fixed : SLOTS;
+    T *X[2] = {Lv.u, u2[l]};
+    for (int s = 0; s < sweeps; ++s) {
+      hipLaunchKernelGGL(k_per_half<T>, dim3(nb), dim3(BLOCK), 0, ctx->stream, Lv,
+                         (const T *)X[s & 1], X[1 - (s & 1)], 0, omega, s, sc, c);
+      hipLaunchKernelGGL(k_per_half<T>, dim3(nb), dim3(BLOCK), 0, ctx->stream, Lv,
+                         (const T *)X[1 - (s & 1)], (T *)nullptr, 1, omega, s, sc, c);
+    }
+    const int resid = l == 0 && !fixed ? 1 : 0;   // the level whose residual is read
+    hipLaunchKernelGGL(k_per_end<T>, dim3(nb), dim3(BLOCK), 0, ctx->stream, Lv,
+                       mdiv((uint32_t)(g.n2 + 3)), (const T *)u2[l], sweeps, resid, sc, c);
+    if (resid) hipLaunchKernelGGL(k_per_res, dim3(1), dim3(BLOCK), 0, ctx->stream, sc, c);
+  }
 
   void sor_slots(int l, bool zero) {
     const KLevelT<T> &Lv = L[l];
@@ -1596,6 +1881,10 @@ struct Solver {
   // sor_rb: returns LEPIC_OK; sweeps are counted on the device.  zero: the
   // level's u is 0 everywhere.
   int sor_rb(int l, double eps, int kmg, int dig, bool zero = false) {
+    if (periodic(l, dig)) {
+      sor_periodic(l);
+      return LEPIC_OK;
+    }
     if (tiled(l, dig)) {
       if (fixed) sor_fixed(l, zero);
       else sor_slots(l, zero);
@@ -1778,12 +2067,13 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   // coarse-level storage (kept across calls; labels zeroed once)
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
   const int64_t fine_nodes = ng > 1 && mp->flag_pbc ? grid_nodes(g) : 0;   // the restriction's residual
-  // the whole-sweep launches' second u arrays, block residuals and slot states
-  const int64_t u2_nodes = ng > 1 && !mp->flag_pbc ? grid_nodes(g) + coarse_nodes : 0;
+  // the sweeps' second u arrays, block residuals and slot states
+  const int64_t u2_nodes = ng > 1 ? grid_nodes(g) + coarse_nodes : 0;
   int64_t sweep_parts = 0;
   for (int l = 0; l < ng; ++l)
     sweep_parts = std::max<int64_t>(sweep_parts, sweep_grid(S.L[l].g).blocks());
-  const int64_t slot_len = 2 * sweep_parts + (int64_t)(SLOTS * sizeof(SlotState) / sizeof(double));
+  sweep_parts = std::max<int64_t>(sweep_parts, PER_BLOCKS);
+  const int64_t slot_len = 3 * sweep_parts + (int64_t)(SLOTS * sizeof(SlotState) / sizeof(double));
   size_t need = sizeof(double) * (size_t)(2 * coarse_nodes + max_parts + rp_len + fine_nodes +
                                           u2_nodes + slot_len) +
                 sizeof(int32_t) * (size_t)coarse_nodes + 4096;
@@ -2069,8 +2359,8 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   }
   const int64_t nodes = grid_nodes(g);
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
-  // the whole-sweep launches' second u arrays
-  const int64_t u2_nodes = ng > 1 && !mp->flag_pbc ? nodes + coarse_nodes : 0;
+  // the sweeps' second u arrays
+  const int64_t u2_nodes = ng > 1 ? nodes + coarse_nodes : 0;
   const int64_t res_nodes = ng > 1 && mp->flag_pbc ? nodes : 0;   // the restriction's residual
   const size_t need = sizeof(double) * (size_t)(MIX_COLS * MIX_BLOCKS + 8) +
                       sizeof(double) * (size_t)nf64 * (size_t)nodes +

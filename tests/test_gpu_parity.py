@@ -333,6 +333,52 @@ def test_poisson_coarse_levels_bitexact(gpu, oracle, rng, n, ng, zero, nmn):
                                atol=1e-12 * np.abs(phi_o).max())
 
 
+# Levels with periodic walls (k_per_half, k_per_end): one and two of them above
+# the one-workgroup levels, a block's share of nodes exceeded, and labels that
+# make the copies differ from node to node: electrodes and plasma on either copied
+# plane, Neumann rows on them, start ghosts that are no copies of anything.
+@pytest.mark.parametrize("n,ng,mess", [((32, 24, 40), 3, False), ((32, 24, 40), 3, True),
+                                       ((20, 12, 36), 2, True), ((64, 48, 64), 4, True),
+                                       ((128, 64, 80), 4, False)])
+def test_poisson_periodic_levels_bitexact(gpu, oracle, rng, n, ng, mess):
+    """phi, ghosts included, within 1e-12 of max |phi| and every level's sweep
+    count equal to the oracle's (same operands and expressions; only the
+    residual's summation order differs)."""
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box(n)
+    bc = H.periodic_yz_bcnd(n)
+    if mess:
+        inner = np.zeros(bc.shape, bool)
+        inner[:, :, 3:n[0]] = True
+        y1, y2 = inner.copy(), inner.copy()
+        y1[:, :1] = y1[:, 2:] = False
+        y2[:, :n[1] + 1] = y2[:, n[1] + 2:] = False
+        z1, z2 = inner.copy(), inner.copy()
+        z1[:1] = z1[2:] = False
+        z2[:n[2] + 1] = z2[n[2] + 2:] = False
+        for plane, lab, share in ((y1, 2, 0.1), (y2, 2, 0.1), (z1, 2, 0.1), (z2, 2, 0.1),
+                                  (y1, -1, 0.05), (z2, -1, 0.05), (y2, -2, 0.02), (z1, -2, 0.02)):
+            bc[plane & (rng.random(bc.shape) < share)] = lab
+        bc[(bc == -1) & (rng.random(bc.shape) < 0.05)] = 3
+    cycles = 1 if mess else 4      # such rows need not converge
+    phi0 = np.where(bc == 2, 2.0, np.where(bc > 0, -1.0, 0.01 * rng.standard_normal(bc.shape)))
+    rho = np.where(bc <= 0, 1e-6 * rng.standard_normal(bc.shape), 0.0)
+    phi_o = phi0.copy()
+    st, info_o = oracle.pdesolver(n, h, phi_o, rho, bc, flag_pbc=1, flag_nmn=0, ng=ng, eps=1e-8,
+                                  omega=1.2, ncycl=cycles)
+    assert st == 0
+    for graph in (True, True, False):
+        phi_g = torch.as_tensor(phi0, device=gpu)
+        info_g = F.solve_poisson_legacy(phi_g, torch.as_tensor(bc, device=gpu),
+                                        torch.as_tensor(rho, device=gpu), h, n, cycles, 1e-8, 1.2,
+                                        ng, 1, 0, graph=graph)
+        assert info_g["cycles"] == info_o["cycles"]
+        assert info_g["sweeps"] == info_o["sweeps"]
+        off = np.abs(phi_g.cpu().numpy() - phi_o) > 1e-12 * np.abs(phi_o).max()
+        assert not off.any(), np.argwhere(off)[:20]
+        np.testing.assert_allclose(info_g["res"], info_o["res"], rtol=1e-9)
+
+
 def test_loader_host_bitexact(oracle):
     """The product's host loader reproduces the reference loader's ran2 stream."""
     from essaitemporaire_lepic_module_amd import particles as P
