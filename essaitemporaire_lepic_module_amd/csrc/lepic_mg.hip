@@ -1319,7 +1319,16 @@ struct CoarseArgs {
   int lds_off[MAX_LEVELS];    // level l's u at lds + lds_off[l], b lds_nn[l] after it
   int lds_nn[MAX_LEVELS];
   int lab_off[MAX_LEVELS];    // level l's labels at labs + lab_off[l]
+  // whole solves: pdesolver's normalisation, tolerance and cycle bound, and the
+  // cycle and first residual to go on from
+  double alpha, tol, res_s;
+  int k, ncycl;
 };
+
+// V-cycles of a whole solve per launch (the host launches again for more).
+constexpr int WHOLE_CYCLES = 64;
+// ctl[0].pad after it: the cycle reached, WHOLE_*, the first residual's bits
+enum : int { WHOLE_DONE = 0, WHOLE_MORE = 1, WHOLE_DIVERGED = 2 };
 
 // A label as the coarse workgroup keeps it: saturated to int16, which keeps
 // its sign and the values 0, -1 and -2, all the solver tests.
@@ -1416,10 +1425,14 @@ __device__ __forceinline__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t 
 //    barriers per sweep, and no residual where the sweep count ends the sor_rb,
 //  - a level of at most 64 SL nodes per colour is left to one wave, whose LDS
 //    accesses are in order without a barrier.
-// Launch of 16^3 and below, FP64: 98 -> 68 us; 8^3 and below 47 -> 32.
+// want_res: the residual after the last sweep is returned, to every thread.
+// Up to 3 pairs per thread have their own copy of the routine: five spill in FP64
+// (16^3: 240 us a solve instead of 281).
+// Launch of 16^3 and below, FP64: 98 -> 62 us; 8^3 and below 47 -> 32.
 template <class T, int NT, int SL>
-__device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l, int dig,
-                                int64_t nr, bool restricts, double *red) {
+__device__ __forceinline__ double wg_level(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l,
+                                           int dig, int64_t nr, bool restricts, bool want_res,
+                                           double *red) {
   const KLevelT<T, int16_t> Lv = lds_level(A, S, Lb, l);
   const KGrid &g = Lv.g;
   const int tid = (int)threadIdx.x;
@@ -1434,6 +1447,7 @@ __device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *
   // (0 not relaxed, 1 plasma, 2 Neumann, 3 other)
   int pk[2][SL];
   T bb[2][SL], uc[2][SL];
+  double res = 0.0;
   auto sync = [&]() {
     if (NT == CBLOCK) {
       __syncthreads();
@@ -1511,18 +1525,18 @@ __device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *
     const std::integral_constant<int, 0> RED{};
     const std::integral_constant<int, 1> BLACK{};
     int64_t ksor = 0;
-    double res = 0.0, res_s = 0.0;
+    double res_s = 0.0;
     phase(RED, true, false, false, nullptr);
     sync();
     for (;;) {
       ++ksor;
-      const bool last = ksor >= nr, judged = !A.fixed && !last;
+      const bool last = ksor >= nr, judged = !A.fixed && (!last || want_res);
       a = 0.0;
       phase(BLACK, true, false, judged, nullptr);
       sync();
-      if (last) break;
+      if (last && !judged) break;
       T old[SL];
-      phase(RED, true, judged, false, old);
+      phase(RED, !last, judged, false, old);
       if (judged) {
         if (NT == CBLOCK) {
           res = wg_sum(a, red);
@@ -1530,6 +1544,7 @@ __device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *
           res = wave_sum(a);
           sync();
         }
+        if (last) break;
         const bool stop = dig == 0 ? res <= A.eps : res_s > 0.0 && (res / res_s) <= 0.6;
         res_s = res;
         if (stop) {   // the next sweep's red half is not to be
@@ -1568,7 +1583,13 @@ __device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *
     }
   }
   __syncthreads();
-  if (!restricts) return;
+  if (want_res && NT != CBLOCK) {
+    if (tid == 0) red[0] = res;
+    __syncthreads();
+    res = red[0];
+    __syncthreads();
+  }
+  if (!restricts) return res;
   const KLevelT<T, int16_t> Cv = lds_level(A, S, Lb, l + 1);
   const int nt = ni2 * (g.n2 / 2 + 1) * (g.n3 / 2 + 1);
   for (int t = tid; t < nt; t += CBLOCK)
@@ -1579,9 +1600,10 @@ __device__ __forceinline__ void wg_level(const CoarseArgs<T> &A, T *S, int16_t *
     for (int s = 0; s < SL; ++s)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        if (pk[c][s] & 3) bl[pk[c][s] >> 5] = bb[c][s];
+        if (pk[c][s] & 16) bl[pk[c][s] >> 5] = bb[c][s];
   }
   // the up leg's reads of b lie behind further barriers
+  return res;
 }
 
 template <class T>
@@ -1614,7 +1636,10 @@ __device__ __forceinline__ void wg_prolongation(const CoarseArgs<T> &A, T *S, in
 // on every level then, and b 0 at the ghost nodes, which no restriction
 // writes.  u of level lc, the only array read after the launch, is copied back
 // at the end.
-template <class T, bool PBC>
+// WHOLE: lc = 0, and the launch is pdesolver's loop (pdesolver.f90:97-115) of
+// up to WHOLE_CYCLES V-cycles.  A V-cycle of 16^3 takes 16 launches and a host
+// round trip else, 108 us; here 55 (solve 434 -> 240 us).
+template <class T, bool PBC, bool WHOLE>
 __global__ __launch_bounds__(CBLOCK) void k_mg_coarse(CoarseArgs<T> A) {
   __shared__ double red[CBLOCK / LEPIC_WAVE];
   __shared__ T lds[2 * COARSE_LDS_NODES];
@@ -1628,12 +1653,13 @@ __global__ __launch_bounds__(CBLOCK) void k_mg_coarse(CoarseArgs<T> A) {
     const KGrid &g = G.g;
     const int nn = A.lds_nn[A.lc], nx = g.n1 + 1, nb = nx * (g.n2 + 1) * (g.n3 + 1);
     int at[RL];
-    T bv[RL];
+    T bv[RL], uv[RL];
     int32_t lv[RL];
 #pragma unroll
     for (int r = 0; r < RL; ++r) {   // every read before the first wait
       const int t = (int)threadIdx.x + r * CBLOCK;
       lv[r] = t < nn ? G.bc[t] : 0;
+      uv[r] = WHOLE && t < nn ? G.u[t] : T(0);
       const uint32_t row = mdiv_q((uint32_t)t, G.d_n1p1), rk = mdiv_q(row, G.d_n2p1);
       at[r] = t < nb ? (int)gidx(g, 1 + t - (int)row * nx, 1 + (int)(row - rk * (g.n2 + 1)),
                                  1 + (int)rk)
@@ -1648,31 +1674,63 @@ __global__ __launch_bounds__(CBLOCK) void k_mg_coarse(CoarseArgs<T> A) {
     for (int r = 0; r < RL; ++r) {
       const int t = (int)threadIdx.x + r * CBLOCK;
       if (t < nn) labs[t] = label16(lv[r]);
+      if (WHOLE && t < nn) lds[t] = uv[r];
       if (at[r] >= 0) lds[nn + at[r]] = bv[r];
     }
   }
   __syncthreads();
   const int64_t nr = A.fixed ? A.nr_fixed : 4;
-  const int64_t nr_last = A.fixed ? A.nr_coarsest : (A.first_cycle ? 1000000 : 4);
-  // down from lc, the coarsest level, back up (one place that calls each
-  // routine: inlined, the arguments stay in scalar memory)
   const int m = ng - 1 - A.lc;
-  for (int v = 0; v <= 2 * m; ++v) {
-    const int l = v <= m ? A.lc + v : A.lc + 2 * m - v;
-    const int dig = v == m ? 0 : (v < m ? l + 1 - ng : ng - 1 - l);
-    const int64_t count = v == m ? nr_last : nr;
-    if (v > m) wg_prolongation(A, S, Lb, l);
-    if (PBC) {
-      wg_sor_rb(A, S, Lb, l, dig, count, red);
-      __syncthreads();
-      if (v < m) wg_restriction(A, S, Lb, l);
-    } else {
-      const KGrid &g = A.L[l].g;
-      if ((g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1) <= 2 * LEPIC_WAVE)
-        wg_level<T, LEPIC_WAVE, 2>(A, S, Lb, l, dig, count, v < m, red);
-      else
-        wg_level<T, CBLOCK, COARSE_SLOTS>(A, S, Lb, l, dig, count, v < m, red);
+  int cycle = WHOLE ? A.k : (A.first_cycle ? 1 : 2), state = WHOLE_DONE;
+  double fine = 0.0, first = A.res_s;
+  for (int done = 0;;) {
+    // down from lc, the coarsest level, back up (one place that calls each
+    // routine: inlined, the arguments stay in scalar memory)
+    for (int v = 0; v <= 2 * m; ++v) {
+      const int l = v <= m ? A.lc + v : A.lc + 2 * m - v;
+      const int dig = v == m ? 0 : (v < m ? l + 1 - ng : ng - 1 - l);
+      const int64_t count =
+          v == m ? (A.fixed ? A.nr_coarsest : (cycle == 1 ? 1000000 : 4)) : nr;
+      if (v > m) wg_prolongation(A, S, Lb, l);
+      if (PBC) {
+        wg_sor_rb(A, S, Lb, l, dig, count, red);
+        __syncthreads();
+        if (v < m) wg_restriction(A, S, Lb, l);
+      } else {
+        const KGrid &g = A.L[l].g;
+        const bool last = WHOLE && v == 2 * m;
+        const int nsor = (g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1);
+        if (nsor <= 2 * LEPIC_WAVE)
+          fine = wg_level<T, LEPIC_WAVE, 2>(A, S, Lb, l, dig, count, v < m, last, red);
+        else if (nsor <= 3 * CBLOCK)
+          fine = wg_level<T, CBLOCK, 3>(A, S, Lb, l, dig, count, v < m, last, red);
+        else
+          fine = wg_level<T, CBLOCK, COARSE_SLOTS>(A, S, Lb, l, dig, count, v < m, last, red);
+      }
     }
+    if (!WHOLE) break;
+    const double res = fine / A.alpha;
+    if (cycle == 1) {
+      first = res;
+    } else if (fabs(res / first) > 10.0) {
+      state = WHOLE_DIVERGED;
+      break;
+    }
+    if (res < A.tol || cycle == A.ncycl) break;
+    ++cycle;
+    if (++done == WHOLE_CYCLES) {
+      state = WHOLE_MORE;
+      break;
+    }
+    for (int c = 1; c < ng; ++c)   // the corrections start from 0 again
+      for (int t = threadIdx.x; t < A.lds_nn[c]; t += CBLOCK) lds[A.lds_off[c] + t] = T(0);
+    __syncthreads();
+  }
+  if (WHOLE && threadIdx.x == 0) {
+    A.ctl[0].res = fine;
+    A.ctl[0].pad[0] = cycle;
+    A.ctl[0].pad[1] = state;
+    A.ctl[0].pad[2] = __double_as_longlong(first);
   }
   __syncthreads();
   {
@@ -1735,8 +1793,8 @@ struct Solver {
   MGCtl *fin = nullptr;              // the level whose last sor_rb is still to be closed
   SlotCtl fin_sc = {};
 
-  void coarse(double eps, int kmg) {
-    CoarseArgs<T> A;
+  CoarseArgs<T> coarse_args(double eps, int kmg) {
+    CoarseArgs<T> A = {};
     for (int l = 0; l < MAX_LEVELS; ++l) A.L[l] = L[l];
     A.lc = lc;
     A.ng = ng;
@@ -1761,10 +1819,26 @@ struct Solver {
       A.lab_off[l] = off / 2;
       off += 2 * A.lds_nn[l];
     }
+    return A;
+  }
+
+  void coarse(double eps, int kmg) {
+    const CoarseArgs<T> A = coarse_args(eps, kmg);
     if (flag_pbc)
-      hipLaunchKernelGGL((k_mg_coarse<T, true>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
+      hipLaunchKernelGGL((k_mg_coarse<T, true, false>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
     else
-      hipLaunchKernelGGL((k_mg_coarse<T, false>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
+      hipLaunchKernelGGL((k_mg_coarse<T, false, false>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
+  }
+
+  // The launch of a whole solve from V-cycle k on (all levels in the workgroup).
+  void whole(double eps, int k, int ncycl, double alpha, double tol, double res_s) {
+    CoarseArgs<T> A = coarse_args(eps, k);
+    A.alpha = alpha;
+    A.tol = tol;
+    A.res_s = res_s;
+    A.k = k;
+    A.ncycl = ncycl;
+    hipLaunchKernelGGL((k_mg_coarse<T, false, true>), dim3(1), dim3(CBLOCK), 0, ctx->stream, A);
   }
 
   // One sweep; first: the sor_rb's first, whose red half arms ctl[l].
@@ -1995,10 +2069,10 @@ struct Solver {
   }
 
   // lc: the first level from which the remaining levels fit the coarse
-  // workgroup's LDS (ng: none do).
-  void choose_lc() {
+  // workgroup's LDS (ng: none do), from the given one on.
+  void choose_lc(int from = 1) {
     lc = ng;
-    for (int l = 1; l < ng; ++l) {
+    for (int l = from; l < ng; ++l) {
       int64_t tot = 0;
       for (int m = l; m < ng; ++m) tot += grid_nodes_k(L[m].g);
       if (tot <= COARSE_LDS_NODES) {
@@ -2127,13 +2201,15 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   double res = 0.0, res_s = 0.0;
   int k = 1;
   int status = LEPIC_OK;
-  S.choose_lc();
+  // a solve that fits one workgroup altogether is one launch
+  S.choose_lc(ng > 1 && !S.flag_pbc ? 0 : 1);
+  const bool whole = S.lc == 0;
   auto vcycle = [&](int kmg) -> int { return S.vcycle(kmg, epsa); };
   // With the coarsest level inside k_mg_coarse a V-cycle's launches are fixed
   // (every decision is taken on the device), so they are captured once per
   // solve configuration -- the first V-cycle and the later ones differ in one
   // argument -- and replayed: one submission per V-cycle instead of ~100.
-  const bool replay = mp->graph && S.lc < ng;
+  const bool replay = mp->graph && !whole && S.lc < ng;
   if (replay) {
     const int32_t ints[9] = {ng, g->n[0], g->n[1], g->n[2], S.flag_pbc, S.flag_nmn, S.lc, 0, 0};
     const void *ptrs[5] = {phi, rho, bcnd, ctx->mg_mem, ctx->d_ctrl};
@@ -2172,7 +2248,9 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
     }
   }
   for (;;) {
-    if (replay) {
+    if (whole) {
+      S.whole(epsa, k, mp->ncycl, alpha, mp->eps, res_s);
+    } else if (replay) {
       LEPIC_HIP(ctx, hipGraphLaunch(ctx->mg_exec[k == 1 ? 0 : 1], ctx->stream));
     } else {
       int st = vcycle(k);
@@ -2188,6 +2266,14 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
     double r;
     std::memcpy(&r, &ctx->h_pinned[2], sizeof(double));
     res = r / alpha;
+    if (whole) {   // the device has judged its cycles by the rules below
+      k = (int)ctx->h_pinned[5];
+      std::memcpy(&res_s, &ctx->h_pinned[7], sizeof(double));
+      if (ctx->h_pinned[6] == WHOLE_MORE) continue;
+      if (ctx->h_pinned[6] == WHOLE_DIVERGED)
+        status = lepic_fail(ctx, LEPIC_ERR_DIVERGED, "poisson: res/res_s > 10 (diverging)");
+      break;
+    }
     if (k == 1) res_s = res;
     else if (std::fabs(res / res_s) > 10.0) {
       status = lepic_fail(ctx, LEPIC_ERR_DIVERGED, "poisson: res/res_s > 10 (diverging)");

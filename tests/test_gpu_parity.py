@@ -333,6 +333,25 @@ def test_poisson_coarse_levels_bitexact(gpu, oracle, rng, n, ng, zero, nmn):
                                atol=1e-12 * np.abs(phi_o).max())
 
 
+def test_poisson_one_launch_cycles(gpu, oracle, rng):
+    """A solve that fits one workgroup runs its V-cycles in one launch of at most
+    64: past that bound and the V-cycle cap the same cycles and phi as the
+    oracle."""
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box((8, 12, 8))
+    bc = H.two_electrode_bcnd(n)
+    rho = np.where(bc <= 0, 1e-4 * rng.standard_normal(bc.shape), 0.0)
+    phi0 = np.where(bc == 2, 20.0, 0.0)
+    dev = [torch.as_tensor(a, device=gpu) for a in (bc, rho)]
+    phi_o, phi_g = phi0.copy(), torch.as_tensor(phi0, device=gpu)
+    st, info_o = oracle.pdesolver(n, h, phi_o, rho, bc, ng=3, eps=0.0, omega=1.4, ncycl=130)
+    info_g = F.solve_poisson_legacy(phi_g, dev[0], dev[1], h, n, 130, 0.0, 1.4, 3, 0, 0)
+    assert st == 0 and info_g["cycles"] == info_o["cycles"] == 130
+    # at the rounding floor (eps = 0) a residual's last bits decide the sweeps
+    np.testing.assert_allclose(phi_g.cpu().numpy(), phi_o, rtol=1e-12,
+                               atol=1e-12 * np.abs(phi_o).max())
+
+
 # Levels with periodic walls (k_per_half, k_per_end): one and two of them above
 # the one-workgroup levels, a block's share of nodes exceeded, and labels that
 # make the copies differ from node to node: electrodes and plasma on either copied
