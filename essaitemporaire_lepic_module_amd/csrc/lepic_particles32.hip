@@ -643,8 +643,15 @@ __global__ __launch_bounds__(BLOCK) void k_deposit32(KG32 g, KP32 p, int64_t n, 
   box32_flush(g, ds, rep);
 }
 
-// dep += sum of the int64 replicas; replicas cleared for the next deposit.
-__global__ void k_rep_flush_i64(long long *dep, unsigned long long *rep, int64_t nodes) {
+// dep += sum of the int64 replicas; replicas cleared for the next deposit.  With
+// wdrep one more block, the last, closes the push's wall diagnostics (a launch
+// of its own is 4 to 5 us).
+__global__ void k_rep_flush_i64(long long *dep, unsigned long long *rep, int64_t nodes,
+                                double *wdrep, double *p_mac, double *P_loss, int npairs) {
+  if (wdrep && blockIdx.x == gridDim.x - 1) {
+    wd_flush(wdrep, p_mac, P_loss, npairs);
+    return;
+  }
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= nodes) return;
   unsigned long long s = (unsigned long long)dep[i];
@@ -835,9 +842,10 @@ __global__ __launch_bounds__(BLOCK) void k_sort_count(KG32 g, const int32_t *__r
   }
 }
 
-// Exclusive scan of count[0..m) into start, in three launches: per-block
-// sums, one block over the block sums, then every block adds its offset.
-// The total goes to *total.
+// Exclusive scan of count[0..m) into start and cursor, in three launches:
+// per-block sums, one block over the block sums, then every block adds its
+// offset; up to SCAN_ONE cells in one block's launch (each launch is 4 us, the
+// one block's 5 at 4096 cells).  The total goes to *total.
 constexpr int SCAN_B = 1024;   // elements per block (4 per thread)
 
 __device__ inline int block_excl_scan(int v, int *wsum, int &total) {
@@ -892,7 +900,8 @@ __global__ __launch_bounds__(BLOCK) void k_scan_top(int32_t *bsum, int64_t nb, i
 }
 
 __global__ __launch_bounds__(BLOCK) void k_scan_apply(const int32_t *count, int64_t m,
-                                                      const int32_t *bsum, int32_t *start) {
+                                                      const int32_t *bsum, int32_t *start,
+                                                      int32_t *cursor) {
   __shared__ int wsum[BLOCK / 64 + 1];
   const int64_t b0 = (int64_t)blockIdx.x * SCAN_B + threadIdx.x * 4;
   int v[4], s = 0;
@@ -903,9 +912,38 @@ __global__ __launch_bounds__(BLOCK) void k_scan_apply(const int32_t *count, int6
   int total;
   int e = block_excl_scan(s, wsum, total) + bsum[blockIdx.x];
   for (int q = 0; q < 4; ++q) {
-    if (b0 + q < m) start[b0 + q] = e;
+    if (b0 + q < m) start[b0 + q] = cursor[b0 + q] = e;
     e += v[q];
   }
+}
+
+constexpr int SCAN_ONE_B = 1024, SCAN_ONE = 16 * SCAN_ONE_B;
+
+__global__ __launch_bounds__(SCAN_ONE_B) void k_scan_one(const int32_t *__restrict__ count, int m,
+                                                         int32_t *start, int32_t *cursor,
+                                                         int64_t *total) {
+  __shared__ int wsum[SCAN_ONE_B / 64];
+  const int b0 = (int)threadIdx.x * 16, lane = __lane_id(), w = (int)threadIdx.x >> 6;
+  int v[16], s = 0;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) v[q] = b0 + q < m ? count[b0 + q] : 0;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) s += v[q];
+  int inc = s;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(inc, d);
+    if (lane >= d) inc += o;
+  }
+  if (lane == 63) wsum[w] = inc;
+  __syncthreads();
+  int e = inc - s;
+  for (int i = 0; i < w; ++i) e += wsum[i];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    if (b0 + q < m) start[b0 + q] = cursor[b0 + q] = e;
+    e += v[q];
+  }
+  if (threadIdx.x == SCAN_ONE_B - 1) *total = e;
 }
 
 // Claim: cursor[c] starts at start[c]; each tile takes one run per cell.
@@ -1061,11 +1099,6 @@ __global__ void k_zero_i32(int32_t *a, int64_t n) {
   if (i < n) a[i] = 0;
 }
 
-__global__ void k_copy_i32(const int32_t *a, int32_t *b, int64_t n) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) b[i] = a[i];
-}
-
 __global__ void k_zero_u64_2(unsigned long long *a) {
   if (threadIdx.x < 2) a[threadIdx.x] = 0ull;
 }
@@ -1148,12 +1181,15 @@ int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, 
   hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, o.count, ncells);
   hipLaunchKernelGGL(k_sort_count, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell,
                      n, o.count);
-  hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, o.bsum, nb, o.total);
-  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
-                     o.start);
-  hipLaunchKernelGGL(k_copy_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, o.start, o.cursor,
-                     ncells);
+  if (ncells <= SCAN_ONE) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_B), 0, s, o.count, (int)ncells, o.start,
+                       o.cursor, o.total);
+  } else {
+    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum);
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, o.bsum, nb, o.total);
+    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
+                       o.start, o.cursor);
+  }
   hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell,
                      n, o.cursor, o.idx);
   LEPIC_LAUNCH_CHECK(ctx, "cell order");
@@ -1261,14 +1297,15 @@ int lepic_push32(lepic_ctx *ctx, const lepic_grid *g, lepic_pset32 *p, const flo
                                 rep, nodes, dd, p_mac, ctx->wdiag, lc, ec); break;
   }
   LEPIC_LAUNCH_CHECK(ctx, "k_push32");
-  hipLaunchKernelGGL(k_wd_flush, dim3(1), dim3(64), 0, ctx->stream, ctx->wdiag, p_mac, P_loss,
-                     std::min(bp->ngrid + 1, LEPIC_WD_LABELS));
-  LEPIC_LAUNCH_CHECK(ctx, "k_wd_flush");
-  if (dep) {
-    hipLaunchKernelGGL(k_rep_flush_i64, dim3(grid_blocks(nodes, 256)), dim3(256), 0, ctx->stream,
-                       reinterpret_cast<long long *>(dep), rep, nodes);
-    LEPIC_LAUNCH_CHECK(ctx, "k_rep_flush_i64");
-  }
+  const int npairs = std::min(bp->ngrid + 1, LEPIC_WD_LABELS);
+  if (dep)
+    hipLaunchKernelGGL(k_rep_flush_i64, dim3(grid_blocks(nodes, 256) + 1), dim3(256), 0,
+                       ctx->stream, reinterpret_cast<long long *>(dep), rep, nodes, ctx->wdiag,
+                       p_mac, P_loss, npairs);
+  else
+    hipLaunchKernelGGL(k_wd_flush, dim3(1), dim3(64), 0, ctx->stream, ctx->wdiag, p_mac, P_loss,
+                       npairs);
+  LEPIC_LAUNCH_CHECK(ctx, "push32 flush");
   return LEPIC_OK;
 }
 
@@ -1289,7 +1326,8 @@ int lepic_deposit32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *p, 
                      make_kg32(g, 0.0), kp32(p), p->n, (float)U, neg, rep, nodes);
   LEPIC_LAUNCH_CHECK(ctx, "k_deposit32");
   hipLaunchKernelGGL(k_rep_flush_i64, dim3(grid_blocks(nodes, 256)), dim3(256), 0, ctx->stream,
-                     reinterpret_cast<long long *>(dep), rep, nodes);
+                     reinterpret_cast<long long *>(dep), rep, nodes, (double *)nullptr,
+                     (double *)nullptr, (double *)nullptr, 0);
   LEPIC_LAUNCH_CHECK(ctx, "k_rep_flush_i64");
   return LEPIC_OK;
 }

@@ -137,7 +137,9 @@ __device__ inline void wd_finish(WallDiagShared &wd, double *rep) {
   }
 }
 
-__global__ void k_wd_flush(double *rep, double *p_mac, double *P_loss, int npairs) {
+// The replicas into p_mac / P_loss, cleared: one block of WD_STRIDE threads or
+// more.
+__device__ inline void wd_flush(double *rep, double *p_mac, double *P_loss, int npairs) {
   const int t = threadIdx.x;
   if (t >= WD_STRIDE) return;
   double v = 0.0;
@@ -150,6 +152,10 @@ __global__ void k_wd_flush(double *rep, double *p_mac, double *P_loss, int npair
   } else if (t < 2 * npairs && v != 0.0) {
     p_mac[t] += v;
   }
+}
+
+__global__ void k_wd_flush(double *rep, double *p_mac, double *P_loss, int npairs) {
+  wd_flush(rep, p_mac, P_loss, npairs);
 }
 
 // floor(t / d) for t, d < 2^16 by one multiply with m = ceil(2^32 / d): with

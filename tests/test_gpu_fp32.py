@@ -179,10 +179,12 @@ def test_sort32_stable_bitexact(gpu, oracle, rng, case):
 
 # k_sort_place: 8, 16, 32 and 64 lanes per cell (mean 2, 6, 18, 60); one and
 # two entries per lane, four (cells of 22 and 210), more (96 and 5018); bricks
-# of 16 x 8 x 8 cells whole, ragged and cut to a row.
+# of 16 x 8 x 8 cells whole, ragged and cut to a row.  16384 and 16385 cells: the
+# most of the one-block scan and one more.
 @pytest.mark.parametrize("n,mean,crowd", [((16, 8, 8), 2, 0), ((17, 9, 10), 2, 20),
                                           ((33, 7, 3), 6, 90), ((9, 20, 17), 18, 0),
                                           ((18, 16, 9), 60, 150), ((50, 1, 1), 18, 5000),
+                                          ((32, 32, 16), 2, 0), ((29, 113, 5), 1, 0),
                                           ((1, 1, 40), 60, 0)])
 def test_sort32_place_bitexact(gpu, oracle, rng, n, mean, crowd):
     """The stable order with holes dropped, exactly, and every field moved."""
