@@ -37,9 +37,9 @@ BYTES_PER_PARTICLE_STEP = 104   # FP64 fused gather+push+BC+deposit, state read 
 BYTES_PER_PARTICLE_STEP_F32 = 56   # FP32: int32 cell + 3 FP32 offsets + 3 FP32 velocities, r + w
 COPY_PROBE_BYTES = 1 << 31
 # FP64 multigrid, per node and executed sweep: u read and written, b and the
-# int32 label read (28 B), and the sweep's residual pass (u, b, label: 20 B);
-# restriction and prolongation not counted
-MG_BYTES_PER_NODE_SWEEP = 48
+# int32 label read (the residual comes out of the same launch); restriction and
+# prolongation not counted
+MG_BYTES_PER_NODE_SWEEP = 28
 SOLVES = {"fp64": "the FP64 multigrid",
           "pcg64": "FP64 conjugate gradients preconditioned with one FP64 V-cycle",
           "pcg": "FP64 conjugate gradients preconditioned with one FP32 V-cycle"}
@@ -231,7 +231,7 @@ def _step_bench(args, precision):
     for _ in range(args.steps):
         sim.advance_one_step(istep)
         istep += 1
-        # sweeps per level of this solve (each with its residual pass) x the
+        # sweeps per level of this solve x the
         # level's nodes, (n / 2^l + 1)^3
         mg_node_sweeps += sum(sw * ((args.n >> l) + 1) ** 3
                               for l, sw in enumerate(sim.last_mg["sweeps"]))
