@@ -17,6 +17,7 @@
 #include <cstring>
 
 #include "lepic_internal.h"
+#include "lepic_walk.h"
 
 namespace {
 
@@ -777,7 +778,7 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
                                                     T omega, int s, SlotCtl sc, MGCtl *ctl) {
   const bool judged = ctl != nullptr;
   const KGrid &g = L.g;
-  const int n = (g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1);
+  const int64_t n = (int64_t)(g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1);
   const T *own = colour ? (const T *)L.u : X, *other = colour ? X : (const T *)L.u;
   T *out = colour ? L.u : Xn;
   const bool pull = colour == 1 || s > 0;
@@ -785,8 +786,8 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
   T b = T(0), uc = T(0);
   Nbr6<T> v = {};
   bool node = false;
-  auto load = [&](int t) {
-    node = t < n && per_node(L, colour, t, i, j, k);
+  auto load = [&](int64_t t) {
+    node = t < n && per_node(L, colour, (int)t, i, j, k);
     if (!node) return;
     const int64_t c = gidx(g, i, j, k);
     lab = L.bc[c];
@@ -795,8 +796,8 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
     v = per_neighbours(L, other, i, j, k, pull);
   };
   // everything the launch reads is under way before the decision
-  int t = blockIdx.x * BLOCK + threadIdx.x;
-  load(t);
+  NodeWalk nw = walk_strided(n, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, BLOCK);
+  load(nw.t);
   if (judged && s > 0) {
     const double share = colour ? per_share(sc, s - 1) : 0.0;
     const SlotState st = sc.state[s - 1];
@@ -846,9 +847,9 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
       }
       if (judged && colour == 1 && lab == -1) a = a + per_resid(L, b, uc, v);
     }
-    t += gridDim.x * BLOCK;
-    if (t >= n) break;
-    load(t);
+    nw.t += nw.step;
+    if (nw.t >= nw.end) break;
+    load(nw.t);
   }
   if (judged && (colour == 1 || s > 0))
     per_partial(a, sc.partials + (colour ? (int64_t)(s & 1) : 2) * sc.nparts);
@@ -869,11 +870,14 @@ __global__ __launch_bounds__(BLOCK) void k_per_end(KLevelT<T> L, MDiv d_n2p3, co
   }
   const KGrid &g = L.g;
   const T *X = (count & 1) ? u2 : (const T *)L.u;
-  const int nx = g.n1 + 3, nodes = nx * (g.n2 + 3) * (g.n3 + 3);
+  const int nx = g.n1 + 3;
   double a = 0.0;
-  for (int t = blockIdx.x * BLOCK + threadIdx.x; t < nodes; t += gridDim.x * BLOCK) {
+  const NodeWalk nw = walk_strided((int64_t)nx * (g.n2 + 3) * (g.n3 + 3), (int)blockIdx.x,
+                                   (int)gridDim.x, (int)threadIdx.x, BLOCK);
+  for (int64_t t = nw.t; t < nw.end; t += nw.step) {
     const uint32_t r = mdiv_q((uint32_t)t, L.d_n1p3), rk = mdiv_q(r, d_n2p3);
-    const int i = t - (int)r * nx, j = (int)(r - rk * (uint32_t)(g.n2 + 3)), k = (int)rk;
+    const int i = (int)((uint32_t)t - r * (uint32_t)nx),
+              j = (int)(r - rk * (uint32_t)(g.n2 + 3)), k = (int)rk;
     const bool is_red = (i + j + k) & 1;
     int sj = j, sk = k;
     per_source(L, i, sj, sk);
@@ -2315,16 +2319,8 @@ constexpr int MIX_BLOCKS = 1024;
 // turn) walks its own eighth of the nodes in order, so that the planes above and
 // below are still in its L2: CG direction at 256^3 221 -> 181 us.  (k_pcg_resid
 // writes more than it reads and is 4 % faster striding over all blocks.)
-struct NodeWalk {
-  int64_t t, end, step;
-};
-
 __device__ inline NodeWalk node_walk(int64_t nodes) {
-  const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (gridDim.x % LEPIC_XCDS != 0) return {i, nodes, (int64_t)gridDim.x * BLOCK};
-  const int64_t per = (nodes / LEPIC_XCDS + BLOCK) / BLOCK * BLOCK, b = blockIdx.x % LEPIC_XCDS * per;
-  return {b + (int64_t)(blockIdx.x / LEPIC_XCDS) * BLOCK + threadIdx.x,
-          b + per < nodes ? b + per : nodes, (int64_t)(gridDim.x / LEPIC_XCDS) * BLOCK};
+  return walk_grouped(nodes, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, BLOCK, LEPIC_XCDS);
 }
 
 // FP64 residual of the refinement step at ghosted node t; r32, e32 (the
