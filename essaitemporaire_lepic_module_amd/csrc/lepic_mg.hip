@@ -2217,7 +2217,8 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   if (replay) {
     const int32_t ints[9] = {ng, g->n[0], g->n[1], g->n[2], S.flag_pbc, S.flag_nmn, S.lc, 0, 0};
     const void *ptrs[5] = {phi, rho, bcnd, ctx->mg_mem, ctx->d_ctrl};
-    const double dbl[5] = {g->h[0], g->h[1], g->h[2], S.omega, epsa};
+    // eps0: the levels' coefficients are in the captured launches
+    const double dbl[6] = {g->h[0], g->h[1], g->h[2], S.omega, epsa, mp->eps0};
     std::vector<unsigned char> key(sizeof(ints) + sizeof(ptrs) + sizeof(dbl));
     std::memcpy(key.data(), ints, sizeof(ints));
     std::memcpy(key.data() + sizeof(ints), ptrs, sizeof(ptrs));

@@ -398,6 +398,27 @@ def test_poisson_periodic_levels_bitexact(gpu, oracle, rng, n, ng, mess):
         np.testing.assert_allclose(info_g["res"], info_o["res"], rtol=1e-9)
 
 
+def test_poisson_graph_follows_eps0(gpu, rng):
+    """Two solves on the same buffers whose alpha * eps is the same number
+    (eps0, eps and 2 eps0, eps / 2): the second is not the first one's captured
+    V-cycles, whose coefficients hold the other eps0."""
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box((32, 32, 32))
+    bc = torch.as_tensor(cfg.biased_wall_bcnd(n, 2), device=gpu)
+    rho = torch.as_tensor(1e-5 * rng.standard_normal(cfg.node_shape(n)), device=gpu)
+    rho = torch.where(bc <= 0, rho, 0.0)
+    phi = torch.empty_like(rho)
+    out = {}
+    for scale, graph in ((1.0, True), (2.0, True), (2.0, False)):
+        phi.copy_(torch.where(bc == 2, 20.0, 0.0))
+        info = F.solve_poisson_legacy(phi, bc, rho, h, n, 20000, 1e-8 / scale, 1.4, 5, 0, 0,
+                                      eps0=scale * F.EPS0, graph=graph)
+        out[scale, graph] = (phi.clone(), info)
+    assert torch.equal(out[2.0, True][0], out[2.0, False][0])
+    assert out[2.0, True][1] == out[2.0, False][1]
+    assert not torch.equal(out[2.0, True][0], out[1.0, True][0])
+
+
 def test_loader_host_bitexact(oracle):
     """The product's host loader reproduces the reference loader's ran2 stream."""
     from essaitemporaire_lepic_module_amd import particles as P
