@@ -2539,6 +2539,17 @@ extern "C" int lepic_poisson_solve_mixed(lepic_ctx *ctx, const lepic_grid *g, do
   float *e32 = M.e32, *r32 = M.r32;
   const double alpha = M.alpha;
   const unsigned rb = M.rb;
+  // phi's periodic ghosts from their images (sors.f90:184-239): before the first
+  // residual, which reads them as a caller left them, and after a correction
+  auto ghosts = [&]() {
+    if (!mp->flag_pbc) return;
+    const KGrid &gg = F64.g;
+    const MGCtl *always = nullptr;
+    hipLaunchKernelGGL(k_per_y<double>, dim3(grid_blocks((int64_t)(gg.n1 + 3) * (gg.n3 + 3), BLOCK)),
+                       dim3(BLOCK), 0, ctx->stream, F64, always);
+    hipLaunchKernelGGL(k_per_z<double>, dim3(grid_blocks((int64_t)(gg.n1 + 3) * (gg.n2 + 3), BLOCK)),
+                       dim3(BLOCK), 0, ctx->stream, F64, always);
+  };
   // the inner V-cycles and the correction of one refinement step: one
   // captured graph per solve configuration
   auto inner = [&]() -> int {
@@ -2548,13 +2559,7 @@ extern "C" int lepic_poisson_solve_mixed(lepic_ctx *ctx, const lepic_grid *g, do
     }
     hipLaunchKernelGGL(k_mix_correct, dim3(grid_blocks(nodes, 256)), dim3(256), 0, ctx->stream,
                        phi, e32, bcnd, nodes);
-    if (mp->flag_pbc) {   // phi's periodic ghosts from their images (sors.f90:184-239)
-      const KGrid &gg = F64.g;
-      hipLaunchKernelGGL(k_per_y<double>, dim3(grid_blocks((int64_t)(gg.n1 + 3) * (gg.n3 + 3), BLOCK)),
-                         dim3(BLOCK), 0, ctx->stream, F64, &S.ctl[0]);
-      hipLaunchKernelGGL(k_per_z<double>, dim3(grid_blocks((int64_t)(gg.n1 + 3) * (gg.n2 + 3), BLOCK)),
-                         dim3(BLOCK), 0, ctx->stream, F64, &S.ctl[0]);
-    }
+    ghosts();
     return LEPIC_OK;
   };
   const bool replay = mp->graph != 0;
@@ -2594,6 +2599,7 @@ extern "C" int lepic_poisson_solve_mixed(lepic_ctx *ctx, const lepic_grid *g, do
     }
   }
   hipLaunchKernelGGL(k_reset_totals, dim3(1), dim3(64), 0, ctx->stream, S.ctl, MAX_LEVELS);
+  ghosts();
   double res = 0.0, res_s = 0.0;
   int k = 0;
   int status = LEPIC_OK;

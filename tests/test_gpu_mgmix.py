@@ -69,6 +69,31 @@ def test_mixed_periodic_and_neumann(gpu, oracle, rng):
     assert np.abs(phi_g[phys] - phi_o[phys]).max() <= 1e-8 * np.abs(phi_o).max()
 
 
+@pytest.mark.parametrize("n,ng,graph", [((16, 16, 16), 4, True), ((24, 20, 12), 3, False),
+                                        ((32, 24, 40), 3, True)])
+def test_mixed_periodic_start_ghosts(gpu, oracle, rng, n, ng, graph):
+    """A start whose periodic ghost planes are no copies of their images: the
+    solve makes the copies before its first residual, so it converges to the
+    FP64 solution, ghosts included (1e-8 of max |phi|, the residual bound's
+    agreement).  Also from a start that needs no step but for its ghosts."""
+    n, h = H.box(n)
+    bc = H.periodic_yz_bcnd(n)
+    phi0 = np.where(bc == 1, 3.0, rng.standard_normal(bc.shape))
+    rhs = np.where(bc == -1, 1e-6 * rng.standard_normal(bc.shape), 0.0)
+    phi_o, phi_g, _, info = _solve_both(oracle, gpu, n, h, bc, phi0, rhs, ng, 1e-10, flag_pbc=1,
+                                        graph=graph)
+    # the planes past the last periodic one belong to neither solver
+    used = np.s_[:n[2] + 2, :n[1] + 2, :n[0] + 2]
+    assert info["res"] < 1e-10
+    assert np.abs(phi_g - phi_o)[used].max() <= 1e-8 * np.abs(phi_o).max()
+    warm = phi_g.copy()
+    warm[:, 0, 2:n[0] + 1] = warm[0, :, 2:n[0] + 1] = 7.0
+    _, phi_w, _, info = _solve_both(oracle, gpu, n, h, bc, warm, rhs, ng, 1e-10, flag_pbc=1,
+                                    graph=graph)
+    assert info["cycles"] == 0 and info["res"] < 1e-10
+    assert np.abs(phi_w - phi_o)[used].max() <= 1e-8 * np.abs(phi_o).max()
+
+
 def test_mixed_warm_start_and_graph(gpu, oracle):
     """A warm start that already meets the tolerance takes no refinement
     step; replaying the captured refinement step (graph) and launching it
