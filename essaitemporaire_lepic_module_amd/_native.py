@@ -23,7 +23,7 @@ MCC_PHILOX = 1
 # Every symbol include/lepic.h declares.
 EXPORTS = (
     "lepic_create", "lepic_destroy", "lepic_last_error", "lepic_set_stream", "lepic_synchronize",
-    "lepic_version", "lepic_ran2", "lepic_seed", "lepic_load_particles_host",
+    "lepic_limit_scratch", "lepic_version", "lepic_ran2", "lepic_seed", "lepic_load_particles_host",
     "lepic_load_uniform_device", "lepic_sort_particles_by_cell", "lepic_move_electrostatic",
     "lepic_move_boris", "lepic_apply_bc", "lepic_build_kq", "lepic_fill", "lepic_deposit",
     "lepic_deposit_fixed",
@@ -151,6 +151,7 @@ def load() -> C.CDLL:
             "lepic_destroy": (C.c_int, [vp]),
             "lepic_last_error": (C.c_char_p, [vp]),
             "lepic_set_stream": (C.c_int, [vp, vp]),
+            "lepic_limit_scratch": (C.c_int, [vp, C.c_int64]),
             "lepic_synchronize": (C.c_int, [vp]),
             "lepic_version": (C.c_char_p, []),
             "lepic_ran2": (C.c_double, [i32p]),

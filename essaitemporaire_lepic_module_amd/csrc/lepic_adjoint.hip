@@ -648,9 +648,15 @@ int adj_order(lepic_ctx *ctx, const lepic_grid *g, const KGrid &kg, const lepic_
   const int64_t n = state->n;
   const int32_t dims[3] = {g->n[0] + 2, g->n[1] + 2, g->n[2] + 2};
   if (n < ORDER_MIN || n >= ((int64_t)1 << 31) - 4096) return LEPIC_OK;
+  // As they stand, too, where the scratch cannot be had, and while the caller
+  // captures the stream: the scratch may not grow then, and its next user would
+  // write into what the graph reads.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+  if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
+  if (capture != hipStreamCaptureStatusNone) return LEPIC_OK;
   CellOrder o;
-  int st = lepic_order_alloc(ctx, dims, n, n, o);
-  if (st) return st;
+  if (!lepic_order_alloc(ctx, dims, n, n, o)) return LEPIC_OK;
+  int st;
   hipLaunchKernelGGL(k_adj_cells, dim3(grid_blocks(n, BLOCK)), dim3(BLOCK), 0, ctx->stream, kg,
                      *state, n, o.extra);
   if ((st = lepic_order_run(ctx, dims, o.extra, n, o))) return st;

@@ -1,4 +1,5 @@
 // lepic_ctx.hip -- context, errors, host RNG and the host loader.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -15,6 +16,12 @@ int lepic_hip_check(lepic_ctx *ctx, hipError_t e, const char *what) {
   return lepic_fail(ctx, LEPIC_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+namespace {
+bool scratch_allowed(const lepic_ctx *ctx, size_t bytes) {
+  return ctx->scratch_limit == 0 || bytes <= ctx->scratch_limit;
+}
+}  // namespace
+
 void *lepic_scratch(lepic_ctx *ctx, size_t bytes, int which) {
   void **p = which == 0 ? &ctx->scratch : &ctx->scratch2;
   size_t *cur = which == 0 ? &ctx->scratch_bytes : &ctx->scratch2_bytes;
@@ -26,7 +33,12 @@ void *lepic_scratch(lepic_ctx *ctx, size_t bytes, int which) {
     *cur = 0;
   }
   size_t want = bytes + bytes / 8 + 4096;
-  if (hipMalloc(p, want) != hipSuccess) return nullptr;
+  if (ctx->scratch_limit) want = std::min(want, std::max(bytes, ctx->scratch_limit));
+  if (!scratch_allowed(ctx, bytes) || hipMalloc(p, want) != hipSuccess) {
+    (void)hipGetLastError();   // the null says it; a caller that goes on checks its launches
+    *p = nullptr;
+    return nullptr;
+  }
   *cur = want;
   return *p;
 }
@@ -120,6 +132,24 @@ const char *lepic_last_error(lepic_ctx *ctx) { return ctx ? ctx->err.c_str() : "
 int lepic_set_stream(lepic_ctx *ctx, void *hip_stream) {
   if (!ctx) return LEPIC_ERR_ARG;
   ctx->stream = reinterpret_cast<hipStream_t>(hip_stream);
+  return LEPIC_OK;
+}
+
+int lepic_limit_scratch(lepic_ctx *ctx, int64_t bytes) {
+  if (!ctx) return LEPIC_ERR_ARG;
+  if (bytes < 0) return lepic_fail(ctx, LEPIC_ERR_ARG, "limit_scratch: negative bound");
+  ctx->scratch_limit = (size_t)bytes;
+  if (bytes > 0 && (ctx->scratch_bytes > (size_t)bytes || ctx->scratch2_bytes > (size_t)bytes)) {
+    LEPIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    for (int which = 0; which < 2; ++which) {
+      void *&p = which == 0 ? ctx->scratch : ctx->scratch2;
+      size_t &held = which == 0 ? ctx->scratch_bytes : ctx->scratch2_bytes;
+      if (held <= (size_t)bytes) continue;
+      LEPIC_HIP(ctx, hipFree(p));
+      p = nullptr;
+      held = 0;
+    }
+  }
   return LEPIC_OK;
 }
 

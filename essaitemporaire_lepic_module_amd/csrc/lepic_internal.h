@@ -25,6 +25,7 @@ struct lepic_ctx {
   size_t scratch_bytes = 0;
   void *scratch2 = nullptr;
   size_t scratch2_bytes = 0;
+  size_t scratch_limit = 0;           // most bytes of either (0: no bound)
   // small device control block: counters, flags, partial sums
   int64_t *d_ctrl = nullptr;          // 4096 int64 words
   int64_t *h_pinned = nullptr;        // 4096 pinned host words for readbacks
@@ -103,7 +104,8 @@ struct CellOrder {
   int32_t *extra;    // the words asked for besides
   int64_t *total;
 };
-int lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o);
+// false: the scratch cannot be had
+bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o);
 int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
                     const CellOrder &o);
 // Resolves, once per device, the static scratch lepic_efield_noalloc uses

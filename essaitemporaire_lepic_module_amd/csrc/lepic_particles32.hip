@@ -1151,12 +1151,12 @@ unsigned long long *int_replicas(lepic_ctx *ctx, int64_t nodes) {
 
 // The order of n particles by cell id (count, scan and claim of the sort): ids
 // below 0 are dropped, the order within a cell is the atomics'.
-int lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o) {
+bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o) {
   const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
   const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
   const size_t words = (size_t)(3 * ncells + nb + n + extra + 64);
   int32_t *w = reinterpret_cast<int32_t *>(lepic_scratch(ctx, sizeof(int32_t) * words, 0));
-  if (!w) return lepic_fail(ctx, LEPIC_ERR_HIP, "cell order: scratch");
+  if (!w) return false;
   o.extra = w;                              // 256-byte aligned
   o.count = w + ((extra + 15) & ~(int64_t)15);
   o.start = o.count + ncells;
@@ -1164,7 +1164,7 @@ int lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t 
   o.bsum = o.cursor + ncells;
   o.idx = o.bsum + nb;
   o.total = ctx->d_ctrl + CTRL_COUNT_OUT;
-  return LEPIC_OK;
+  return true;
 }
 
 int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
@@ -1364,8 +1364,9 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
   const KG32 kg = make_kg32(g, 0.0);
   const hipStream_t s = ctx->stream;
   CellOrder o;
-  if ((st = lepic_order_alloc(ctx, g->n, n, 0, o)) || (st = lepic_order_run(ctx, g->n, src->cell, n, o)))
-    return st;
+  if (!lepic_order_alloc(ctx, g->n, n, 0, o))
+    return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: scratch");
+  if ((st = lepic_order_run(ctx, g->n, src->cell, n, o))) return st;
   // lanes per cell: the mean cell and twice its spread in one entry per lane
   const double mean = (double)n / (double)ncells, wide = mean + 2.0 * std::sqrt(mean);
   const int bx = (g->n[0] + BRX - 1) / BRX, by = (g->n[1] + BRY - 1) / BRY,

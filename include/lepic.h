@@ -146,6 +146,10 @@ int lepic_create(int32_t device, lepic_ctx **out);
 int lepic_destroy(lepic_ctx *ctx);
 const char *lepic_last_error(lepic_ctx *ctx);
 int lepic_set_stream(lepic_ctx *ctx, void *hip_stream); /* NULL = null stream */
+/* Bounds the context's scratch: each of its two buffers stays within bytes (0:
+ * no bound).  A call that can do without takes another path, the others
+ * return LEPIC_ERR_HIP. */
+int lepic_limit_scratch(lepic_ctx *ctx, int64_t bytes);
 int lepic_synchronize(lepic_ctx *ctx);
 const char *lepic_version(void);
 

@@ -234,6 +234,63 @@ def test_adj_push_cell_order_matches_slot_order(gpu, field):
         assert np.abs(u - v).max() <= 1e-12 * max(np.abs(v).max(), 1e-300)
 
 
+def test_adj_push_without_scratch_and_captured(gpu):
+    """From 2^19 particles the push adjoint orders them on the context's scratch.
+    Where that cannot be had, and while the caller captures the stream, it takes
+    them as they stand: every particle's values bit-identical, dL/dE to 1e-12 of
+    its largest entry, each replay of the graph included."""
+    n, h, bc = _box((13, 9, 14))
+    rng = np.random.default_rng(8)
+    N = (1 << 19) + 5
+    pos, vel = _particles(rng, n, h, N, 1e5)
+    E4 = torch.as_tensor(1e4 * rng.standard_normal(cfg.node_shape(n) + (4,)), device=gpu)
+    p, keep = _dev_state(pos, vel)
+    lx, lv = rng.standard_normal((N, 3)), rng.standard_normal((N, 3)) * 1e-7
+    g = _native.grid(n, h)
+    ctx = _native.Context(0)     # its own scratch, none yet
+    a, lam = _adj_set((*lx.T, *lv.T))
+    start = {k: v.clone() for k, v in lam.items()}
+    lamE = torch.zeros(cfg.node_shape(n) + (4,), dtype=torch.float64, device=gpu)
+
+    def push(count=N):
+        p.n = a.n = count
+        ctx.bind_stream(torch.cuda.current_stream().cuda_stream)
+        ctx.check(ctx.lib.lepic_adj_push(ctx.h, C.byref(g), C.byref(p), C.byref(a),
+                                         E4.data_ptr(), None, -QE, ME, DT, lamE.data_ptr(), None))
+
+    def reset():
+        for k, v in lam.items():
+            v.copy_(start[k])
+        lamE.zero_()
+
+    def result():
+        torch.cuda.synchronize()
+        return {k: v.cpu().numpy() for k, v in lam.items()}, lamE.cpu().numpy()
+
+    ctx.check(ctx.lib.lepic_limit_scratch(ctx.h, 1 << 16))
+    push()
+    out = [result()]
+    push(1000)                   # its later launches report no error left behind
+    reset()
+    graph = torch.cuda.CUDAGraph()
+    ctx.check(ctx.lib.lepic_limit_scratch(ctx.h, 0))
+    with torch.cuda.graph(graph):
+        push()
+    for _ in range(3):
+        reset()
+        graph.replay()
+        out.append(result())
+    reset()
+    push()
+    ordered = result()
+    for vals, dE in out:
+        for k in vals:
+            np.testing.assert_array_equal(vals[k], ordered[0][k])
+        assert np.abs(dE - ordered[1]).max() <= 1e-12 * np.abs(ordered[1]).max()
+    torch.cuda.synchronize()
+    ctx.close()
+
+
 @pytest.mark.parametrize("geometry", ["block", "thin_gaps"])
 def test_adj_efield_is_the_transpose(gpu, rng, geometry):
     """<lamE, D phi> = <D^T lamE, phi> with D = lepic_efield, and D^T lamE
