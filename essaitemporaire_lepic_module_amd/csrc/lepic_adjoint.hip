@@ -52,15 +52,6 @@ __device__ inline void weight_grads(double px, double py, double pz, const doubl
        px * qy * (e[3] - e[7]);
 }
 
-// The mover's stencil lower node (make_stencil): ix = int(x/h) + 1 clamped
-// to [0, n + 1] per axis.
-__device__ inline void stencil_lo(const KGrid &g, double xp, double yp, double zp, int &ix,
-                                  int &iy, int &iz) {
-  ix = imax(0, imin(g.n1 + 1, (int)qdiv(xp, g.q1) + 1));
-  iy = imax(0, imin(g.n2 + 1, (int)qdiv(yp, g.q2) + 1));
-  iz = imax(0, imin(g.n3 + 1, (int)qdiv(zp, g.q3) + 1));
-}
-
 // The mover's stencil (make_stencil) with its fractions kept.
 __device__ inline void stencil_fracs(const KGrid &g, double xp, double yp, double zp,
                                      int64_t &base, double &px, double &py, double &pz,
@@ -118,17 +109,26 @@ __device__ inline void adj_flush(const KGrid &g, double *dst, int64_t b, const d
 constexpr int ABOX = 1536;                            // nodes: 36 KB of LDS
 constexpr int ABOX_X = 24, ABOX_Y = 8, ABOX_Z = 8;    // cut extents, product <= ABOX
 static_assert(ABOX_X * ABOX_Y * ABOX_Z <= ABOX, "adjoint box limits exceed the box");
-struct AdjBox {
+struct AdjBounds {
   int mn[3], mx[3], sum[3], cnt;
   int x0, y0, z0, ex, ey, ez, vol;   // vol 0: no box
+};
+struct AdjBox : AdjBounds {
   double v[3 * ABOX];
 };
+
+// Whether the stencil at lower node (ix, iy, iz) lies in the box.
+__device__ inline bool adj_in_box(const AdjBounds &bx, int ix, int iy, int iz) {
+  const int lx = ix - bx.x0, ly = iy - bx.y0, lz = iz - bx.z0;
+  return bx.vol > 0 && lx >= 0 && ly >= 0 && lz >= 0 && lx + 1 < bx.ex && ly + 1 < bx.ey &&
+         lz + 1 < bx.ez;
+}
 
 // lo / hi / sm / cnt: the lane's lower nodes' bounds, sum and count.  The
 // box spans the block's lower nodes and one node above (the stencils), cut
 // to ABOX_* around the mean lower node when that exceeds ABOX nodes.
-__device__ inline void adj_box_begin(const KGrid &g, AdjBox &bx, const int lo[3], const int hi[3],
-                                     const int sm[3], int cnt) {
+__device__ inline void adj_box_bounds(const KGrid &g, AdjBounds &bx, const int lo[3],
+                                      const int hi[3], const int sm[3], int cnt) {
   if (threadIdx.x == 0) {
     bx.mn[0] = bx.mn[1] = bx.mn[2] = 1 << 30;
     bx.mx[0] = bx.mx[1] = bx.mx[2] = -(1 << 30);
@@ -176,6 +176,11 @@ __device__ inline void adj_box_begin(const KGrid &g, AdjBox &bx, const int lo[3]
     bx.vol = vol;
   }
   __syncthreads();
+}
+
+__device__ inline void adj_box_begin(const KGrid &g, AdjBox &bx, const int lo[3], const int hi[3],
+                                     const int sm[3], int cnt) {
+  adj_box_bounds(g, bx, lo, hi, sm, cnt);
   for (int t = threadIdx.x; t < 3 * bx.vol; t += BLOCK) bx.v[t] = 0.0;
   __syncthreads();
 }
@@ -185,10 +190,8 @@ __device__ inline void adj_box_begin(const KGrid &g, AdjBox &bx, const int lo[3]
 __device__ inline void adj_flush_box(const KGrid &g, AdjBox &bx, double *dst, int64_t b, int ix,
                                      int iy, int iz, const double acc[8][3]) {
   if (b < 0) return;
-  const int lx = ix - bx.x0, ly = iy - bx.y0, lz = iz - bx.z0;
-  if (bx.vol > 0 && lx >= 0 && ly >= 0 && lz >= 0 && lx + 1 < bx.ex && ly + 1 < bx.ey &&
-      lz + 1 < bx.ez) {
-    const int l = lx + bx.ex * (ly + bx.ey * lz);
+  if (adj_in_box(bx, ix, iy, iz)) {
+    const int l = (ix - bx.x0) + bx.ex * ((iy - bx.y0) + bx.ey * (iz - bx.z0));
     const int sy = bx.ex, sz = bx.ex * bx.ey;
     const int o[8] = {0, 1, sy + 1, sy, sz, sz + 1, sz + sy + 1, sz + sy};
 #pragma unroll
@@ -218,19 +221,67 @@ __device__ inline void adj_box_flush(const KGrid &g, AdjBox &bx, double *dst) {
   }
 }
 
-// The cell (lower node, [0, n + 1] per axis) of each live particle, -1 of the
-// others.
-__global__ __launch_bounds__(BLOCK) void k_adj_cells(KGrid g, lepic_pset st, int64_t n,
-                                                     int32_t *cell) {
-  const int64_t i = blockIdx.x * (int64_t)BLOCK + threadIdx.x;
-  if (i >= n) return;
-  int c = -1;
-  if (st.dead[i] == 0) {
-    int jx, jy, jz;
-    stencil_lo(g, st.x[i], st.y[i], st.z[i], jx, jy, jz);
-    c = jx + (g.n1 + 2) * (jy + (g.n2 + 2) * jz);
+// Clears count, and one block's worth of particles of each ORDER_SAMPLES-th part
+// of the set, as they stand, votes in its word of gate on whether the cells' order
+// pays: -1 per particle and, unless they are in that order already, ORDER_SHARE
+// per run outside the block's box (24 global atomics each).  The line lies where
+// both orders take as long.  As they stand and ordered anew (us): 8.4M on 128^3
+// with 0.10 runs outside per particle 1200 and 1115, with 0.24 2190 and 1125; 2.1M
+// on 64^3 with 0.11 361 and 326, with 0.03 255 and 310; 0.5M on 32^3 with 0.12 161
+// and 158; 2.2M on 48^3 with 0.05 274 and 464.  A vote against costs 10 to 15 us
+// (this launch and the idle ones after it).
+constexpr int ORDER_SHARE = 10;
+
+__global__ __launch_bounds__(BLOCK) void k_adj_probe(KGrid g, lepic_pset st, int64_t n,
+                                                     int32_t *count, int64_t ncells,
+                                                     int32_t *gate) {
+  const int64_t t = blockIdx.x * (int64_t)BLOCK + threadIdx.x;
+  if (t < ncells) count[t] = 0;
+  if (blockIdx.x >= ORDER_SAMPLES) return;
+  __shared__ AdjBounds bx;
+  __shared__ int vote;
+  const int64_t blocks = (n + BLOCK * APT - 1) / (BLOCK * APT);
+  // somewhere in its part: evenly spaced blocks may all lie on the step from one
+  // plane of cells to the next
+  const int64_t b0 = blockIdx.x * blocks / ORDER_SAMPLES,
+                b1 = (blockIdx.x + 1) * blocks / ORDER_SAMPLES;
+  const int64_t b = b0 + (int64_t)(((uint32_t)blockIdx.x * 2654435769u) >> 8) % (b1 - b0);
+  const int64_t i0 = (b * BLOCK + threadIdx.x) * APT;
+  int lo[3] = {1 << 30, 1 << 30, 1 << 30}, hi[3] = {-(1 << 30), -(1 << 30), -(1 << 30)};
+  int sm[3] = {0, 0, 0}, cnt = 0;
+  int j[APT][3];
+#pragma unroll
+  for (int q = 0; q < APT; ++q) {
+    j[q][0] = -1;
+    if (i0 + q >= n || st.dead[i0 + q] != 0) continue;
+    stencil_lo(g, st.x[i0 + q], st.y[i0 + q], st.z[i0 + q], j[q][0], j[q][1], j[q][2]);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      lo[d] = min(lo[d], j[q][d]);
+      hi[d] = max(hi[d], j[q][d]);
+      sm[d] += j[q][d];
+    }
+    ++cnt;
   }
-  cell[i] = c;
+  if (threadIdx.x == 0) vote = 0;
+  adj_box_bounds(g, bx, lo, hi, sm, cnt);
+  int outside = 0, first = -1, last = -1;
+  bool falls = false;
+#pragma unroll
+  for (int q = 0; q < APT; ++q) {
+    if (j[q][0] < 0) continue;
+    const int c = j[q][0] + (g.n1 + 2) * (j[q][1] + (g.n2 + 2) * j[q][2]);
+    if (c != last && !adj_in_box(bx, j[q][0], j[q][1], j[q][2])) ++outside;
+    if (first < 0) first = c;
+    falls = falls || c < last;
+    last = c;
+  }
+  const int next = __shfl_down(first, 1);   // the wave's last lane: its own, no fall
+  falls = falls || (next >= 0 && next < last && __lane_id() < LEPIC_WAVE - 1);
+  const int v = wave_sum_i(ORDER_SHARE * outside);
+  if (__lane_id() == 0) atomicAdd(&vote, v);
+  if (!__syncthreads_or(falls) && threadIdx.x == 0) vote = 0;
+  if (threadIdx.x == 0) gate[blockIdx.x] = vote - bx.cnt;
 }
 
 // MAP: B is a map on the E grid gathered with the particle's stencil and
@@ -243,16 +294,18 @@ __global__ __launch_bounds__(BLOCK) void k_adj_push(KGrid g, lepic_pset st, KAdj
                                                     double k1, double dt, double *rep,
                                                     int64_t nodes, double *lamB,
                                                     const int32_t *__restrict__ idx,
-                                                    const int64_t *__restrict__ total) {
+                                                    const int64_t *__restrict__ total,
+                                                    const int32_t *__restrict__ gate) {
   __shared__ AdjBox bx;
   const int64_t i0 = (blockIdx.x * (int64_t)BLOCK + threadIdx.x) * APT;
   double *dst = rep + (int64_t)xcc_id() * 4 * nodes;
   int64_t pi[APT];   // the lane's particles
   {
-    const int64_t m = idx ? *total : n;
+    const bool ordered = idx && order_open(gate);
+    const int64_t m = ordered ? *total : n;
     if (blockIdx.x * (int64_t)(BLOCK * APT) >= m) return;   // uniform across the block
 #pragma unroll
-    for (int q = 0; q < APT; ++q) pi[q] = i0 + q >= m ? n : (idx ? idx[i0 + q] : i0 + q);
+    for (int q = 0; q < APT; ++q) pi[q] = i0 + q >= m ? n : (ordered ? idx[i0 + q] : i0 + q);
     int lo[3] = {1 << 30, 1 << 30, 1 << 30}, hi[3] = {-(1 << 30), -(1 << 30), -(1 << 30)};
     int sm[3] = {0, 0, 0}, cnt = 0;
 #pragma unroll
@@ -632,19 +685,24 @@ int check_adj(lepic_ctx *ctx, const lepic_pset *p, const lepic_adjoint_set *a, c
 
 namespace {
 
-// The particles in the order of their cells (idx, null: as they stand).  The
+// The particles in the order of their cells (idx null: as they stand).  The
 // slots keep the order of the last sort, so a fast species' blocks spread over
 // more nodes than the box holds and most of their runs become 24 global atomics:
-// 2.1M electrons on 64^3 take 240 us sorted and 1650 after 10 steps.  Ordered by
-// cell anew they take 625 and the order 85, and the sorted ions 55 more than
-// before; a run of 20 steps 141.7 -> 125.7 ms.  From ORDER_MIN particles: the
-// launches cost a run of 48^3 x 10 (1.1M) -3 %, of 32^3 x 6 (0.2M) +0.6 %.
+// 2.1M electrons on 64^3 take 240 us sorted, 1040 after one step and 1640 after 5;
+// ordered anew 400 and 580 with the order (50); a run of 20 steps 141.7 -> 125.7
+// ms.  k_adj_probe decides whether the order is formed.  From ORDER_MIN particles:
+// the launches cost a run of 48^3 x 10 (1.1M) -3 %, of 32^3 x 6 (0.2M) +0.6 %.
 constexpr int64_t ORDER_MIN = (int64_t)1 << 19;
+static_assert(ORDER_MIN >= (int64_t)BLOCK * APT * ORDER_SAMPLES, "a block per sample");
+
+struct AdjOrder {
+  const int32_t *idx = nullptr;
+  const int64_t *total = nullptr;
+  const int32_t *gate = nullptr;
+};
 
 int adj_order(lepic_ctx *ctx, const lepic_grid *g, const KGrid &kg, const lepic_pset *state,
-              const int32_t **idx, const int64_t **total) {
-  *idx = nullptr;
-  *total = nullptr;
+              AdjOrder &a) {
   const int64_t n = state->n;
   const int32_t dims[3] = {g->n[0] + 2, g->n[1] + 2, g->n[2] + 2};
   if (n < ORDER_MIN || n >= ((int64_t)1 << 31) - 4096) return LEPIC_OK;
@@ -655,13 +713,18 @@ int adj_order(lepic_ctx *ctx, const lepic_grid *g, const KGrid &kg, const lepic_
   if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
   if (capture != hipStreamCaptureStatusNone) return LEPIC_OK;
   CellOrder o;
-  if (!lepic_order_alloc(ctx, dims, n, n, o)) return LEPIC_OK;
-  int st;
-  hipLaunchKernelGGL(k_adj_cells, dim3(grid_blocks(n, BLOCK)), dim3(BLOCK), 0, ctx->stream, kg,
-                     *state, n, o.extra);
-  if ((st = lepic_order_run(ctx, dims, o.extra, n, o))) return st;
-  *idx = o.idx;
-  *total = o.total;
+  if (!lepic_order_alloc(ctx, dims, n, n + ORDER_SAMPLES, o)) return LEPIC_OK;
+  const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
+  int32_t *gate = o.extra, *cell = o.extra + ORDER_SAMPLES;
+  o.gate = gate;
+  hipLaunchKernelGGL(k_adj_probe,
+                     dim3(std::max<unsigned>(grid_blocks(ncells, BLOCK), ORDER_SAMPLES)),
+                     dim3(BLOCK), 0, ctx->stream, kg, *state, n, o.count, ncells, gate);
+  const int st = lepic_order_run_set(ctx, g, state, cell, o);
+  if (st) return st;
+  a.idx = o.idx;
+  a.total = o.total;
+  a.gate = o.gate;
   return LEPIC_OK;
 }
 
@@ -696,13 +759,12 @@ int lepic_adj_push(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset *state,
   double *rep = lepic_replicas(ctx, 4 * nodes);
   if (!rep) return lepic_fail(ctx, LEPIC_ERR_HIP, "adj_push: replicas");
   const KGrid kg = make_kgrid(g);
-  const int32_t *idx;
-  const int64_t *total;
-  if ((st = adj_order(ctx, g, kg, state, &idx, &total))) return st;
+  AdjOrder o;
+  if ((st = adj_order(ctx, g, kg, state, o))) return st;
   hipLaunchKernelGGL(k_adj_push<false>, dim3(grid_blocks(n, BLOCK * APT)), dim3(BLOCK), 0,
                      ctx->stream, kg, *state, kadj(adj), n,
-                     reinterpret_cast<const double4 *>(E4), bf, k1, dt, rep, nodes, lamB, idx,
-                     total);
+                     reinterpret_cast<const double4 *>(E4), bf, k1, dt, rep, nodes, lamB,
+                     o.idx, o.total, o.gate);
   LEPIC_LAUNCH_CHECK(ctx, "k_adj_push");
   hipLaunchKernelGGL(k_adj_rep_flush, dim3(grid_blocks(4 * nodes, 256)), dim3(256), 0,
                      ctx->stream, lamE4, rep, 4 * nodes);
@@ -731,13 +793,12 @@ int lepic_adj_push_map(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset *st
   double *rep = lepic_replicas(ctx, 4 * nodes);
   if (!rep) return lepic_fail(ctx, LEPIC_ERR_HIP, "adj_push_map: replicas");
   const KGrid kg = make_kgrid(g);
-  const int32_t *idx;
-  const int64_t *total;
-  if ((st = adj_order(ctx, g, kg, state, &idx, &total))) return st;
+  AdjOrder o;
+  if ((st = adj_order(ctx, g, kg, state, o))) return st;
   hipLaunchKernelGGL(k_adj_push<true>, dim3(grid_blocks(n, BLOCK * APT)), dim3(BLOCK), 0,
                      ctx->stream, kg, *state, kadj(adj), n,
                      reinterpret_cast<const double4 *>(E4), bf, k1, dt, rep, nodes, nullptr,
-                     idx, total);
+                     o.idx, o.total, o.gate);
   LEPIC_LAUNCH_CHECK(ctx, "k_adj_push_map");
   hipLaunchKernelGGL(k_adj_rep_flush, dim3(grid_blocks(4 * nodes, 256)), dim3(256), 0,
                      ctx->stream, lamE4, rep, 4 * nodes);

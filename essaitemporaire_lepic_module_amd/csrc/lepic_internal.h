@@ -102,12 +102,18 @@ void *lepic_scratch(lepic_ctx *ctx, size_t bytes, int which);
 struct CellOrder {
   int32_t *count, *start, *cursor, *bsum, *idx;
   int32_t *extra;    // the words asked for besides
+  const int32_t *gate = nullptr;   // order_open (lepic_partutil.h): the kernels that form it
+                                   // do so only then; count cleared by the caller
   int64_t *total;
 };
 // false: the scratch cannot be had
 bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o);
 int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
                     const CellOrder &o);
+// The same of an FP64 set by its stencils' lower nodes (n + 2 per axis), which go
+// to cell (16-byte aligned).
+int lepic_order_run_set(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset *set, int32_t *cell,
+                        const CellOrder &o);
 // Resolves, once per device, the static scratch lepic_efield_noalloc uses
 // (lepic_fields.hip); the device must be current.
 void lepic_efield_scratch_setup(int device);

@@ -809,12 +809,10 @@ __device__ inline void load_cells(const KG32 &g, const int32_t *cell, int64_t n,
     if (c[q] >= g.ncells) c[q] = -1;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_sort_count(KG32 g, const int32_t *__restrict__ cell,
-                                                      int64_t n, int32_t *count) {
+// A tile's cells added to count.
+__device__ inline void count_cells(const KG32 &g, const int c[CPT], int32_t *count) {
   __shared__ SortShared bs;
-  const int64_t i0 = (int64_t)blockIdx.x * CTILE + (int64_t)threadIdx.x * CPT;
-  int c[CPT], cx[CPT], cy[CPT], cz[CPT];
-  load_cells(g, cell, n, i0, c);
+  int cx[CPT], cy[CPT], cz[CPT];
   int lo[3] = {1 << 30, 1 << 30, 1 << 30}, hi[3] = {-(1 << 30), -(1 << 30), -(1 << 30)};
 #pragma unroll
   for (int q = 0; q < CPT; ++q) {
@@ -842,11 +840,43 @@ __global__ __launch_bounds__(BLOCK) void k_sort_count(KG32 g, const int32_t *__r
   }
 }
 
-// Exclusive scan of count[0..m) into start and cursor, in three launches:
-// per-block sums, one block over the block sums, then every block adds its
-// offset; up to SCAN_ONE cells in one block's launch (each launch is 4 us, the
-// one block's 5 at 4096 cells).  The total goes to *total.
+__global__ __launch_bounds__(BLOCK) void k_sort_count(KG32 g, const int32_t *__restrict__ cell,
+                                                      int64_t n, int32_t *count) {
+  const int64_t i0 = (int64_t)blockIdx.x * CTILE + (int64_t)threadIdx.x * CPT;
+  int c[CPT];
+  load_cells(g, cell, n, i0, c);
+  count_cells(g, c, count);
+}
+
+// The same for an FP64 set, whose cells (the lower node of the stencil, [0, n + 1]
+// per axis; -1 of a hole) it writes on the way.
+__global__ __launch_bounds__(BLOCK) void k_order_count(KG32 g, KGrid fg, lepic_pset st, int64_t n,
+                                                       int32_t *cell, int32_t *count,
+                                                       const int32_t *__restrict__ gate) {
+  if (!order_open(gate)) return;
+  const int64_t i0 = (int64_t)blockIdx.x * CTILE + (int64_t)threadIdx.x * CPT;
+  int c[CPT];
+#pragma unroll
+  for (int q = 0; q < CPT; ++q) {
+    const int64_t i = i0 + q;
+    c[q] = -1;
+    if (i < n && st.dead[i] == 0) {
+      int jx, jy, jz;
+      stencil_lo(fg, st.x[i], st.y[i], st.z[i], jx, jy, jz);
+      c[q] = jx + g.n1 * (jy + g.n2 * jz);
+    }
+    if (i < n) cell[i] = c[q];
+  }
+  count_cells(g, c, count);
+}
+
+// Exclusive scan of count[0..m) into start and cursor: per-block sums, then
+// every block adds the sums of the blocks before it (past SCAN_OWN blocks from a
+// launch of one block between the two); up to SCAN_ONE cells in one block's
+// launch (each launch is 4 us, the one block's 7 at 4096 cells).  The total goes
+// to *total.
 constexpr int SCAN_B = 1024;   // elements per block (4 per thread)
+constexpr int64_t SCAN_OWN = 4096;
 
 __device__ inline int block_excl_scan(int v, int *wsum, int &total) {
   const int lane = __lane_id(), w = threadIdx.x >> 6;
@@ -874,8 +904,10 @@ __device__ inline int block_excl_scan(int v, int *wsum, int &total) {
 }
 
 __global__ __launch_bounds__(BLOCK) void k_scan_sums(const int32_t *count, int64_t m,
-                                                     int32_t *bsum) {
+                                                     int32_t *bsum,
+                                                     const int32_t *__restrict__ gate) {
   __shared__ int wsum[BLOCK / 64 + 1];
+  if (!order_open(gate)) return;
   const int64_t b0 = (int64_t)blockIdx.x * SCAN_B + threadIdx.x * 4;
   int s = 0;
   for (int q = 0; q < 4; ++q)
@@ -885,8 +917,10 @@ __global__ __launch_bounds__(BLOCK) void k_scan_sums(const int32_t *count, int64
   if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_scan_top(int32_t *bsum, int64_t nb, int64_t *total_out) {
+__global__ __launch_bounds__(BLOCK) void k_scan_top(int32_t *bsum, int64_t nb, int64_t *total_out,
+                                                    const int32_t *__restrict__ gate) {
   __shared__ int wsum[BLOCK / 64 + 1];
+  if (!order_open(gate)) return;
   int carry = 0;
   for (int64_t base = 0; base < nb; base += BLOCK) {
     const int64_t i = base + threadIdx.x;
@@ -901,16 +935,26 @@ __global__ __launch_bounds__(BLOCK) void k_scan_top(int32_t *bsum, int64_t nb, i
 
 __global__ __launch_bounds__(BLOCK) void k_scan_apply(const int32_t *count, int64_t m,
                                                       const int32_t *bsum, int32_t *start,
-                                                      int32_t *cursor) {
+                                                      int32_t *cursor, int64_t *total_out,
+                                                      const int32_t *__restrict__ gate) {
   __shared__ int wsum[BLOCK / 64 + 1];
+  if (!order_open(gate)) return;
   const int64_t b0 = (int64_t)blockIdx.x * SCAN_B + threadIdx.x * 4;
   int v[4], s = 0;
   for (int q = 0; q < 4; ++q) {
     v[q] = b0 + q < m ? count[b0 + q] : 0;
     s += v[q];
   }
-  int total;
-  int e = block_excl_scan(s, wsum, total) + bsum[blockIdx.x];
+  int before = 0, total;
+  if (total_out) {
+    int a = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += BLOCK) a += bsum[i];
+    block_excl_scan(a, wsum, before);
+  } else {
+    before = bsum[blockIdx.x];
+  }
+  int e = block_excl_scan(s, wsum, total) + before;
+  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total_out = before + total;
   for (int q = 0; q < 4; ++q) {
     if (b0 + q < m) start[b0 + q] = cursor[b0 + q] = e;
     e += v[q];
@@ -921,8 +965,10 @@ constexpr int SCAN_ONE_B = 1024, SCAN_ONE = 16 * SCAN_ONE_B;
 
 __global__ __launch_bounds__(SCAN_ONE_B) void k_scan_one(const int32_t *__restrict__ count, int m,
                                                          int32_t *start, int32_t *cursor,
-                                                         int64_t *total) {
+                                                         int64_t *total,
+                                                         const int32_t *__restrict__ gate) {
   __shared__ int wsum[SCAN_ONE_B / 64];
+  if (!order_open(gate)) return;
   const int b0 = (int)threadIdx.x * 16, lane = __lane_id(), w = (int)threadIdx.x >> 6;
   int v[16], s = 0;
 #pragma unroll
@@ -948,8 +994,10 @@ __global__ __launch_bounds__(SCAN_ONE_B) void k_scan_one(const int32_t *__restri
 
 // Claim: cursor[c] starts at start[c]; each tile takes one run per cell.
 __global__ __launch_bounds__(BLOCK) void k_sort_claim(KG32 g, const int32_t *__restrict__ cell,
-                                                      int64_t n, int32_t *cursor, int32_t *idx) {
+                                                      int64_t n, int32_t *cursor, int32_t *idx,
+                                                      const int32_t *__restrict__ gate) {
   __shared__ SortShared bs;
+  if (!order_open(gate)) return;
   const int64_t i0 = (int64_t)blockIdx.x * CTILE + (int64_t)threadIdx.x * CPT;
   int c[CPT], cx[CPT], cy[CPT], cz[CPT];
   load_cells(g, cell, n, i0, c);
@@ -1167,33 +1215,59 @@ bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t
   return true;
 }
 
-int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
-                    const CellOrder &o) {
+namespace {
+
+// count is done: the scan and the claim.
+int order_finish(lepic_ctx *ctx, const KG32 &kg, const int32_t *cell, int64_t n,
+                 const CellOrder &o) {
+  const int64_t ncells = kg.ncells, nb = (ncells + SCAN_B - 1) / SCAN_B;
+  const hipStream_t s = ctx->stream;
+  if (ncells <= SCAN_ONE) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_B), 0, s, o.count, (int)ncells, o.start,
+                       o.cursor, o.total, o.gate);
+  } else {
+    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
+                       o.gate);
+    const bool own = nb <= SCAN_OWN;
+    if (!own)
+      hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, o.bsum, nb, o.total, o.gate);
+    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
+                       o.start, o.cursor, own ? o.total : (int64_t *)nullptr, o.gate);
+  }
+  hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell, n,
+                     o.cursor, o.idx, o.gate);
+  LEPIC_LAUNCH_CHECK(ctx, "cell order");
+  return LEPIC_OK;
+}
+
+KG32 cell_grid(const int32_t dims[3]) {
   lepic_grid g;
   for (int d = 0; d < 3; ++d) {
     g.n[d] = dims[d];
     g.h[d] = 1.0;
   }
-  const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
-  const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
-  const KG32 kg = make_kg32(&g, 0.0);
-  const hipStream_t s = ctx->stream;
-  hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks(ncells, 256)), dim3(256), 0, s, o.count, ncells);
-  hipLaunchKernelGGL(k_sort_count, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell,
-                     n, o.count);
-  if (ncells <= SCAN_ONE) {
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_B), 0, s, o.count, (int)ncells, o.start,
-                       o.cursor, o.total);
-  } else {
-    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, o.bsum, nb, o.total);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
-                       o.start, o.cursor);
-  }
-  hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell,
-                     n, o.cursor, o.idx);
-  LEPIC_LAUNCH_CHECK(ctx, "cell order");
-  return LEPIC_OK;
+  return make_kg32(&g, 0.0);
+}
+
+}  // namespace
+
+int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
+                    const CellOrder &o) {
+  const KG32 kg = cell_grid(dims);
+  hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks(kg.ncells, 256)), dim3(256), 0, ctx->stream,
+                     o.count, (int64_t)kg.ncells);
+  hipLaunchKernelGGL(k_sort_count, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, ctx->stream, kg,
+                     cell, n, o.count);
+  return order_finish(ctx, kg, cell, n, o);
+}
+
+int lepic_order_run_set(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset *set, int32_t *cell,
+                        const CellOrder &o) {
+  const int32_t dims[3] = {g->n[0] + 2, g->n[1] + 2, g->n[2] + 2};
+  const KG32 kg = cell_grid(dims);
+  hipLaunchKernelGGL(k_order_count, dim3(grid_blocks(set->n, CTILE)), dim3(BLOCK), 0, ctx->stream,
+                     kg, make_kgrid(g), *set, set->n, cell, o.count, o.gate);
+  return order_finish(ctx, kg, cell, set->n, o);
 }
 
 extern "C" {

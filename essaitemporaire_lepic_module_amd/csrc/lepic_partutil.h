@@ -30,6 +30,15 @@ inline KBC kbc(const lepic_bc_params *b) {
   return k;
 }
 
+// The mover's stencil lower node (make_stencil): ix = int(x/h) + 1 clamped
+// to [0, n + 1] per axis.
+__device__ inline void stencil_lo(const KGrid &g, double xp, double yp, double zp, int &ix,
+                                  int &iy, int &iz) {
+  ix = imax(0, imin(g.n1 + 1, (int)qdiv(xp, g.q1) + 1));
+  iy = imax(0, imin(g.n2 + 1, (int)qdiv(yp, g.q2) + 1));
+  iz = imax(0, imin(g.n3 + 1, (int)qdiv(zp, g.q3) + 1));
+}
+
 // Reductions of a full wave by DPP row operations (row_shr:1, 2, 4, 8, then
 // row_bcast:15 and :31, the result in lane 63, handed to every lane): register
 // moves instead of six shuffles through LDS.  A lane without a source takes
@@ -48,6 +57,14 @@ LEPIC_WAVE_REDUCE(wave_min, v, min(v, o))
 LEPIC_WAVE_REDUCE(wave_max, v, max(v, o))
 LEPIC_WAVE_REDUCE(wave_sum_i, 0, v + o)
 #undef LEPIC_WAVE_REDUCE
+
+// Whether an order of particles is worth forming: the sum of ORDER_SAMPLES words,
+// each a sample's vote.  No words: it is.  Called by full waves.
+constexpr int ORDER_SAMPLES = 64;
+__device__ inline bool order_open(const int32_t *gate) {
+  static_assert(ORDER_SAMPLES == LEPIC_WAVE, "a word per lane");
+  return !gate || wave_sum_i(gate[__lane_id()]) > 0;
+}
 
 __device__ inline double wave_sum_d(double v) {
   for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
