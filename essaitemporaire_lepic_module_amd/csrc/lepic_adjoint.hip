@@ -713,7 +713,7 @@ int adj_order(lepic_ctx *ctx, const lepic_grid *g, const KGrid &kg, const lepic_
   if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
   if (capture != hipStreamCaptureStatusNone) return LEPIC_OK;
   CellOrder o;
-  if (!lepic_order_alloc(ctx, dims, n, n + ORDER_SAMPLES, o)) return LEPIC_OK;
+  if (!lepic_order_alloc(ctx, dims, n, n + ORDER_SAMPLES, 0, o)) return LEPIC_OK;
   const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
   int32_t *gate = o.extra, *cell = o.extra + ORDER_SAMPLES;
   o.gate = gate;

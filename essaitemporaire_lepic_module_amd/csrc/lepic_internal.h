@@ -105,9 +105,12 @@ struct CellOrder {
   const int32_t *gate = nullptr;   // order_open (lepic_partutil.h): the kernels that form it
                                    // do so only then; count cleared by the caller
   int64_t *total;
+  int32_t big = 0;                 // > 0: the cells of more go to list, *nlist of them
+  int32_t *list, *nlist;           // (n / big at most)
 };
 // false: the scratch cannot be had
-bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o);
+bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra,
+                       int32_t big, CellOrder &o);
 int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
                     const CellOrder &o);
 // The same of an FP64 set by its stencils' lower nodes (n + 2 per axis), which go

@@ -933,9 +933,28 @@ __global__ __launch_bounds__(BLOCK) void k_scan_top(int32_t *bsum, int64_t nb, i
   if (threadIdx.x == 0) *total_out = carry;
 }
 
+// The list of the cells of more than big particles (big 0: none).
+struct BigCells {
+  int big;
+  int32_t *list, *n;
+};
+
+// Cell c of v particles, one atomic per wave.  Called by full waves.
+__device__ inline void list_big(const BigCells &l, int64_t c, int v) {
+  if (l.big == 0) return;
+  const bool mine = v > l.big;
+  const unsigned long long m = __ballot(mine);
+  if (m == 0) return;
+  int at = 0;
+  if (__lane_id() == 0) at = atomicAdd(l.n, (int)__popcll(m));
+  at = __builtin_amdgcn_readfirstlane(at) + (int)__popcll(m & ((1ull << __lane_id()) - 1));
+  if (mine) l.list[at] = (int32_t)c;
+}
+
 __global__ __launch_bounds__(BLOCK) void k_scan_apply(const int32_t *count, int64_t m,
                                                       const int32_t *bsum, int32_t *start,
                                                       int32_t *cursor, int64_t *total_out,
+                                                      BigCells big,
                                                       const int32_t *__restrict__ gate) {
   __shared__ int wsum[BLOCK / 64 + 1];
   if (!order_open(gate)) return;
@@ -956,6 +975,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_apply(const int32_t *count, int6
   int e = block_excl_scan(s, wsum, total) + before;
   if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total_out = before + total;
   for (int q = 0; q < 4; ++q) {
+    list_big(big, b0 + q, v[q]);
     if (b0 + q < m) start[b0 + q] = cursor[b0 + q] = e;
     e += v[q];
   }
@@ -965,7 +985,7 @@ constexpr int SCAN_ONE_B = 1024, SCAN_ONE = 16 * SCAN_ONE_B;
 
 __global__ __launch_bounds__(SCAN_ONE_B) void k_scan_one(const int32_t *__restrict__ count, int m,
                                                          int32_t *start, int32_t *cursor,
-                                                         int64_t *total,
+                                                         int64_t *total, BigCells big,
                                                          const int32_t *__restrict__ gate) {
   __shared__ int wsum[SCAN_ONE_B / 64];
   if (!order_open(gate)) return;
@@ -986,6 +1006,7 @@ __global__ __launch_bounds__(SCAN_ONE_B) void k_scan_one(const int32_t *__restri
   for (int i = 0; i < w; ++i) e += wsum[i];
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
+    list_big(big, b0 + q, v[q]);
     if (b0 + q < m) start[b0 + q] = cursor[b0 + q] = e;
     e += v[q];
   }
@@ -1040,8 +1061,9 @@ __global__ __launch_bounds__(BLOCK) void k_sort_claim(KG32 g, const int32_t *__r
 // Place: W lanes per cell sort its source indices ascending (they are
 // distinct) in registers, bitonic over the cell padded to W x R entries
 // (position q*W + ln in register q: partners W or more apart in the same
-// lane, nearer ones across lanes), and copy the particles; cells beyond 4 W:
-// each index's rank counted over the cell.
+// lane, nearer ones across lanes), and copy the particles.  The cells beyond 4 W
+// come from a list that the scan made, one wave to each (beyond 256: each index's
+// rank counted over the cell), in the first `extra` blocks.
 //
 // A cell's particles come from the lines of all cells around it, so the copy
 // is bound by how often a source line is fetched.  Slot order, blocks in turn
@@ -1104,16 +1126,46 @@ __device__ inline void place_cell(const KP32 &src, const KP32 &dst, const int32_
     if (q * W + ln < s) place_one(src, dst, c, b + q * W + ln, v[q]);
 }
 
+__device__ inline void place_big(const KP32 &src, const KP32 &dst, const int32_t *__restrict__ idx,
+                                 int c, int64_t b, int s, int ln) {
+  if (s <= 64) {
+    place_cell<64, 1>(src, dst, idx, c, b, s, ln);
+  } else if (s <= 128) {
+    place_cell<64, 2>(src, dst, idx, c, b, s, ln);
+  } else if (s <= 256) {
+    place_cell<64, 4>(src, dst, idx, c, b, s, ln);
+  } else {
+    for (int e = ln; e < s; e += 64) {
+      const int v = idx[b + e];
+      int r = 0;
+      for (int j = 0; j < s; ++j) r += idx[b + j] < v ? 1 : 0;
+      place_one(src, dst, c, b + r, v);
+    }
+  }
+}
+
 template <int W>
 __global__ __launch_bounds__(BLOCK) void k_sort_place(KG32 g, KP32 src, KP32 dst,
                                                       const int32_t *__restrict__ count,
                                                       const int32_t *__restrict__ start,
                                                       const int32_t *__restrict__ idx, int bricks_x,
-                                                      int bricks_y) {
-  // consecutive bricks on one XCD (the grid is a multiple of LEPIC_XCDS blocks)
+                                                      int bricks_y, int extra,
+                                                      const int32_t *__restrict__ list,
+                                                      const int32_t *__restrict__ nlist) {
+  if ((int)blockIdx.x < extra) {
+    const int n = *nlist, w = (int)threadIdx.x / LEPIC_WAVE;
+    for (int i = (int)blockIdx.x + w * extra; i < n; i += extra * (BLOCK / LEPIC_WAVE)) {
+      const int c = list[i];
+      int ln = __lane_id();
+      asm("" : "+v"(ln));   // the network's lane masks formed here, not kept over the loop
+      place_big(src, dst, idx, c, start[c], count[c], ln);
+    }
+    return;
+  }
+  const int blocks = (int)gridDim.x - extra, block = (int)blockIdx.x - extra;
+  // consecutive bricks on one XCD (blocks is a multiple of LEPIC_XCDS)
   constexpr int CELLS = BLOCK / W, BLOCKS = BRX * BRY * BRZ / CELLS;   // per block, per brick
-  const int t = ((int)blockIdx.x % LEPIC_XCDS) * ((int)gridDim.x / LEPIC_XCDS) +
-                (int)blockIdx.x / LEPIC_XCDS;
+  const int t = (block % LEPIC_XCDS) * (blocks / LEPIC_XCDS) + block / LEPIC_XCDS;
   const int brick = t / BLOCKS, l = (t - brick * BLOCKS) * CELLS + (int)threadIdx.x / W;
   const int br = brick / bricks_x, bz = br / bricks_y;
   const int cx = (brick - br * bricks_x) * BRX + l % BRX,
@@ -1126,19 +1178,14 @@ __global__ __launch_bounds__(BLOCK) void k_sort_place(KG32 g, KP32 src, KP32 dst
     s = count[c];
     b = start[c];
   }
+  if (s > 4 * W) s = 0;   // on the list
+  if (!__any(s > 0)) return;
   if (!__any(s > W)) {
     place_cell<W, 1>(src, dst, idx, c, b, s, ln);
   } else if (!__any(s > 2 * W)) {
     place_cell<W, 2>(src, dst, idx, c, b, s, ln);
-  } else if (!__any(s > 4 * W)) {
-    place_cell<W, 4>(src, dst, idx, c, b, s, ln);
   } else {
-    for (int e = ln; e < s; e += W) {
-      const int v = idx[b + e];
-      int r = 0;
-      for (int j = 0; j < s; ++j) r += idx[b + j] < v ? 1 : 0;
-      place_one(src, dst, c, b + r, v);
-    }
+    place_cell<W, 4>(src, dst, idx, c, b, s, ln);
   }
 }
 
@@ -1199,18 +1246,22 @@ unsigned long long *int_replicas(lepic_ctx *ctx, int64_t nodes) {
 
 // The order of n particles by cell id (count, scan and claim of the sort): ids
 // below 0 are dropped, the order within a cell is the atomics'.
-bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra, CellOrder &o) {
+bool lepic_order_alloc(lepic_ctx *ctx, const int32_t dims[3], int64_t n, int64_t extra,
+                       int32_t big, CellOrder &o) {
   const int64_t ncells = (int64_t)dims[0] * dims[1] * dims[2];
-  const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B;
-  const size_t words = (size_t)(3 * ncells + nb + n + extra + 64);
+  const int64_t nb = (ncells + SCAN_B - 1) / SCAN_B, nlist = big ? n / big + 1 : 0;
+  const size_t words = (size_t)(3 * ncells + nb + nlist + n + extra + 64);
   int32_t *w = reinterpret_cast<int32_t *>(lepic_scratch(ctx, sizeof(int32_t) * words, 0));
   if (!w) return false;
   o.extra = w;                              // 256-byte aligned
   o.count = w + ((extra + 15) & ~(int64_t)15);
-  o.start = o.count + ncells;
+  o.nlist = o.count + ncells;               // cleared with count
+  o.start = o.nlist + 1;
   o.cursor = o.start + ncells;
   o.bsum = o.cursor + ncells;
-  o.idx = o.bsum + nb;
+  o.list = o.bsum + nb;
+  o.idx = o.list + nlist;
+  o.big = big;
   o.total = ctx->d_ctrl + CTRL_COUNT_OUT;
   return true;
 }
@@ -1221,10 +1272,11 @@ namespace {
 int order_finish(lepic_ctx *ctx, const KG32 &kg, const int32_t *cell, int64_t n,
                  const CellOrder &o) {
   const int64_t ncells = kg.ncells, nb = (ncells + SCAN_B - 1) / SCAN_B;
+  const BigCells big{o.big, o.list, o.nlist};
   const hipStream_t s = ctx->stream;
   if (ncells <= SCAN_ONE) {
     hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_B), 0, s, o.count, (int)ncells, o.start,
-                       o.cursor, o.total, o.gate);
+                       o.cursor, o.total, big, o.gate);
   } else {
     hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
                        o.gate);
@@ -1232,7 +1284,7 @@ int order_finish(lepic_ctx *ctx, const KG32 &kg, const int32_t *cell, int64_t n,
     if (!own)
       hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, o.bsum, nb, o.total, o.gate);
     hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(BLOCK), 0, s, o.count, ncells, o.bsum,
-                       o.start, o.cursor, own ? o.total : (int64_t *)nullptr, o.gate);
+                       o.start, o.cursor, own ? o.total : (int64_t *)nullptr, big, o.gate);
   }
   hipLaunchKernelGGL(k_sort_claim, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, s, kg, cell, n,
                      o.cursor, o.idx, o.gate);
@@ -1254,8 +1306,8 @@ KG32 cell_grid(const int32_t dims[3]) {
 int lepic_order_run(lepic_ctx *ctx, const int32_t dims[3], const int32_t *cell, int64_t n,
                     const CellOrder &o) {
   const KG32 kg = cell_grid(dims);
-  hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks(kg.ncells, 256)), dim3(256), 0, ctx->stream,
-                     o.count, (int64_t)kg.ncells);
+  hipLaunchKernelGGL(k_zero_i32, dim3(grid_blocks((int64_t)kg.ncells + 1, 256)), dim3(256), 0, ctx->stream,
+                     o.count, (int64_t)kg.ncells + 1);
   hipLaunchKernelGGL(k_sort_count, dim3(grid_blocks(n, CTILE)), dim3(BLOCK), 0, ctx->stream, kg,
                      cell, n, o.count);
   return order_finish(ctx, kg, cell, n, o);
@@ -1437,23 +1489,32 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
   const int64_t ncells = (int64_t)g->n[0] * g->n[1] * g->n[2];
   const KG32 kg = make_kg32(g, 0.0);
   const hipStream_t s = ctx->stream;
-  CellOrder o;
-  if (!lepic_order_alloc(ctx, g->n, n, 0, o))
-    return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: scratch");
-  if ((st = lepic_order_run(ctx, g->n, src->cell, n, o))) return st;
   // lanes per cell: the mean cell and twice its spread in one entry per lane
   const double mean = (double)n / (double)ncells, wide = mean + 2.0 * std::sqrt(mean);
+  const int lanes = wide <= 8.0 ? 8 : wide <= 16.0 ? 16 : wide <= 32.0 ? 32 : 64;
+  CellOrder o;
+  if (!lepic_order_alloc(ctx, g->n, n, 0, 4 * lanes, o))
+    return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: scratch");
+  if ((st = lepic_order_run(ctx, g->n, src->cell, n, o))) return st;
   const int bx = (g->n[0] + BRX - 1) / BRX, by = (g->n[1] + BRY - 1) / BRY,
             bz = (g->n[2] + BRZ - 1) / BRZ;
-  auto place = [&](auto kernel, int w) {
-    const int64_t blocks = (int64_t)bx * by * bz * (BRX * BRY * BRZ * w / BLOCK);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((blocks + LEPIC_XCDS - 1) / LEPIC_XCDS * LEPIC_XCDS)),
-                       dim3(BLOCK), 0, s, kg, kp32(src), kp32(dst), o.count, o.start, o.idx, bx, by);
+  auto xcds = [](int64_t blocks) {
+    return (unsigned)((blocks + LEPIC_XCDS - 1) / LEPIC_XCDS * LEPIC_XCDS);
   };
-  if (wide <= 8.0) place(k_sort_place<8>, 8);
-  else if (wide <= 16.0) place(k_sort_place<16>, 16);
-  else if (wide <= 32.0) place(k_sort_place<32>, 32);
-  else place(k_sort_place<64>, 64);
+  // a wave per listed cell, up to half of the waves that the chip holds
+  const unsigned extra =
+      xcds(std::min<int64_t>(1024, grid_blocks(n / (4 * lanes + 1), BLOCK / LEPIC_WAVE)));
+  auto place = [&](auto kernel) {
+    const int64_t blocks = (int64_t)bx * by * bz * (BRX * BRY * BRZ * lanes / BLOCK);
+    hipLaunchKernelGGL(kernel, dim3(xcds(blocks) + extra), dim3(BLOCK), 0, s, kg, kp32(src),
+                       kp32(dst), o.count, o.start, o.idx, bx, by, (int)extra, o.list, o.nlist);
+  };
+  switch (lanes) {
+    case 8: place(k_sort_place<8>); break;
+    case 16: place(k_sort_place<16>); break;
+    case 32: place(k_sort_place<32>); break;
+    default: place(k_sort_place<64>); break;
+  }
   LEPIC_LAUNCH_CHECK(ctx, "sort32 passes");
   LEPIC_HIP(ctx, hipMemcpyAsync(ctx->h_pinned, o.total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   LEPIC_HIP(ctx, hipStreamSynchronize(s));

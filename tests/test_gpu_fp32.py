@@ -2,12 +2,14 @@
 restatement (itself pinned against the FP64 phase in test_oracle32.py):
 cells, offsets, velocities, loss counts and the fixed-point density are
 bit-identical; wall diagnostics (FP64 atomics) agree to 1e-12."""
+import ctypes as C
 import math
 
 import numpy as np
 import pytest
 import torch
 
+from essaitemporaire_lepic_module_amd import _native
 from essaitemporaire_lepic_module_amd import config as cfg
 from tests import helpers as H
 
@@ -203,6 +205,80 @@ def test_sort32_place_bitexact(gpu, oracle, rng, n, mean, crowd):
     P32.sort32(g, n, h)
     assert g.n == ref.n
     _same32(g, ref)
+
+
+def _sort_set(P32, gpu, n, cells, seed=3, window=500):
+    """A set whose slots are the given cells' in near order (moved by a few
+    hundred slots, as particles between two sorts)."""
+    r = torch.Generator(device=gpu)
+    r.manual_seed(seed)
+    m = cells.numel()
+    c = cells.sort().values
+    at = torch.arange(m, device=gpu) + window * torch.randn(m, device=gpu, generator=r)
+    c = c[at.sort().indices]
+    p = P32.ParticleSet32(m, gpu)
+    p._buf[0]["cell"][:m].copy_(c)
+    for k in ("fx", "fy", "fz", "vx", "vy", "vz"):
+        p._buf[0][k].uniform_(0, 0.99, generator=r)
+    p.n = m
+    return p
+
+
+def _sort_time(p, n, reps=10):
+    """Best time of the sort from the set's buffer to its other one, ms."""
+    from essaitemporaire_lepic_module_amd.device import context
+    ctx = context(p.device)
+    g = _native.grid(n, (1e-3,) * 3)
+    src, dst = p.pset(), p.pset(other=True)
+    best = 1e9
+    for _ in range(reps):
+        t0, t1 = torch.cuda.Event(True), torch.cuda.Event(True)
+        t0.record()
+        ctx.check(ctx.lib.lepic_sort32(ctx.h, C.byref(g), C.byref(src), C.byref(dst)))
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1))
+    return best, int(dst.n)
+
+
+def _check_sorted(p, m):
+    """The other buffer holds the set's stable order by cell."""
+    b, o = p._buf[p._cur], p._buf[p._cur ^ 1]
+    c = b["cell"][: p.n]
+    live = (c >= 0).nonzero()[:, 0]
+    order = live[c[live].sort(stable=True).indices]
+    assert m == order.numel()
+    for k in b:
+        assert torch.equal(o[k][:m], b[k][order]), k
+
+
+# Cells far above the mean (a beam, a cluster, a local load): more than four
+# entries per lane of the box's mean cell.  Sizes of the list's waves: up to 64
+# entries, 128, 256 and beyond (ranks counted).
+@pytest.mark.parametrize("n,box,per", [((64, 64, 64), (16, 16, 16), 50),
+                                       ((64, 64, 64), (16, 16, 16), 110),
+                                       ((64, 64, 64), (16, 16, 16), 200),
+                                       ((128, 128, 128), (128, 16, 16), 64),
+                                       ((40, 40, 40), (3, 3, 3), 700)])
+def test_sort32_crowded_cells(gpu, n, box, per):
+    """The stable order, and at most 2.5 times the time of as many particles
+    spread over the whole box (measured below 1.1; 6 to 10 times where the
+    lanes of the mean cell took the crowded ones; cells past 256, whose ranks
+    are counted, are checked for their order only)."""
+    from essaitemporaire_lepic_module_amd import particles32 as P32
+    r = torch.Generator(device=gpu)
+    r.manual_seed(17)
+    k = torch.stack([torch.randint(0, b, (box[0] * box[1] * box[2] * per,), device=gpu,
+                                   generator=r) for b in box])
+    cells = (k[0] + n[0] * (k[1] + n[1] * k[2])).int()
+    cells[torch.rand(cells.numel(), device=gpu, generator=r) < 0.02] = -1
+    p = _sort_set(P32, gpu, n, cells)
+    crowded, m = _sort_time(p, n)
+    _check_sorted(p, m)
+    even = torch.randint(0, n[0] * n[1] * n[2], (cells.numel(),), device=gpu, generator=r)
+    spread, _ = _sort_time(_sort_set(P32, gpu, n, even.int()), n)
+    if per <= 256:
+        assert crowded <= 2.5 * spread, (crowded, spread)
 
 
 def test_collisions32_deposit_exact(gpu, oracle, rng):
