@@ -18,6 +18,7 @@
 
 #include "lepic_internal.h"
 #include "lepic_partutil.h"
+#include "lepic_walk.h"
 
 namespace {
 
@@ -34,25 +35,6 @@ struct KP32 {
 inline KP32 kp32(const lepic_pset32 *p) {
   KP32 k{p->cell, p->fx, p->fy, p->fz, p->vx, p->vy, p->vz};
   return k;
-}
-
-// Exact x / d for x, d < 2^32: m = ceil(2^64 / d) (2^64 / d for powers of
-// two), q = high 64 bits of x * m.  x m / 2^64 exceeds x / d by less than
-// x / 2^64 < 2^-32 <= 1/d, so the floor is exact.
-struct UDiv {
-  uint64_t m;
-  uint32_t d;
-};
-
-inline UDiv make_udiv(uint32_t d) {
-  UDiv u;
-  u.d = d;
-  u.m = d <= 1 ? 0 : (~0ull) / d + 1;
-  return u;
-}
-
-__device__ inline uint32_t udiv(uint32_t x, const UDiv &u) {
-  return u.d <= 1 ? x : (uint32_t)__umul64hi((uint64_t)x, u.m);
 }
 
 struct KG32 {
@@ -1069,11 +1051,11 @@ __global__ __launch_bounds__(BLOCK) void k_sort_claim(KG32 g, const int32_t *__r
 // is bound by how often a source line is fetched.  Slot order, blocks in turn
 // over the XCDs, fetches every line 5.5 times (24 GB and 4.3 ms for 134M
 // electrons, besides 0.9 ms for a separate sort of the indices).  Here the
-// cells in flight on an XCD are a brick (16 x 8 x 8: about what its 32 CUs
-// hold at once), whose sources and their neighbours fit its 4 MB L2: fetched 2.4
-// times, 4.1 ms for both (5.3M ions on 93 x 61 x 47: 139 -> 76 us); what is left is
-// the rate of scattered reads a CU keeps in flight.
-constexpr int BRX = 16, BRY = 8, BRZ = 8;
+// cells in flight on an XCD are a brick (BrickPlan), whose sources and their
+// neighbours fit its 4 MB L2: fetched 2.4 times, 4.0 ms for both (5.3M ions on 93
+// x 61 x 47: 139 -> 76 us); what is left is the rate of scattered reads a CU keeps
+// in flight.
+static_assert(BRICK_XCDS == LEPIC_XCDS, "bricks are dealt to the XCDs");
 
 template <int W, int R>
 __device__ inline void cell_bitonic(int v[R], int ln) {
@@ -1145,15 +1127,15 @@ __device__ inline void place_big(const KP32 &src, const KP32 &dst, const int32_t
 }
 
 template <int W>
-__global__ __launch_bounds__(BLOCK) void k_sort_place(KG32 g, KP32 src, KP32 dst,
+__global__ __launch_bounds__(BLOCK, 8) void k_sort_place(BrickPlan plan, KP32 src, KP32 dst,
                                                       const int32_t *__restrict__ count,
                                                       const int32_t *__restrict__ start,
-                                                      const int32_t *__restrict__ idx, int bricks_x,
-                                                      int bricks_y, int extra,
+                                                      const int32_t *__restrict__ idx, int extra,
                                                       const int32_t *__restrict__ list,
                                                       const int32_t *__restrict__ nlist) {
+  const int w = (int)threadIdx.x / LEPIC_WAVE;
   if ((int)blockIdx.x < extra) {
-    const int n = *nlist, w = (int)threadIdx.x / LEPIC_WAVE;
+    const int n = *nlist;
     for (int i = (int)blockIdx.x + w * extra; i < n; i += extra * (BLOCK / LEPIC_WAVE)) {
       const int c = list[i];
       int ln = __lane_id();
@@ -1162,30 +1144,25 @@ __global__ __launch_bounds__(BLOCK) void k_sort_place(KG32 g, KP32 src, KP32 dst
     }
     return;
   }
-  const int blocks = (int)gridDim.x - extra, block = (int)blockIdx.x - extra;
-  // consecutive bricks on one XCD (blocks is a multiple of LEPIC_XCDS)
-  constexpr int CELLS = BLOCK / W, BLOCKS = BRX * BRY * BRZ / CELLS;   // per block, per brick
-  const int t = (block % LEPIC_XCDS) * (blocks / LEPIC_XCDS) + block / LEPIC_XCDS;
-  const int brick = t / BLOCKS, l = (t - brick * BLOCKS) * CELLS + (int)threadIdx.x / W;
-  const int br = brick / bricks_x, bz = br / bricks_y;
-  const int cx = (brick - br * bricks_x) * BRX + l % BRX,
-            cy = (br - bz * bricks_y) * BRY + l / BRX % BRY, cz = bz * BRZ + l / (BRX * BRY);
-  const int ln = (int)threadIdx.x % W;
-  int c = 0, s = 0;
-  int64_t b = 0;
-  if (cx < g.n1 && cy < g.n2 && cz < g.n3) {
-    c = cx + g.n1 * (cy + g.n2 * cz);
-    s = count[c];
-    b = start[c];
-  }
-  if (s > 4 * W) s = 0;   // on the list
-  if (!__any(s > 0)) return;
-  if (!__any(s > W)) {
-    place_cell<W, 1>(src, dst, idx, c, b, s, ln);
-  } else if (!__any(s > 2 * W)) {
-    place_cell<W, 2>(src, dst, idx, c, b, s, ln);
-  } else {
-    place_cell<W, 4>(src, dst, idx, c, b, s, ln);
+  // blocks go to the XCDs in turn (extra is a multiple of their number)
+  const uint32_t block = blockIdx.x - (uint32_t)extra, blocks = gridDim.x - (uint32_t)extra;
+  const uint32_t step = blocks / LEPIC_XCDS * (BLOCK / W);
+  for (uint32_t t = block / LEPIC_XCDS * (BLOCK / W) + threadIdx.x / W;
+       __any(t < plan.tasks); t += step) {
+    int ln = (int)threadIdx.x % W;
+    asm("" : "+v"(ln));
+    const int c = t < plan.tasks ? brick_cell(plan, block % LEPIC_XCDS, t) : -1;
+    int s = c >= 0 ? count[c] : 0;
+    const int64_t b = c >= 0 ? start[c] : 0;
+    if (s > 4 * W) s = 0;   // on the list
+    if (!__any(s > 0)) continue;
+    if (!__any(s > W)) {
+      place_cell<W, 1>(src, dst, idx, c, b, s, ln);
+    } else if (!__any(s > 2 * W)) {
+      place_cell<W, 2>(src, dst, idx, c, b, s, ln);
+    } else {
+      place_cell<W, 4>(src, dst, idx, c, b, s, ln);
+    }
   }
 }
 
@@ -1487,7 +1464,6 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
     return LEPIC_OK;
   }
   const int64_t ncells = (int64_t)g->n[0] * g->n[1] * g->n[2];
-  const KG32 kg = make_kg32(g, 0.0);
   const hipStream_t s = ctx->stream;
   // lanes per cell: the mean cell and twice its spread in one entry per lane
   const double mean = (double)n / (double)ncells, wide = mean + 2.0 * std::sqrt(mean);
@@ -1496,18 +1472,14 @@ int lepic_sort32(lepic_ctx *ctx, const lepic_grid *g, const lepic_pset32 *src, l
   if (!lepic_order_alloc(ctx, g->n, n, 0, 4 * lanes, o))
     return lepic_fail(ctx, LEPIC_ERR_HIP, "sort32: scratch");
   if ((st = lepic_order_run(ctx, g->n, src->cell, n, o))) return st;
-  const int bx = (g->n[0] + BRX - 1) / BRX, by = (g->n[1] + BRY - 1) / BRY,
-            bz = (g->n[2] + BRZ - 1) / BRZ;
-  auto xcds = [](int64_t blocks) {
-    return (unsigned)((blocks + LEPIC_XCDS - 1) / LEPIC_XCDS * LEPIC_XCDS);
-  };
+  const BrickPlan plan = brick_plan(g->n, lanes);
   // a wave per listed cell, up to half of the waves that the chip holds
-  const unsigned extra =
-      xcds(std::min<int64_t>(1024, grid_blocks(n / (4 * lanes + 1), BLOCK / LEPIC_WAVE)));
+  const int64_t big = std::min<int64_t>(1024, grid_blocks(n / (4 * lanes + 1), BLOCK / LEPIC_WAVE));
+  const unsigned extra = (unsigned)((big + LEPIC_XCDS - 1) / LEPIC_XCDS * LEPIC_XCDS);
   auto place = [&](auto kernel) {
-    const int64_t blocks = (int64_t)bx * by * bz * (BRX * BRY * BRZ * lanes / BLOCK);
-    hipLaunchKernelGGL(kernel, dim3(xcds(blocks) + extra), dim3(BLOCK), 0, s, kg, kp32(src),
-                       kp32(dst), o.count, o.start, o.idx, bx, by, (int)extra, o.list, o.nlist);
+    hipLaunchKernelGGL(kernel, dim3(extra + brick_blocks(plan, lanes, BLOCK) * LEPIC_XCDS),
+                       dim3(BLOCK), 0, s, plan, kp32(src), kp32(dst), o.count, o.start, o.idx,
+                       (int)extra, o.list, o.nlist);
   };
   switch (lanes) {
     case 8: place(k_sort_place<8>); break;

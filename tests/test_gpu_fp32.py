@@ -281,6 +281,46 @@ def test_sort32_crowded_cells(gpu, n, box, per):
         assert crowded <= 2.5 * spread, (crowded, spread)
 
 
+# Where the cells lie must not matter to the place pass: a slab of planes (once
+# all on one of the XCDs), a single row along each axis (once bricks that were
+# mostly empty), against the same particles spread over a box of as many cells.
+@pytest.mark.parametrize("n,box,per,even", [((128, 128, 128), (128, 128, 13), 20, (128, 128, 128)),
+                                            ((65536, 1, 1), None, 8, (64, 32, 32)),
+                                            ((1, 65536, 1), None, 8, (64, 32, 32)),
+                                            ((1, 1, 65536), None, 8, (64, 32, 32))])
+def test_sort32_place_is_even(gpu, n, box, per, even):
+    """The stable order, and at most twice the time of the even box (measured 0.7
+    to 1.1; 2.9 and more before)."""
+    from essaitemporaire_lepic_module_amd import particles32 as P32
+    r = torch.Generator(device=gpu)
+    r.manual_seed(5)
+    box = box or n
+    k = torch.stack([torch.randint(0, b, (box[0] * box[1] * box[2] * per,), device=gpu,
+                                   generator=r) for b in box])
+    p = _sort_set(P32, gpu, n, (k[0] + n[0] * (k[1] + n[1] * k[2])).int())
+    here, m = _sort_time(p, n)
+    _check_sorted(p, m)
+    c = torch.randint(0, even[0] * even[1] * even[2], (p.n,), device=gpu, generator=r)
+    there, _ = _sort_time(_sort_set(P32, gpu, even, c.int()), even)
+    assert here <= 2.0 * there, (here, there)
+
+
+@pytest.mark.parametrize("n,count", [((4096, 4096, 3), 900001), ((1, 4099, 1021), 3000007),
+                                     ((17, 9, 9), 30001), ((65, 17, 9), 70001)])
+def test_sort32_wide_grids(gpu, n, count):
+    """The stable order on grids past the place pass's most blocks (50M cells: its
+    waves stride over the bricks) and one cell past a brick."""
+    from essaitemporaire_lepic_module_amd import particles32 as P32
+    r = torch.Generator(device=gpu)
+    r.manual_seed(6)
+    cells = torch.randint(0, n[0] * n[1] * n[2], (count,), device=gpu, generator=r).int()
+    cells[:3] = n[0] * n[1] * n[2] - 1
+    cells[torch.rand(count, device=gpu, generator=r) < 0.02] = -1
+    p = _sort_set(P32, gpu, n, cells, window=5000)
+    _, m = _sort_time(p, n, reps=2)
+    _check_sorted(p, m)
+
+
 def test_collisions32_deposit_exact(gpu, oracle, rng):
     """MCC on FP32 sets (cfg2's argon chemistry): products and kills adjust
     the fixed-point density exactly -- afterwards it equals a fresh deposit

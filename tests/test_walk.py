@@ -1,6 +1,8 @@
-"""The node walks of the bounded launches (lepic_walk.h), compiled for the
-host: every node once and, for levels of up to 2^31 - 1 nodes, no step that
-wraps (a 32-bit counter wraps within 262144 nodes of that bound)."""
+"""The walks of the bounded launches (lepic_walk.h), compiled for the host: every
+node once and, for levels of up to 2^31 - 1 nodes, no step that wraps (a 32-bit
+counter wraps within 262144 nodes of that bound); every cell of the sort's bricks
+once, at most 2^32 threads a launch however thin the grid, and slabs and rods of
+cells spread over the XCDs to 1.6 of their mean."""
 import os
 import subprocess
 

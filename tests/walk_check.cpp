@@ -1,9 +1,95 @@
-// lepic_walk.h: every node once, none outside, up to the most nodes of a solve.
+// lepic_walk.h: every node and every cell once, none outside, up to the largest
+// grids; launches within what HIP takes; localised sets spread over the XCDs.
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <vector>
 
 #include "../essaitemporaire_lepic_module_amd/csrc/lepic_walk.h"
+
+namespace {
+
+const int LANES[4] = {8, 16, 32, 64};
+
+// Every cell once; the most an XCD has of the cells that fill() takes, over the mean.
+double spread(const int32_t n[3], int lanes, const std::function<bool(int, int, int)> &fill,
+              long &bad) {
+  const BrickPlan b = brick_plan(n, lanes);
+  std::vector<unsigned char> seen((size_t)n[0] * n[1] * n[2], 0);
+  long load[BRICK_XCDS] = {}, total = 0;
+  for (uint32_t x = 0; x < BRICK_XCDS; ++x)
+    for (uint32_t t = 0; t < b.tasks; ++t) {
+      const int c = brick_cell(b, x, t);
+      if (c < 0) continue;
+      if (c >= (int)seen.size() || seen[c]++) {
+        ++bad;
+        continue;
+      }
+      if (fill(c % n[0], c / n[0] % n[1], c / (n[0] * n[1]))) ++load[x], ++total;
+    }
+  for (unsigned char v : seen) bad += v != 1;
+  return (double)*std::max_element(load, load + BRICK_XCDS) * BRICK_XCDS / (double)total;
+}
+
+long check_bricks() {
+  long bad = 0;
+  const int32_t grids[][3] = {{1, 1, 1},    {1, 1, 40},  {40, 1, 1},   {1, 40, 1},  {17, 9, 9},
+                              {16, 8, 8},   {33, 17, 9}, {65, 64, 63}, {5, 3, 200}, {129, 7, 2},
+                              {300, 300, 1}, {1, 257, 255}, {31, 2, 77}};
+  const auto all = [](int, int, int) { return true; };
+  for (const auto &n : grids)
+    for (int lanes : LANES) {
+      const double most = spread(n, lanes, all, bad);
+      // a grid one cell past a brick: no XCD holds most of it
+      if ((int64_t)n[0] * n[1] * n[2] >= 1000 && most > 1.5) {
+        std::printf("%d %d %d lanes %d: %.2f\n", n[0], n[1], n[2], lanes, most);
+        ++bad;
+      }
+    }
+  const int32_t cube[3] = {128, 128, 128};
+  const std::function<bool(int, int, int)> sets[] = {
+      [](int x, int, int) { return x < 13; }, [](int, int y, int) { return y < 13; },
+      [](int, int, int z) { return z < 13; }, [](int, int, int z) { return z >= 100; },
+      [](int x, int y, int) { return (x - 64) * (x - 64) + (y - 64) * (y - 64) < 900; },
+      [](int x, int y, int z) { return x < 64 && y < 64 && z < 64; }};
+  for (const auto &f : sets)
+    for (int lanes : LANES) {
+      const double most = spread(cube, lanes, f, bad);
+      if (most > 1.6) {
+        std::printf("set %d lanes %d: %.2f\n", (int)(&f - sets), lanes, most);
+        ++bad;
+      }
+    }
+  // launches: fewer than 2^32 threads with the listed cells' blocks (1024 at most),
+  // on the widest grids (2^31 nodes with their ghosts)
+  const int32_t wide[][3] = {{4096, 4096, 1},   {1, 4096, 4096},  {4096, 1, 4096},
+                             {134217000, 1, 1}, {1, 1, 134217000}, {23160, 23160, 1},
+                             {1, 23160, 23160}, {1287, 1287, 1287}, {2, 20724, 20724}};
+  for (const auto &n : wide)
+    for (int lanes : LANES) {
+      const BrickPlan b = brick_plan(n, lanes);
+      const uint64_t threads = ((uint64_t)brick_blocks(b, lanes, 256) * BRICK_XCDS + 1024) * 256;
+      const uint64_t cells = (uint64_t)n[0] * n[1] * n[2];
+      const uint64_t tasks = (uint64_t)((b.bricks + 7) / 8) * b.cells;
+      // a thread's last step past the tasks stays in 32 bits
+      if (threads >= 1ull << 32 || tasks != b.tasks || tasks * 8 < cells ||
+          tasks * 8 > cells + cells / 3 + 64 * 4096 || tasks + threads / 64 >= 1ull << 32) {
+        std::printf("%d %d %d lanes %d: threads %llu tasks %llu\n", n[0], n[1], n[2], lanes,
+                    (unsigned long long)threads, (unsigned long long)tasks);
+        ++bad;
+      }
+      // the last tasks decode to cells of the grid
+      for (uint32_t x = 0; x < BRICK_XCDS; ++x)
+        for (uint32_t t = b.tasks - 1; t + 300 > b.tasks && t < b.tasks; --t) {
+          const int c = brick_cell(b, x, t);
+          bad += c < -1 || (c >= 0 && (uint64_t)c >= cells);
+        }
+    }
+  return bad;
+}
+
+}  // namespace
 
 int main() {
   const int threads = 256, groups = 8;
@@ -47,6 +133,7 @@ int main() {
       bad += visits != nodes;
     }
   }
+  bad += check_bricks();
   std::printf("bad %ld\n", bad);
   return bad != 0;
 }
