@@ -1136,19 +1136,17 @@ __global__ __launch_bounds__(BLOCK) void k_restrict(KLevelT<T> F, KLevelT<T> C, 
 }
 
 // The restriction without periodic walls: a block takes RCX x RCY x RCZ coarse
-// nodes (one per thread), forms getres (mg.f90:809-848) of the fine nodes they
+// nodes (one per thread; 16 x 4 x 4, on narrow grids 4 x 8 x 8), forms getres (mg.f90:809-848) of the fine nodes they
 // read in LDS, 0 where the reference takes none, and sums the 27 values there.
 // The residual goes to memory and back otherwise, and 27 labels are waited for
 // before the values they admit: 16 + 15 us at 128^3, 11 + 5 at 32^3 (FP64), 87
 // + 78 at 256^3 (FP32); this launch 20, 6.5 and 90.  The wrap of j = 1 (labels
 // <= 0 there) takes the general routine.  fin != nullptr: one more block, the
 // last, closes the sor_rb before it (slots_finish).
-constexpr int RCX = 16, RCY = 4, RCZ = 4;
-static_assert(RCX * RCY * RCZ == BLOCK, "a thread per coarse node");
-
-template <class T>
+template <class T, int RCX, int RCY, int RCZ>
 __global__ __launch_bounds__(BLOCK) void k_restrict_tile(KLevelT<T> F, KLevelT<T> C, int flag_nmn,
                                                          int ntx, int nty, SlotCtl sc, MGCtl *fin) {
+  static_assert(RCX * RCY * RCZ == BLOCK, "a thread per coarse node");
   constexpr int FX = 2 * RCX + 1, FY = 2 * RCY + 1, FZ = 2 * RCZ + 1;
   constexpr int UN = sizeof(T) == 8 ? 11 : 4;   // nodes of a thread read before the first wait
   __shared__ T R[FX * FY * FZ];
@@ -1773,6 +1771,29 @@ inline SweepGrid sweep_grid(const KGrid &g) {
   return w;
 }
 
+// Blocks of a restriction whose tiles are x x y x z coarse nodes.
+struct RestrictGrid {
+  int nx, ny, nz;
+  RestrictGrid(const KGrid &g, int x, int y, int z)
+      : nx((g.n1 / 2 + x) / x), ny((g.n2 / 2 + y) / y), nz((g.n3 / 2 + z) / z) {}
+  unsigned blocks() const { return (unsigned)nx * (unsigned)ny * (unsigned)nz; }
+};
+
+// Whether a level sweeps in whole-sweep launches.  A flat or narrow grid leaves
+// most of a large tile empty, which costs as much as a full one: unless the grid
+// fills 0.42 of them (0.27 up to two tiles per CU), one launch per colour is as
+// fast or faster.  Solves with tiles / per colour (FP64, and CG with the FP64
+// preconditioner, ms): 8 x 1024 x 1024 (0.26 filled) 17.8 / 11.7 and 10.0 / 7.9, 12 x
+// 1024 x 1024 (0.39) 18.8 / 15.3 and 11.5 / 10.3, 12 x 512 x 512 (0.37) 5.2 / 5.6 and
+// 3.5 / 3.4, 16 x 512 x 512 (0.49) 5.7 / 6.8 and 3.6 / 4.0, 512 x 512 x 4 (0.28, 496
+// tiles) 1.6 / 2.0 and 1.2 / 1.3.  The small tiles' levels are launch-bound: always.
+inline bool sweeps_tiled(const KGrid &g) {
+  const SweepGrid w = sweep_grid(g);
+  const double filled = (double)(g.n1 + 1) * (g.n2 + 1) * (g.n3 + 1) /
+                        ((double)w.blocks() * (BIG_X * BIG_Y * BIG_Z));
+  return !w.big || filled >= (w.blocks() <= 512 ? 0.27 : 0.42);
+}
+
 template <class T>
 struct Solver {
   lepic_ctx *ctx;
@@ -2001,10 +2022,16 @@ struct Solver {
       if (l + 1 < lc && !(l + 1 < ng - 1 && u2[l + 1]))
         hipLaunchKernelGGL(k_fill_d<T>, dim3(grid_blocks(nc, BLOCK)), dim3(BLOCK), 0, ctx->stream,
                            C.u, nc, T(0));
-      const int nx = (g.n1 / 2 + RCX) / RCX, ny = (g.n2 / 2 + RCY) / RCY,
-                nz = (g.n3 / 2 + RCZ) / RCZ;
-      hipLaunchKernelGGL(k_restrict_tile<T>, dim3((unsigned)nx * ny * nz + (fin ? 1 : 0)),
-                         dim3(BLOCK), 0, ctx->stream, F, C, flag_nmn, nx, ny, fin_sc, fin);
+      // 42 us against 22 at 8 x 32768 x 8 (FP64), where the first fills a fifth of its tiles
+      auto launch = [&](auto kernel, const RestrictGrid &r) {
+        hipLaunchKernelGGL(kernel, dim3(r.blocks() + (fin ? 1 : 0)), dim3(BLOCK), 0, ctx->stream, F,
+                           C, flag_nmn, r.nx, r.ny, fin_sc, fin);
+      };
+      const RestrictGrid wide(g, 16, 4, 4), narrow(g, 4, 8, 8);
+      if (2 * (int64_t)wide.blocks() < 3 * (int64_t)narrow.blocks())
+        launch(k_restrict_tile<T, 16, 4, 4>, wide);
+      else
+        launch(k_restrict_tile<T, 4, 8, 8>, narrow);
       fin = nullptr;
       return;
     }
@@ -2025,6 +2052,20 @@ struct Solver {
     hipLaunchKernelGGL(k_prolong<T>, dim3(grid_blocks(nt, BLOCK) + (fin ? 1 : 0)), dim3(BLOCK), 0, ctx->stream,
                        L[l], L[l + 1], fin_sc, fin);
     fin = nullptr;
+  }
+
+  // The levels with a second u array, its nodes in all, and its places from at on.
+  bool has_u2(int l) const { return ng > 1 && (flag_pbc || sweeps_tiled(L[l].g)); }
+  int64_t u2_nodes() const {
+    int64_t n = 0;
+    for (int l = 0; l < ng; ++l) n += has_u2(l) ? grid_nodes_k(L[l].g) : 0;
+    return n;
+  }
+  void place_u2(T *at) {
+    for (int l = 0; l < ng; ++l) {
+      u2[l] = has_u2(l) ? at : nullptr;
+      at += has_u2(l) ? grid_nodes_k(L[l].g) : 0;
+    }
   }
 
   static int64_t grid_nodes_k(const KGrid &g) {
@@ -2146,7 +2187,7 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
   const int64_t fine_nodes = ng > 1 && mp->flag_pbc ? grid_nodes(g) : 0;   // the restriction's residual
   // the sweeps' second u arrays, block residuals and slot states
-  const int64_t u2_nodes = ng > 1 ? grid_nodes(g) + coarse_nodes : 0;
+  const int64_t u2_nodes = S.u2_nodes();
   int64_t sweep_parts = 0;
   for (int l = 0; l < ng; ++l)
     sweep_parts = std::max<int64_t>(sweep_parts, sweep_grid(S.L[l].g).blocks());
@@ -2191,10 +2232,7 @@ extern "C" int lepic_poisson_solve(lepic_ctx *ctx, const lepic_grid *g, double *
     S.L[l].bc = lb;
     lb += nn;
   }
-  for (int l = 0; l < ng && u2_nodes; ++l) {
-    S.u2[l] = u2;
-    u2 += Solver<double>::grid_nodes_k(S.L[l].g);
-  }
+  S.place_u2(u2);
   S.ctl = reinterpret_cast<MGCtl *>(ctx->d_ctrl + CTRL_MG);
   hipLaunchKernelGGL(k_reset_totals, dim3(1), dim3(64), 0, ctx->stream, S.ctl, MAX_LEVELS);
 
@@ -2319,8 +2357,12 @@ constexpr int MIX_BLOCKS = 1024;
 // A thread's nodes in k_mix_resid and k_pcg_dir: each XCD (blocks go to them in
 // turn) walks its own eighth of the nodes in order, so that the planes above and
 // below are still in its L2: CG direction at 256^3 221 -> 181 us.  (k_pcg_resid
-// writes more than it reads and is 4 % faster striding over all blocks.)
-__device__ inline NodeWalk node_walk(int64_t nodes) {
+// writes more than it reads and is 4 % faster striding over all blocks.)  On fewer
+// than 16 planes an XCD has one or two, and the outermost little plasma in its:
+// striding, 33 us against 42 at 8 x 32768 x 8.
+__device__ inline NodeWalk node_walk(const KGrid &g, int64_t nodes) {
+  if (g.n3 + 3 < 16)
+    return walk_strided(nodes, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, BLOCK);
   return walk_grouped(nodes, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, BLOCK, LEPIC_XCDS);
 }
 
@@ -2333,7 +2375,7 @@ __global__ __launch_bounds__(BLOCK) void k_mix_resid(KLevel L, float *r32, float
   __shared__ double red[BLOCK / LEPIC_WAVE];
   const KGrid &g = L.g;
   double a = 0.0;
-  const NodeWalk nw = node_walk(nodes);
+  const NodeWalk nw = node_walk(g, nodes);
   for (int64_t t = nw.t; t < nw.end; t += nw.step) {
     const int i = (int)(t % g.sy);
     const int64_t q = t / g.sy;
@@ -2459,7 +2501,7 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   const int64_t nodes = grid_nodes(g);
   const int64_t rp_len = ((int64_t)g->n[0] + 2) * ((int64_t)g->n[1] + 2);
   // the sweeps' second u arrays
-  const int64_t u2_nodes = ng > 1 ? nodes + coarse_nodes : 0;
+  const int64_t u2_nodes = S.u2_nodes();
   const int64_t res_nodes = ng > 1 && mp->flag_pbc ? nodes : 0;   // the restriction's residual
   const size_t need = sizeof(double) * (size_t)(MIX_COLS * MIX_BLOCKS + 8) +
                       sizeof(double) * (size_t)nf64 * (size_t)nodes +
@@ -2492,10 +2534,7 @@ int mix_setup(lepic_ctx *ctx, const lepic_grid *g, double *phi, const double *rh
   S.resbuf = res_nodes ? lv + 2 * coarse_nodes : nullptr;
   T *u2 = lv + 2 * coarse_nodes + res_nodes;
   int32_t *lb = reinterpret_cast<int32_t *>(u2 + u2_nodes);
-  for (int l = 0; l < ng && u2_nodes; ++l) {
-    S.u2[l] = u2;
-    u2 += Solver<T>::grid_nodes_k(S.L[l].g);
-  }
+  S.place_u2(u2);
   S.L[0].u = M.e32;
   S.L[0].b = M.r32;
   S.L[0].bc = const_cast<int32_t *>(bcnd);
@@ -2740,7 +2779,7 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_dir(KLevel L, const T *e32, const
   const KGrid &g = L.g;
   const double beta = scal[2] != 0.0 ? scal[1] / scal[2] : 0.0;
   double apq = 0.0, apr = 0.0;
-  const NodeWalk nw = node_walk(nodes);
+  const NodeWalk nw = node_walk(g, nodes);
   for (int64_t t = nw.t; t < nw.end; t += nw.step) {
     double pn = 0.0, qv = 0.0;
     if (L.bc[t] == -1) {

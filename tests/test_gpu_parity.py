@@ -292,6 +292,67 @@ def test_poisson_tiles_bitexact(gpu, oracle, rng, n, ng, nmn):
         np.testing.assert_allclose(info_g["res"], info_o["res"], rtol=1e-9)
 
 
+# Narrow and flat grids: levels that leave most of the large tiles empty take one
+# launch per colour (5 x 257 x 257 nodes, 9 x 401 x 401, 701 x 5 x 701), not so many
+# of them the tiles (521 x 5 x 401), and the restriction takes tiles of 4 x 8 x 8
+# where those are fewer (9 x 25 x 41 and the first two).
+@pytest.mark.parametrize("n,ng,nmn", [((4, 256, 256), 3, 0), ((8, 400, 400), 4, 1),
+                                      ((700, 4, 700), 3, 0), ((520, 4, 400), 3, 1),
+                                      ((8, 24, 40), 3, 0), ((8, 24, 40), 3, 1),
+                                      ((4, 4, 4096), 3, 0)])
+def test_poisson_narrow_grids(gpu, oracle, rng, n, ng, nmn):
+    """phi within 1e-12 of max |phi| and every level's sweeps equal to the
+    oracle's (same operands and expressions; only the residual's summation
+    order differs)."""
+    from essaitemporaire_lepic_module_amd import fields as F
+    n, h = H.box(n)
+    bc = H.two_electrode_bcnd(n)
+    bc[(bc == -1) & (rng.random(bc.shape) < 0.05)] = 4
+    bc[2:n[2] + 1, 0:2, 2:n[0] + 1] = 0
+    bc[0:2, 2:n[1] + 1, 2:n[0] + 1] = 0
+    if nmn:
+        bc[2:n[2] + 1, 2:n[1] + 1, 0:2] = -2
+    rho = np.where(bc <= 0, 1e-4 * rng.standard_normal(bc.shape), 0.0)
+    phi0 = np.where(bc == 2, 20.0, np.where(bc == 4, -5.0, 0.0))
+    phi_o = phi0.copy()
+    st, info_o = oracle.pdesolver(n, h, phi_o, rho, bc, flag_pbc=0, flag_nmn=nmn, ng=ng, eps=1e-8,
+                                  omega=1.4, ncycl=3)
+    assert st == 0
+    for graph in (True, True, False):
+        phi_g = torch.as_tensor(phi0, device=gpu)
+        info_g = F.solve_poisson_legacy(phi_g, torch.as_tensor(bc, device=gpu),
+                                        torch.as_tensor(rho, device=gpu), h, n, 3, 1e-8, 1.4, ng,
+                                        0, nmn, graph=graph)
+        assert info_g["cycles"] == info_o["cycles"]
+        assert info_g["sweeps"] == info_o["sweeps"]
+        np.testing.assert_allclose(phi_g.cpu().numpy(), phi_o, rtol=1e-12,
+                                   atol=1e-12 * np.abs(phi_o).max())
+
+
+def test_poisson_narrow_grid_time(gpu, rng):
+    """A V-cycle of a narrow grid takes at most twice that of a cube of as many
+    nodes (measured 1.2; 3 with its levels on mostly empty tiles)."""
+    import time
+    from essaitemporaire_lepic_module_amd import fields as F
+    best = {}
+    for n, ng in (((4, 4, 32768), 3), ((96, 96, 96), 6)):
+        n, h = H.box(n)
+        bc = torch.as_tensor(cfg.biased_wall_bcnd(n, 2), device=gpu)
+        rho = torch.where(bc <= 0, 1e-5 * torch.as_tensor(rng.standard_normal(cfg.node_shape(n)),
+                                                          device=gpu), 0.0)
+        phi = torch.empty_like(rho)
+        best[n] = 1e9
+        for _ in range(8):
+            phi.copy_(torch.where(bc == 2, 20.0, 0.0))
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            info = F.solve_poisson_legacy(phi, bc, rho, h, n, 20000, 1e-8, 1.4, ng, 0, 0)
+            torch.cuda.synchronize()
+            best[n] = min(best[n], (time.perf_counter() - t) / info["cycles"])
+    narrow, cube = best.values()
+    assert narrow <= 2.0 * cube, (narrow, cube)
+
+
 # The one-workgroup levels (wg_level): one wave up to 128 nodes of a colour
 # (6 x 4 x 4: 100, 6 x 6 x 4: 140), one to five per thread (34 x 32 x 4 is 3060
 # of a colour, 10 x 80 x 4 2430, 2 x 2 x 340 6138 nodes in all), electrodes
