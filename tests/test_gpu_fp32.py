@@ -207,6 +207,44 @@ def test_sort32_place_bitexact(gpu, oracle, rng, n, mean, crowd):
     _same32(g, ref)
 
 
+@pytest.mark.parametrize("n", [(64, 48, 40), (129, 17, 33)])
+@pytest.mark.parametrize("Nm", [3.0, -3.0])
+def test_deposit32_outside_the_box(gpu, n, Nm):
+    """Blocks whose particles spread past their LDS box: lanes of one cell and
+    lanes of different cells take other orders there.  The density is the same
+    int64 per node for the sorted set, the set in random order, pairs and
+    quadruples of one cell in random order and slots a few rows apart, and its
+    sum is the particles times one full weight."""
+    from essaitemporaire_lepic_module_amd import particles32 as P32
+    n, h = H.box(n)
+    r = torch.Generator(device=gpu)
+    r.manual_seed(23)
+    m = 300000
+    cells = torch.randint(0, n[0] * n[1] * n[2], (m // 4,), device=gpu, generator=r)
+    cells = cells.repeat_interleave(4)
+    f = [torch.rand(m, device=gpu, generator=r) for _ in range(3)]
+    near = (torch.arange(m, device=gpu) + 3000 * torch.randn(m, device=gpu, generator=r)).argsort()
+    by_cell = cells.argsort(stable=True)
+    mix = lambda k: torch.randperm(m // k, device=gpu, generator=r)[:, None] * k + torch.arange(
+        k, device=gpu)[None]
+    orders = [by_cell, mix(1).flatten(), mix(2).flatten(), mix(4).flatten(), by_cell[near]]
+    bits = _bits(n, h, Nm)
+    out = []
+    for o in orders:
+        p = P32.ParticleSet32(m, gpu)
+        p._buf[0]["cell"][:m].copy_(cells[o])
+        for k, v in zip(("fx", "fy", "fz"), f):
+            p._buf[0][k][:m].copy_(v[o])
+        p.n = m
+        dep = torch.zeros(cfg.node_shape(n), dtype=torch.int64, device=gpu)
+        P32.deposit32(p, n, h, Nm, bits, dep)
+        out.append(dep)
+    unit = round(abs(Nm) / (h[0] * h[1] * h[2]) * 2.0 ** bits)
+    assert int(out[0].sum()) == (unit if Nm > 0 else -unit) * m
+    for d in out[1:]:
+        assert torch.equal(d, out[0])
+
+
 def _sort_set(P32, gpu, n, cells, seed=3, window=500):
     """A set whose slots are the given cells' in near order (moved by a few
     hundred slots, as particles between two sorts)."""
