@@ -778,7 +778,7 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
                                                     T omega, int s, SlotCtl sc, MGCtl *ctl) {
   const bool judged = ctl != nullptr;
   const KGrid &g = L.g;
-  const int64_t n = (int64_t)(g.n1 / 2 + 1) * (g.n2 + 1) * (g.n3 + 1);
+  const uint32_t n = (uint32_t)(g.n1 / 2 + 1) * (uint32_t)(g.n2 + 1) * (uint32_t)(g.n3 + 1);
   const T *own = colour ? (const T *)L.u : X, *other = colour ? X : (const T *)L.u;
   T *out = colour ? L.u : Xn;
   const bool pull = colour == 1 || s > 0;
@@ -786,7 +786,7 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
   T b = T(0), uc = T(0);
   Nbr6<T> v = {};
   bool node = false;
-  auto load = [&](int64_t t) {
+  auto load = [&](uint32_t t) {
     node = t < n && per_node(L, colour, (int)t, i, j, k);
     if (!node) return;
     const int64_t c = gidx(g, i, j, k);
@@ -796,7 +796,7 @@ __global__ __launch_bounds__(BLOCK) void k_per_half(KLevelT<T> L, const T *X, T 
     v = per_neighbours(L, other, i, j, k, pull);
   };
   // everything the launch reads is under way before the decision
-  NodeWalk nw = walk_strided(n, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, BLOCK);
+  auto nw = walk_strided<uint32_t>(n, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, BLOCK);
   load(nw.t);
   if (judged && s > 0) {
     const double share = colour ? per_share(sc, s - 1) : 0.0;
@@ -872,12 +872,12 @@ __global__ __launch_bounds__(BLOCK) void k_per_end(KLevelT<T> L, MDiv d_n2p3, co
   const T *X = (count & 1) ? u2 : (const T *)L.u;
   const int nx = g.n1 + 3;
   double a = 0.0;
-  const NodeWalk nw = walk_strided((int64_t)nx * (g.n2 + 3) * (g.n3 + 3), (int)blockIdx.x,
-                                   (int)gridDim.x, (int)threadIdx.x, BLOCK);
-  for (int64_t t = nw.t; t < nw.end; t += nw.step) {
-    const uint32_t r = mdiv_q((uint32_t)t, L.d_n1p3), rk = mdiv_q(r, d_n2p3);
-    const int i = (int)((uint32_t)t - r * (uint32_t)nx),
-              j = (int)(r - rk * (uint32_t)(g.n2 + 3)), k = (int)rk;
+  const auto nw = walk_strided<uint32_t>((int64_t)nx * (g.n2 + 3) * (g.n3 + 3), (int)blockIdx.x,
+                                         (int)gridDim.x, (int)threadIdx.x, BLOCK);
+  for (uint32_t t = nw.t; t < nw.end; t += nw.step) {
+    const uint32_t r = mdiv_q(t, L.d_n1p3), rk = mdiv_q(r, d_n2p3);
+    const int i = (int)(t - r * (uint32_t)nx), j = (int)(r - rk * (uint32_t)(g.n2 + 3)),
+              k = (int)rk;
     const bool is_red = (i + j + k) & 1;
     int sj = j, sk = k;
     per_source(L, i, sj, sk);

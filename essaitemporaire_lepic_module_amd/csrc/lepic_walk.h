@@ -11,17 +11,21 @@
 #define LEPIC_HD
 #endif
 
-// for (t; t < end; t += step).  64-bit: a level has up to 2^31 - 1 nodes, and
-// the step past its last node has to stay beyond end (in 32 bits it wraps to a
-// negative number, which the loop takes for a node).
-struct NodeWalk {
-  int64_t t, end, step;
+// for (t; t < end; t += step).  I: int64_t, or uint32_t (2 % of a periodic solve):
+// a level has up to 2^31 - 1 nodes, and the step past its last node has to stay
+// beyond end.  In an int it wraps to a negative number, which the loop takes for
+// a node; in 32 unsigned bits it does not, for steps below 2^31.
+template <class I>
+struct WalkT {
+  I t, end, step;
 };
+using NodeWalk = WalkT<int64_t>;
 
 // Striding over all blocks.
-LEPIC_HD inline NodeWalk walk_strided(int64_t nodes, int block, int blocks, int thread,
+template <class I = int64_t>
+LEPIC_HD inline WalkT<I> walk_strided(int64_t nodes, int block, int blocks, int thread,
                                       int threads) {
-  return {(int64_t)block * threads + thread, nodes, (int64_t)blocks * threads};
+  return {(I)((int64_t)block * threads + thread), (I)nodes, (I)((int64_t)blocks * threads)};
 }
 
 // The blocks of each of `groups` (the XCDs, which take blocks in turn) walk

@@ -89,6 +89,37 @@ long check_bricks() {
   return bad;
 }
 
+// The largest levels: every visit in range and as many visits as nodes, over all
+// threads (a thread's visits counted from its first and last node).
+template <class I>
+long check_largest() {
+  const int threads = 256, groups = 8, blocks = 1024;
+  long bad = 0;
+  for (int64_t nodes : {(int64_t)INT32_MAX, (int64_t)2147458027, (int64_t)INT32_MAX - 262144}) {
+    for (int grouped = 0; grouped < (sizeof(I) == 8 ? 2 : 1); ++grouped) {
+      int64_t visits = 0;
+      for (int b = 0; b < blocks; ++b)
+        for (int t = 0; t < threads; ++t) {
+          WalkT<I> w;
+          if (grouped) {
+            const NodeWalk g = walk_grouped(nodes, b, blocks, t, threads, groups);
+            w = {(I)g.t, (I)g.end, (I)g.step};
+          } else {
+            w = walk_strided<I>(nodes, b, blocks, t, threads);
+          }
+          if (w.t >= w.end) continue;
+          const int64_t n = ((int64_t)w.end - w.t + w.step - 1) / w.step;
+          // the loop's own type carries the step past the last node
+          const I last = (I)(w.t + (I)(n - 1) * w.step), past = (I)(last + w.step);
+          if ((int64_t)w.t < 0 || (int64_t)w.end > nodes || past < w.end || last >= w.end) ++bad;
+          visits += n;
+        }
+      bad += visits != nodes;
+    }
+  }
+  return bad;
+}
+
 }  // namespace
 
 int main() {
@@ -112,27 +143,7 @@ int main() {
       }
     }
   }
-  // the largest levels: every visit in range and as many visits as nodes, over
-  // all threads (a thread's visits counted from its first and last node)
-  const int blocks = 1024;
-  for (int64_t nodes : {(int64_t)INT32_MAX, (int64_t)2147458027, (int64_t)INT32_MAX - 262144}) {
-    for (int grouped = 0; grouped < 2; ++grouped) {
-      int64_t visits = 0;
-      for (int b = 0; b < blocks; ++b)
-        for (int t = 0; t < threads; ++t) {
-          const NodeWalk w = grouped ? walk_grouped(nodes, b, blocks, t, threads, groups)
-                                     : walk_strided(nodes, b, blocks, t, threads);
-          if (w.t >= w.end) continue;
-          const auto n = (w.end - w.t + w.step - 1) / w.step;
-          // the loop's own type carries the step past the last node
-          decltype(NodeWalk::t) past = (decltype(NodeWalk::t))(w.t + (n - 1) * w.step);
-          past += w.step;
-          if (w.t < 0 || w.end > nodes || past < w.end || past - w.step >= nodes) ++bad;
-          visits += n;
-        }
-      bad += visits != nodes;
-    }
-  }
+  bad += check_largest<int64_t>() + check_largest<uint32_t>();
   bad += check_bricks();
   std::printf("bad %ld\n", bad);
   return bad != 0;
