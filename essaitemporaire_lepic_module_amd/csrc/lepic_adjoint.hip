@@ -691,7 +691,9 @@ namespace {
 // 2.1M electrons on 64^3 take 240 us sorted, 1040 after one step and 1640 after 5;
 // ordered anew 400 and 580 with the order (50); a run of 20 steps 141.7 -> 125.7
 // ms.  k_adj_probe decides whether the order is formed.  From ORDER_MIN particles:
-// the launches cost a run of 48^3 x 10 (1.1M) -3 %, of 32^3 x 6 (0.2M) +0.6 %.
+// there (0.5M on 32^3) a call takes 110 us instead of 96 sorted, 160 both 3 steps
+// later, 222 instead of 375 after 10; a run of 48^3 x 10 (1.1M) was 3 % faster with
+// the order, one of 32^3 x 6 (0.2M), which now goes without, 0.6 % slower.
 constexpr int64_t ORDER_MIN = (int64_t)1 << 19;
 static_assert(ORDER_MIN >= (int64_t)BLOCK * APT * ORDER_SAMPLES, "a block per sample");
 

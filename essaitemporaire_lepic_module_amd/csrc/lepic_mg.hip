@@ -347,8 +347,8 @@ __global__ __launch_bounds__(BLOCK) void k_decide(const double *partials, int64_
 // the same bits as the owner's) and writes its own nodes to the other of two
 // u arrays, which the next launch reads.  One launch per colour, residual and
 // decision spends 60 us per sweep at 128^3 (19.6 + 19.6 + 15.2 + 5) and 12 at
-// 16^3, all of it launches and L2 round trips; the fused sweep takes 29 us and
-// 9 (an idle one 3), FP64, split about evenly between the reads (390 KB per
+// 16^3, all of it launches and L2 round trips; the fused sweep takes 28 us and
+// 9 (an idle one 4.5), FP64, split about evenly between the reads (390 KB per
 // block through one CU's L1), the three LDS phases and launch + decision.
 //
 // The two colours are held apart in LDS, so that the lanes of a phase read
@@ -1429,7 +1429,9 @@ __device__ __forceinline__ void wg_sor_rb(const CoarseArgs<T> &A, T *S, int16_t 
 //    accesses are in order without a barrier.
 // want_res: the residual after the last sweep is returned, to every thread.
 // Up to 3 pairs per thread have their own copy of the routine: five spill in FP64
-// (16^3: 240 us a solve instead of 281).
+// (16^3: 240 us a solve instead of 281).  With its spills the copy of five is
+// still the faster form past 3072 pairs (coarsest levels of 3213 and 3519: 24
+// V-cycles of 32 x 32 x 40 4.6 -> 3.5 ms, 26 of 32 x 32 x 44 7.5 -> 3.8).
 // Launch of 16^3 and below, FP64: 98 -> 62 us; 8^3 and below 47 -> 32.
 template <class T, int NT, int SL>
 __device__ __forceinline__ double wg_level(const CoarseArgs<T> &A, T *S, int16_t *Lb, int l,
