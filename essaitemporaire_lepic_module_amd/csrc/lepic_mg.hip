@@ -6,9 +6,9 @@
 // A sweep of a global level is one launch over tiles held in LDS (k_sweep):
 // red, black and the L1 residual, with sor_rb's exit rule (res/res_s <= 0.6,
 // at most 4 sweeps) taken by every block of the next launch.  Levels with
-// periodic walls take two launches per sweep (k_per_half); a coarsest level too
-// large for one workgroup takes one per colour, a deterministic block-tree
-// residual and a one-block decision.  Sweeps queued after the exit return at
+// periodic walls take two launches per sweep (k_per_half); narrow and flat levels
+// (sweeps_tiled) and a coarsest level too large for one workgroup take one per
+// colour, a deterministic block-tree residual and a one-block decision.  Sweeps queued after the exit return at
 // once, so a V-cycle needs no host round trip; the host reads the fine
 // residual once per V-cycle for pdesolver's convergence test.  Levels below a
 // few thousand nodes run inside one workgroup (k_mg_coarse).
@@ -1894,9 +1894,9 @@ struct Solver {
                        dig, nr);
   }
 
-  // A level sweeps in whole-sweep launches, with periodic walls in two per
-  // sweep; the coarsest level's sor_rb (another exit rule, up to 10^6 sweeps)
-  // keeps one launch per colour.
+  // A level with a second u array sweeps in whole-sweep launches, with periodic
+  // walls in two per sweep; the others and the coarsest level's sor_rb (another
+  // exit rule, up to 10^6 sweeps) in one launch per colour.
   bool tiled(int l, int dig) const { return !flag_pbc && dig != 0 && u2[l]; }
   bool periodic(int l, int dig) const { return flag_pbc && dig != 0 && u2[l]; }
 
